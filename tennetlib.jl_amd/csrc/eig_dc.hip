@@ -1,13 +1,17 @@
-// Symmetric eigen-decomposition of the density matrix for p > 64, in FP64:
+// Symmetric / Hermitian eigen-decomposition of the density matrix, in FP64.
+// Up to DC_SMALL_MAX rows one workgroup does each stage (eig_small.hip).
+// Above that:
 //
 //  1. Householder tridiagonalisation G = H T H^T on the device, one column
 //     per step: trd_reflect_kernel forms the reflector from row j (every
 //     workgroup redundantly, so no extra launch) and y = tau G22 v;
 //     trd_update_kernel applies G22 -= v w^T + w v^T.  The reflectors are
-//     kept below the diagonal of G.
+//     kept below the diagonal of G.  The last TRD_SMALL_MAX columns are
+//     reduced by one workgroup in registers (416 us for 192 columns; 136
+//     columns in LDS took 556 us, one launch per column 7.1 us each).
 //  2. Divide and conquer on T (Cuppen's tearing, bottom-up): leaves of at
-//     most 32 rows are diagonalised by parallel Jacobi in LDS (one
-//     wavefront per leaf); each merge of two neighbouring blocks solves
+//     most DC_SMALL_MAX rows are solved one workgroup each (dc_small); each
+//     merge of two neighbouring blocks solves
 //     D + rho z z^T: deflation (small |rho z_i|, or a Givens rotation for
 //     nearly equal d_i) on the host, the secular equation for every
 //     remaining root on the device (one wavefront per root, bracketed Newton
@@ -15,11 +19,13 @@
 //     Gu-Eisenstat z-hat, the eigenvectors z-hat / (d - lambda), and the
 //     block update Q <- Q U as an FP64 MFMA GEMM.  The host keeps the
 //     eigenvalues and only reads z and the roots once per level.
-//  3. Back-transformation Q <- H Q with blocks of 64 reflectors in the
+//  3. Back-transformation Q <- H Q: up to BACK_SMALL_MAX rows one reflector
+//     after the other with the columns of Q in registers (370 rows: 105 us;
+//     the blocked form below takes six rounds of five launches, about 600 us);
+//     above, with blocks of 64 reflectors in the
 //     compact WY form I - V T V^T: three GEMMs per block and a triangular
 //     solve with T^{-1} = diag(1/tau) + striu(V^T V) in place of T.
-// Accuracy: eigenvalues to ~eps * ||G||, orthonormal eigenvectors; the
-// same absolute accuracy as the block-Jacobi solver used for p <= 64.
+// Accuracy: eigenvalues to ~eps * ||G||, orthonormal eigenvectors.
 #include "tn_internal.h"
 
 #include <algorithm>
@@ -34,7 +40,7 @@ namespace {
 
 constexpr double EPS = 2.220446049250313e-16;
 constexpr int HR = 4;     // rows of y per workgroup in the reflector step (one per wave)
-constexpr int LEAF = 32;  // leaf size of the divide and conquer
+constexpr int LEAF = DC_SMALL_MAX;  // leaf size of the divide and conquer
 constexpr int NBW = 64;   // reflectors per compact-WY block
 
 // sum over the 256 threads of a workgroup; every thread gets the same value
@@ -619,20 +625,6 @@ __global__ __launch_bounds__(256) void trd_panel_wlast_kernel(int p, int j, int 
 // a fixed order, so the result does not depend on scheduling.
 constexpr int SYT = 64;
 
-// tau, alpha and the reflector scale of column j from the sum of squares ss
-// of x_1.. and x_0 (every kernel that needs them computes them this way)
-__device__ __forceinline__ void trd_reflector(double x0, double ss, double& tau, double& alpha, double& scale) {
-  tau = 0.0;
-  alpha = x0;
-  scale = 0.0;
-  if (ss > 0.0) {
-    const double nrm = sqrt(x0 * x0 + ss);
-    alpha = (x0 >= 0.0) ? -nrm : nrm;
-    tau = (alpha - x0) / alpha;
-    scale = 1.0 / (x0 - alpha);
-  }
-}
-
 // sum of squares of x_1.. from the row kernel's partial sums, reduced by the
 // calling wave (every lane gets the same bits; both kernels below use it, so
 // they agree on tau and the reflector scale)
@@ -939,105 +931,8 @@ __global__ __launch_bounds__(256) void trd_mirror_lower_kernel(double* __restric
   }
 }
 
-// ---- the last columns in LDS: the trailing block A[j0:, j0:] (m0 = p - j0
-// <= TAIL rows) is reduced by one workgroup without leaving LDS; reflectors,
-// d, e and tau are written exactly as by the per-column kernels.
-constexpr int TAIL = 136;  // 136 x 137 doubles + two vectors: 148 KB of LDS
-__global__ __launch_bounds__(256) void trd_tail_lds_kernel(double* __restrict__ A, long ld, int p, int j0,
-                                                           double* __restrict__ dv, double* __restrict__ ev,
-                                                           double* __restrict__ tauv) {
-  extern __shared__ double lds[];
-  __shared__ double red[4];
-  const int m0 = p - j0, L = m0 + 1;
-  double* M = lds;               // m0 x L
-  double* vs = M + (long)m0 * L; // m0
-  double* ys = vs + m0;          // m0
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  {  // load the block in batches of 8 elements per thread (loads before stores)
-    const int tot = m0 * m0;
-    for (int base = 0; base < tot; base += 256 * 8) {
-      double t[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + 256 * u + tid;
-        t[u] = (idx < tot) ? A[(long)(j0 + idx / m0) * ld + (j0 + idx % m0)] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int idx = base + 256 * u + tid;
-        if (idx < tot) M[(idx / m0) * L + idx % m0] = t[u];
-      }
-    }
-  }
-  __syncthreads();
-  for (int jj = 0; jj < m0 - 2; ++jj) {
-    const int j = j0 + jj, m = m0 - jj - 1;
-    const double* x = M + jj * L + (jj + 1);
-    double ss = 0.0;
-    for (int c = tid; c < m; c += 256) {
-      const double t = x[c];
-      vs[c] = t;
-      if (c > 0) ss += t * t;
-    }
-    ss = block_sum(ss, red);
-    const double x0 = vs[0];
-    double tau = 0.0, alpha = x0, scale = 0.0;
-    if (ss > 0.0) {
-      const double nrm = sqrt(x0 * x0 + ss);
-      alpha = (x0 >= 0.0) ? -nrm : nrm;
-      tau = (alpha - x0) / alpha;
-      scale = 1.0 / (x0 - alpha);
-    }
-    __syncthreads();
-    for (int c = tid; c < m; c += 256) {
-      const double v = (c == 0) ? 1.0 : vs[c] * scale;
-      vs[c] = v;
-      A[(long)(j + 1 + c) * ld + j] = v;
-    }
-    if (tid == 0) {
-      dv[j] = M[jj * L + jj];
-      ev[j] = alpha;
-      tauv[j] = tau;
-    }
-    __syncthreads();
-    if (tau == 0.0) continue;  // uniform
-    // y = tau M22 v, one thread per row (odd row stride: no bank conflicts)
-    double dot = 0.0;
-    if (tid < m) {
-      const double* row = M + (jj + 1 + tid) * L + (jj + 1);
-      double sacc = 0.0;
-      for (int c = 0; c < m; ++c) sacc += row[c] * vs[c];
-      const double yr = tau * sacc;
-      ys[tid] = yr;
-      dot = yr * vs[tid];
-    }
-    dot = block_sum(dot, red);
-    const double hs = 0.5 * tau * dot;
-    for (int c = tid; c < m; c += 256) ys[c] = ys[c] - hs * vs[c];  // w
-    __syncthreads();
-    for (int c = lane; c < m; c += 64) {
-      const double vc = vs[c], wc = ys[c];
-      for (int r = wave; r < m; r += 4) M[(jj + 1 + r) * L + (jj + 1 + c)] -= vs[r] * wc + ys[r] * vc;
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    dv[p - 2] = M[(m0 - 2) * L + (m0 - 2)];
-    ev[p - 2] = M[(m0 - 2) * L + (m0 - 1)];
-    dv[p - 1] = M[(m0 - 1) * L + (m0 - 1)];
-  }
-}
-
-// last 2 x 2 corner and the explicit reflector matrix V (p x p, column j =
-// v_j with zeros above row j + 1; columns j >= p - 2 are zero)
-__global__ void trd_tail_kernel(const double* __restrict__ A, long ld, int p, double* dv, double* ev) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (p >= 2) {
-    dv[p - 2] = A[(long)(p - 2) * ld + (p - 2)];
-    ev[p - 2] = A[(long)(p - 2) * ld + (p - 1)];
-  }
-  dv[p - 1] = A[(long)(p - 1) * ld + (p - 1)];
-}
+// the explicit reflector matrix V (p x p, column j = v_j with zeros above row
+// j + 1; columns j >= p - 2 are zero)
 __global__ __launch_bounds__(256) void trd_extract_v_kernel(const double* __restrict__ A, long ld, int p,
                                                             const double* __restrict__ tauv, double* __restrict__ V) {
   const long tot = (long)p * p;
@@ -1199,74 +1094,6 @@ __global__ __launch_bounds__(256) void trdz_update_kernel(double2* __restrict__ 
   }
 }
 
-// the last columns in LDS (m0 = p - j0 <= TAILZ), including the final
-// one-element reflector that makes e_{p-2} real
-constexpr int TAILZ = 90;
-__global__ __launch_bounds__(256) void trdz_tail_lds_kernel(double2* __restrict__ A, long ld, int p, int j0,
-                                                            double* __restrict__ dv, double* __restrict__ ev,
-                                                            double2* __restrict__ tauv) {
-  extern __shared__ double2 zl[];
-  __shared__ double red[4];
-  const int m0 = p - j0, L = m0 + 1;
-  double2* M = zl;                // m0 x L
-  double2* vs = M + (long)m0 * L; // m0
-  double2* ys = vs + m0;          // m0
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int r = wave; r < m0; r += 4)
-    for (int c = lane; c < m0; c += 64) M[r * L + c] = A[(long)(j0 + r) * ld + (j0 + c)];
-  __syncthreads();
-  for (int jj = 0; jj < m0 - 1; ++jj) {
-    const int j = j0 + jj, m = m0 - jj - 1;
-    double ss = 0.0;
-    for (int c = tid; c < m; c += 256) {
-      const double2 t = zconj(M[jj * L + (jj + 1 + c)]);
-      vs[c] = t;
-      if (c > 0) ss += t.x * t.x + t.y * t.y;
-    }
-    ss = block_sum(ss, red);
-    const ZRefl R = zlarfg(vs[0], ss);
-    __syncthreads();
-    for (int c = tid; c < m; c += 256) {
-      const double2 v = (c == 0) ? make_double2(1.0, 0.0) : zmul(vs[c], R.scale);
-      vs[c] = v;
-      A[(long)(j + 1 + c) * ld + j] = v;
-    }
-    if (tid == 0) {
-      dv[j] = M[jj * L + jj].x;
-      ev[j] = R.beta;
-      tauv[j] = R.tau;
-    }
-    __syncthreads();
-    if (R.tau.x == 0.0 && R.tau.y == 0.0) continue;  // uniform
-    double2 dot = make_double2(0.0, 0.0);
-    if (tid < m) {
-      const double2* row = M + (jj + 1 + tid) * L + (jj + 1);
-      double sre = 0.0, sim = 0.0;
-      for (int c = 0; c < m; ++c) {
-        const double2 t = zmul(row[c], vs[c]);
-        sre += t.x;
-        sim += t.y;
-      }
-      const double2 yr = zmul(R.tau, make_double2(sre, sim));
-      ys[tid] = yr;
-      dot = zmul(zconj(yr), vs[tid]);
-    }
-    dot = block_sum_z(dot, red);
-    const double2 al = zscale(zmul(R.tau, dot), -0.5);
-    for (int c = tid; c < m; c += 256) ys[c] = zadd(ys[c], zmul(al, vs[c]));  // w
-    __syncthreads();
-    for (int c = lane; c < m; c += 64) {
-      const double2 cvc = zconj(vs[c]), cwc = zconj(ys[c]);
-      for (int r = wave; r < m; r += 4) {
-        double2* a = M + (jj + 1 + r) * L + (jj + 1 + c);
-        *a = zsub(*a, zadd(zmul(vs[r], cwc), zmul(ys[r], cvc)));
-      }
-    }
-    __syncthreads();
-  }
-  if (tid == 0) dv[p - 1] = M[(m0 - 1) * L + (m0 - 1)].x;
-}
-
 // explicit complex reflectors (p x p): column j = v_j below row j, zero elsewhere
 __global__ __launch_bounds__(256) void trdz_extract_v_kernel(const double2* __restrict__ A, long ld, int p,
                                                              const double2* __restrict__ tauv,
@@ -1331,103 +1158,6 @@ __global__ __launch_bounds__(256) void adjoint_z_kernel(const double2* __restric
 // ---------------------------------------------------------------------------
 // 2. divide and conquer
 // ---------------------------------------------------------------------------
-// Leaf Jacobi: block [a, a + n) of the torn tridiagonal (n <= LEAF = 32),
-// one wavefront per leaf; eigenvectors into Q[a:a+n, a:a+n] (columns),
-// values into lam[a:a+n].  Lane t owns rotation pair t/4 of a step and 8 of
-// its columns (rows).
-__global__ __launch_bounds__(64) void dc_leaf_kernel(const double* __restrict__ d, const double* __restrict__ e,
-                                                     const int* __restrict__ leaf_a, const int* __restrict__ leaf_n,
-                                                     double tol_abs, double* __restrict__ Q, long ldq,
-                                                     double* __restrict__ lam) {
-  constexpr int P = LEAF, LD = LEAF + 1;
-  __shared__ double Gs[P][LD];
-  __shared__ double Js[P][LD];
-  __shared__ double cs[P / 2], sn[P / 2];
-  __shared__ int pi_[P / 2], pj_[P / 2], fl[P / 2];
-  const int a = leaf_a[blockIdx.x], n = leaf_n[blockIdx.x], tid = threadIdx.x;
-  for (int idx = tid; idx < P * P; idx += 64) {
-    const int r = idx / P, c = idx % P;
-    double g = 0.0;
-    if (r < n && c < n) {
-      if (r == c) g = d[a + r];
-      else if (c == r + 1) g = e[a + r];
-      else if (r == c + 1) g = e[a + c];
-    }
-    Gs[r][c] = g;
-    Js[r][c] = (r == c) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  const double tol_rel = 64.0 * EPS;
-  const int pp = tid >> 2, sub = tid & 3;
-  // the tournament runs over the leaf's own size rounded up to even (Pe - 1
-  // rounds of Pe / 2 pairs), not over all P slots: a padding index has no
-  // coupling and never rotates
-  const int Pe = (n + 1) & ~1;
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    int nsweep = 0;
-    for (int step = 0; step < Pe - 1; ++step) {
-      int f = 0;
-      if (tid < P / 2 && tid >= Pe / 2) {
-        pi_[tid] = 0; pj_[tid] = 0; cs[tid] = 1.0; sn[tid] = 0.0; fl[tid] = 0;
-      } else if (tid < P / 2) {
-        const int pa = tid, pb = Pe - 1 - tid;
-        const int i = (pa == 0) ? 0 : 1 + ((pa - 1 + step) % (Pe - 1));
-        const int jj = 1 + ((pb - 1 + step) % (Pe - 1));
-        const double x = Gs[i][i], z = Gs[jj][jj], g = Gs[i][jj];
-        double c = 1.0, s = 0.0;
-        if (fabs(g) > fmax(tol_rel * sqrt(fabs(x)) * sqrt(fabs(z)), tol_abs)) {
-          const double zeta = (z - x) / (2.0 * g);
-          double t;
-          if (fabs(zeta) > 1e150) t = 0.5 / zeta;
-          else t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-          c = 1.0 / sqrt(1.0 + t * t);
-          s = c * t;
-          f = 1;
-        }
-        pi_[tid] = i; pj_[tid] = jj; cs[tid] = c; sn[tid] = s; fl[tid] = f;
-      }
-      const int nrot = __syncthreads_count(f);
-      if (nrot == 0) continue;
-      nsweep += nrot;
-      if (fl[pp]) {
-        const int i = pi_[pp], jj = pj_[pp];
-        const double c = cs[pp], s = sn[pp];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int col = sub * 8 + u;
-          const double gi = Gs[i][col], gj = Gs[jj][col];
-          Gs[i][col] = c * gi - s * gj;
-          Gs[jj][col] = s * gi + c * gj;
-        }
-      }
-      __syncthreads();
-      if (fl[pp]) {
-        const int i = pi_[pp], jj = pj_[pp];
-        const double c = cs[pp], s = sn[pp];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int row = sub * 8 + u;
-          const double gi = Gs[row][i], gj = Gs[row][jj];
-          Gs[row][i] = c * gi - s * gj;
-          Gs[row][jj] = s * gi + c * gj;
-          const double ji = Js[row][i], jv = Js[row][jj];
-          Js[row][i] = c * ji - s * jv;
-          Js[row][jj] = s * ji + c * jv;
-        }
-      }
-      __syncthreads();
-    }
-    if (nsweep == 0) break;
-  }
-  // padding indices never rotate with real ones (zero coupling), so the
-  // first n columns of J restricted to the first n rows are the eigenvectors
-  for (int idx = tid; idx < n * n; idx += 64) {
-    const int r = idx / n, c = idx % n;
-    Q[(long)(a + r) * ldq + (a + c)] = Js[r][c];
-  }
-  if (tid < n) lam[a + tid] = Gs[tid][tid];
-}
-
 // Zero the two off-diagonal sub-blocks of each merge block, so that every
 // column of the block is explicit over all n rows.
 struct MergeDev {
@@ -1665,6 +1395,22 @@ __global__ __launch_bounds__(256) void dc_put_cols_kernel(double* __restrict__ Q
 // ---------------------------------------------------------------------------
 // 3. back-transformation helpers
 // ---------------------------------------------------------------------------
+// reflectors as rows: R[j][r] = A[r][j] for r > j, zero elsewhere (R p x p; 32 x 32 tiles)
+template <typename T>
+__global__ __launch_bounds__(256) void reflector_rows_kernel(const T* __restrict__ A, long ld, int p,
+                                                             T* __restrict__ R) {
+  __shared__ T t[32][33];
+  const int r0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int k = ty; k < 32; k += 8)
+    if (r0 + k < p && j0 + tx < p && r0 + k > j0 + tx) t[k][tx] = A[(long)(r0 + k) * ld + (j0 + tx)];
+  __syncthreads();
+  for (int k = ty; k < 32; k += 8) {
+    const int j = j0 + k, r = r0 + tx;
+    if (j < p && r < p) R[(long)j * p + r] = r > j ? t[tx][k] : T{};
+  }
+}
+
 // W <- T W for the compact WY form, through T^{-1} = diag(1/tau) + striu(S),
 // S = V^T V (Joffrain et al.): back-substitution, one thread per column of
 // W (nb x n, ld n).  A reflector with tau = 0 has a zero column in V.
@@ -1807,9 +1553,6 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
   char* hs = (char*)c->host_stage(lvb + 8 * (size_t)p * sizeof(double) + 256);
   double* hx = (double*)(hs + ((lvb + 255) & ~(size_t)255));
   // ---- 2. divide and conquer on (d, e)
-  double tnorm = 0.0;
-  for (long i = 0; i < p; ++i) tnorm = std::max(tnorm, std::fabs(d[i]));
-  for (long i = 0; i + 1 < p; ++i) tnorm = std::max(tnorm, 2.0 * std::fabs(e[i]));
   struct Blk { int a, n; };
   std::vector<Blk> blocks;
   {  // ceil(P / LEAF) leaves of nearly equal size (the slowest leaf sets the time)
@@ -1827,24 +1570,25 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
     dt[k] -= e[k - 1];
   }
   const long ldq = p;
-  double* small = (double*)c->workspace(WS_DC_SMALL, (size_t)(8 * p + 64) * sizeof(double));
+  double* small = (double*)c->workspace(WS_DC_SMALL, (size_t)3 * p * sizeof(double) + blocks.size() * sizeof(SmallEig));
   double* d_dt = small;
   double* d_e = d_dt + p;
   double* d_lam = d_e + p;
-  int* d_la = (int*)(d_lam + p);
-  int* d_ln = d_la + p;
+  SmallEig* d_leaf = (SmallEig*)(d_lam + p);
   {
-    // mirror of the `small` layout: dt, e, lam (p doubles each), leaf starts and sizes (p ints each)
+    // mirror of the `small` layout: dt, e, lam (p doubles each), leaves
     std::copy(dt.begin(), dt.end(), hx);
     std::copy(e.begin(), e.end(), hx + p);
-    int* hla = (int*)(hx + 3 * p);
-    int* hln = hla + p;
-    for (size_t b = 0; b < blocks.size(); ++b) { hla[b] = blocks[b].a; hln[b] = blocks[b].n; }
-    TN_HIP(hipMemcpyAsync(small, hx, (size_t)3 * p * sizeof(double) + 2 * (size_t)p * sizeof(int),
+    SmallEig* hl = (SmallEig*)(hx + 3 * p);
+    int nmax = 0;
+    for (size_t b = 0; b < blocks.size(); ++b) {
+      const int a = blocks[b].a;
+      hl[b] = SmallEig{blocks[b].n, a, 0, 0, (long)a * ldq + a, ldq, 0, 0};
+      nmax = std::max(nmax, blocks[b].n);
+    }
+    TN_HIP(hipMemcpyAsync(small, hx, (size_t)3 * p * sizeof(double) + blocks.size() * sizeof(SmallEig),
                           hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(dc_leaf_kernel, dim3((unsigned)blocks.size()), dim3(64), 0, c->stream, d_dt, d_e, d_la,
-                       d_ln, EPS * tnorm, Q, ldq, d_lam);
-    TN_HIP(hipGetLastError());
+    dc_small(c, nmax, (int)blocks.size(), SmallEig{}, d_leaf, d_dt, d_e, Q, d_lam);
   }
   TN_HIP(hipMemcpyAsync(hx + 2 * p, d_lam, p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   stage("leaves");
@@ -2011,7 +1755,7 @@ constexpr int TRD_BLOCKED_MIN = 3072;
 constexpr int TRD_TILE_MIN = 1024;
 
 void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, std::vector<double>& w) {
-  TN_REQUIRE(p >= 3 && p <= 16384, TN_E_INVALID, "sym_eig_dc: size out of range");
+  TN_REQUIRE(p >= 1 && p <= 16384, TN_E_INVALID, "sym_eig_dc: size out of range");
   const int P = (int)p;
   EigStages stage(c, p);
   // ---- 1. tridiagonalisation
@@ -2019,11 +1763,25 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
   double* dv = vecs;
   double* ev = dv + p;
   double* tauv = ev + p;
+  if (P <= DC_SMALL_MAX) {  // one workgroup holds the block: three launches, one read-back
+    double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
+    double* lam = tauv + p;
+    const SmallEig one{P, 0, 0, ldg, 0, p, 0, ldv};
+    trd_small(c, false, P, 1, one, nullptr, G, dv, ev, tauv, true);
+    dc_small(c, P, 1, one, nullptr, dv, ev, Q, lam);
+    back_small(c, false, P, 1, one, nullptr, G, tauv, Q, Vt);
+    double* hx = (double*)c->host_stage((size_t)p * sizeof(double));
+    TN_HIP(hipMemcpyAsync(hx, lam, (size_t)p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    TN_HIP(hipStreamSynchronize(c->stream));
+    w.assign(hx, hx + p);
+    stage("one workgroup");
+    return;
+  }
   double* y = tauv + p;
   double* part = y + p;  // <= ceil(p / HR) entries
   // panels of NBT columns (one pass over the trailing block per column) from
   // p = TRD_BLOCKED_MIN on; below it one fused launch per column
-  const int jt = std::max(0, P - TAIL);  // columns jt.. are reduced in LDS
+  const int jt = std::max(0, P - TRD_SMALL_MAX);  // columns jt.. are reduced by one workgroup
   bool done = false;
   if (jt >= 1 && P >= TRD_BLOCKED_MIN) {
     const int nAmax = (P + RCHUNK - 1) / RCHUNK;
@@ -2105,16 +1863,12 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
         gemm(c, Prec::F64, g);
       }
     }
-    const int m0 = P - jt;
-    const size_t tshm = ((size_t)m0 * (m0 + 1) + 2 * (size_t)m0) * sizeof(double);
-    raise_lds_limit((const void*)trd_tail_lds_kernel, ((size_t)TAIL * (TAIL + 1) + 2 * TAIL) * sizeof(double));
-    hipLaunchKernelGGL(trd_tail_lds_kernel, dim3(1), dim3(256), tshm, c->stream, G, ldg, P, jt, dv, ev, tauv);
     done = true;
   }
   if (!done) {
     const size_t lds_bytes = (size_t)p * sizeof(double);
     raise_lds_limit((const void*)trd_reflect_kernel, (size_t)lds_bytes);
-    const int j0 = std::max(0, P - TAIL);  // columns j0.. are reduced in LDS
+    const int j0 = jt;
     if (j0 >= 1 && P <= 6000) {
       // fused path: reflector 0, then one launch per column, then the update of step j0 - 1
       double* vA = vecs + 6 * p + 512;
@@ -2154,11 +1908,9 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
                            nparts, tauv);
       }
     }
-    const int m0 = P - j0;
-    const size_t tshm = ((size_t)m0 * (m0 + 1) + 2 * (size_t)m0) * sizeof(double);
-    raise_lds_limit((const void*)trd_tail_lds_kernel, ((size_t)TAIL * (TAIL + 1) + 2 * TAIL) * sizeof(double));
-    hipLaunchKernelGGL(trd_tail_lds_kernel, dim3(1), dim3(256), tshm, c->stream, G, ldg, P, j0, dv, ev, tauv);
   }
+  trd_small(c, false, P - jt, 1, SmallEig{P - jt, jt, (long)jt * ldg + jt, ldg, 0, 0, 0, 0}, nullptr, G, dv, ev, tauv,
+            false);
   TN_HIP(hipGetLastError());
   // d, e to the host through the pinned staging buffer
   double* hx = (double*)c->host_stage(2 * (size_t)p * sizeof(double));
@@ -2169,6 +1921,18 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
   double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
   const long ldq = p;
   std::vector<double> D = dc_tridiag(c, p, d, e, Q, stage);
+  if (P <= BACK_SMALL_MAX) {
+    // ---- 3. back-transformation with the reflectors as rows
+    double* rows = (double*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double));
+    const unsigned nt = (unsigned)((P + 31) / 32);
+    hipLaunchKernelGGL(reflector_rows_kernel<double>, dim3(nt, nt), dim3(256), 0, c->stream, G, ldg, P, rows);
+    TN_HIP(hipGetLastError());
+    back_small(c, false, P, 1, SmallEig{P, 0, 0, p, 0, ldq, 0, ldv}, nullptr, rows, tauv, Q, Vt);
+    stage("back-transform");
+    w.assign(D.begin(), D.end());
+    TN_HIP(hipStreamSynchronize(c->stream));
+    return;
+  }
   double* tmp = (double*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double));
 
   // ---- 3. back-transformation Q <- H Q, H = H_0 ... H_{p-3}
@@ -2223,7 +1987,7 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
 
 
 void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv, std::vector<double>& w) {
-  TN_REQUIRE(p >= 2 && p <= 16384, TN_E_INVALID, "sym_eig_dc_z: size out of range");
+  TN_REQUIRE(p >= 1 && p <= 16384, TN_E_INVALID, "sym_eig_dc_z: size out of range");
   double2* G = reinterpret_cast<double2*>(Gd);
   double2* Vt = reinterpret_cast<double2*>(Vtd);
   const int P = (int)p;
@@ -2235,7 +1999,21 @@ void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv
   double2* tauz = reinterpret_cast<double2*>(ev + p);  // p
   double2* yz = tauz + p;                              // p
   double2* partz = yz + p;                             // <= ceil(p / HR)
-  const int j0 = std::max(0, P - TAILZ);
+  if (P <= std::min(DC_SMALL_MAX, TRD_SMALL_MAX_Z)) {
+    double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
+    double* lam = (double*)yz;
+    const SmallEig one{P, 0, 0, ldg, 0, p, 0, ldv};
+    trd_small(c, true, P, 1, one, nullptr, G, dv, ev, tauz, true);
+    dc_small(c, P, 1, one, nullptr, dv, ev, Q, lam);
+    back_small(c, true, P, 1, one, nullptr, G, tauz, Q, Vt);
+    double* hx = (double*)c->host_stage((size_t)p * sizeof(double));
+    TN_HIP(hipMemcpyAsync(hx, lam, (size_t)p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    TN_HIP(hipStreamSynchronize(c->stream));
+    w.assign(hx, hx + p);
+    stage("one workgroup");
+    return;
+  }
+  const int j0 = P - TRD_SMALL_MAX_Z;
   {
     const size_t lds_max = (size_t)p * sizeof(double2);
     raise_lds_limit((const void*)trdz_reflect_kernel, lds_max);
@@ -2249,12 +2027,8 @@ void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv
     hipLaunchKernelGGL(trdz_update_kernel, dim3(tiles, tiles), dim3(256), 0, c->stream, G, ldg, P, j, yz, partz,
                        nparts, tauz);
   }
-  {
-    const int m0 = P - j0;
-    const size_t tshm = ((size_t)m0 * (m0 + 1) + 2 * (size_t)m0) * sizeof(double2);
-    raise_lds_limit((const void*)trdz_tail_lds_kernel, ((size_t)TAILZ * (TAILZ + 1) + 2 * TAILZ) * sizeof(double2));
-    hipLaunchKernelGGL(trdz_tail_lds_kernel, dim3(1), dim3(256), tshm, c->stream, G, ldg, P, j0, dv, ev, tauz);
-  }
+  trd_small(c, true, P - j0, 1, SmallEig{P - j0, j0, (long)j0 * ldg + j0, ldg, 0, 0, 0, 0}, nullptr, G, dv, ev, tauz,
+            false);
   TN_HIP(hipGetLastError());
   double* hx = (double*)c->host_stage(2 * (size_t)p * sizeof(double));
   TN_HIP(hipMemcpyAsync(hx, dv, (2 * p - 1) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -2264,6 +2038,17 @@ void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv
   // ---- 2. real divide and conquer
   double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
   std::vector<double> D = dc_tridiag(c, p, d, e, Q, stage);
+  if (P <= BACK_SMALL_MAX_Z) {
+    double2* rows = (double2*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double2));
+    const unsigned nt = (unsigned)((P + 31) / 32);
+    hipLaunchKernelGGL(reflector_rows_kernel<double2>, dim3(nt, nt), dim3(256), 0, c->stream, G, ldg, P, rows);
+    TN_HIP(hipGetLastError());
+    back_small(c, true, P, 1, SmallEig{P, 0, 0, p, 0, p, 0, ldv}, nullptr, rows, tauz, Q, Vt);
+    stage("back-transform");
+    w.assign(D.begin(), D.end());
+    TN_HIP(hipStreamSynchronize(c->stream));
+    return;
+  }
   // ---- 3. E = H_0 ... H_{p-2} Q (complex), blocks of 32 reflectors in compact WY form
   double2* V = (double2*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double2));
   double2* E = (double2*)c->workspace(WS_DC_UT, (size_t)p * p * sizeof(double2));

@@ -187,10 +187,24 @@ __device__ __forceinline__ double wave_sum64(double x) {
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
+// tau, alpha and the reflector scale of x from the sum of squares ss of x_1..
+// and x_0 (every kernel that needs them computes them this way)
+__device__ __forceinline__ void trd_reflector(double x0, double ss, double& tau, double& alpha, double& scale) {
+  tau = 0.0;
+  alpha = x0;
+  scale = 0.0;
+  if (ss > 0.0) {
+    const double nrm = sqrt(x0 * x0 + ss);
+    alpha = (x0 >= 0.0) ? -nrm : nrm;
+    tau = (alpha - x0) / alpha;
+    scale = 1.0 / (x0 - alpha);
+  }
+}
+
 // workspace slot ids (each slot is an independent grow-only buffer)
 enum WsSlot {
   WS_T1 = 0, WS_T2, WS_PSI32, WS_OUT32, WS_KRY_BASIS, WS_KRY_W, WS_KRY_PART, WS_KRY_COEF,
-  WS_SVD_X, WS_SVD_Q, WS_SVD_GRAM, WS_SVD_J, WS_SVD_CNT, WS_SVD_PAIRS, WS_SVD_S, WS_SVD_PERM,
+  WS_SVD_X, WS_SVD_Q, WS_SVD_GRAM, WS_SVD_S, WS_SVD_PERM,
   WS_SVD_SCALE, WS_PHI, WS_MISC, WS_ENV_X, WS_ENV_Y, WS_KRY_TMP,
   WS_DC_VEC, WS_DC_Q, WS_DC_SMALL, WS_DC_TMP, WS_DC_UT, WS_DC_LEVEL, WS_DC_W, WS_PROJ_X, WS_PROJ_Y, WS_PROJ_C,
   WS_QR_X, WS_QR_V, WS_QR_Q, WS_QR_R, WS_QR_S, WS_QR_W, WS_TTN_A, WS_TTN_S, WS_TTN_G, WS_TTN_P, WS_TTN_F,
@@ -382,7 +396,7 @@ void gather_rows_T(tn_ctx* c, const double* src, long ld_src, const int* perm,
                    const double* scale, long kcount, long L, double* out);
 
 // ---------------------------------------------------------------------------
-// density-matrix eigen-decomposition (two-sided block Jacobi) -- svd.hip
+// density-matrix eigen-decomposition -- svd.hip
 // ---------------------------------------------------------------------------
 struct GramEig {
   long p = 0, ppad = 0;     // Gram size (m if left, n otherwise), padded to 64
@@ -390,7 +404,6 @@ struct GramEig {
   bool cplx = false;        // complex128 data (interleaved)
   void* Vt = nullptr;       // ppad x ppad workspace: V^T (real) / V^H (complex), first p columns
   std::vector<double> w;    // eigenvalues (unsorted, length p) = weights s^2
-  int sweeps = 0;
 };
 // G = M M^H (left) or M^H M (right), plus xs * X X^H (left, X: p x kx with
 // row stride ldx, default kx) or xs * X^H X (right, X: kx x p) when X is
@@ -401,13 +414,6 @@ void gram_eig(tn_ctx* c, const void* M, long m, long n, bool left, bool cplx, Gr
 // left unchanged): out.w the eigenvalues, out.Vt rows the conjugated
 // eigenvectors (ld out.ppad), as gram_eig gives them
 void herm_eig(tn_ctx* c, const void* H, long p, long ldh, bool cplx, GramEig& out);
-// eigen-decomposition of a symmetric / Hermitian p x p device matrix G (ld
-// ldg, padding rows/columns zero); Vt (ld = padded size) receives V^T / V^H
-void sym_eig_jacobi(tn_ctx* c, void* G, long p, long ldg, void* Vt, long ldv, bool cplx, std::vector<double>& w,
-                    int* sweeps_out);
-// real symmetric p x p (3 <= p <= 16384) by Householder tridiagonalisation and
-// divide and conquer (eig_dc.hip); same contract as sym_eig_jacobi (G is
-// overwritten, Vt rows are the eigenvectors, w their eigenvalues)
 // One library call at a time per process: every C entry point holds this
 // lock for its duration (calls on different contexts from different host
 // threads are serialised; their GPU work still overlaps where it is queued
@@ -438,8 +444,33 @@ void concat3_f64(tn_ctx* c, const double* A, const long* dims, int ax, const dou
 // the start vector and receives the Ritz vector; returns the Ritz value
 double krylov_eig_op(tn_ctx* c, bool cx, long n, const std::function<void(const double*, double*)>& apply,
                      double* phi, int kdim, int maxiter, double tol, tn_krylov_info* info);
+// real symmetric p x p (1 <= p <= 16384) by Householder tridiagonalisation and
+// divide and conquer (eig_dc.hip): G (row stride ldg) is overwritten, the rows
+// of Vt are the eigenvectors, w their eigenvalues
 void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, std::vector<double>& w);
-// Hermitian p x p complex128 (interleaved, 2 <= p <= 16384): complex Householder
+
+// Blocks that one workgroup holds (eig_small.hip).  Offsets in elements from
+// the base pointers of a call: d, e, tau and eigenvalues at de, the matrix at
+// a (row stride lda), the tridiagonal's eigenvectors (columns, real) at q,
+// the block's eigenvectors (rows, conjugated when complex) at v.
+struct SmallEig {
+  int n, de;
+  long a, lda, q, ldq, v, ldv;
+};
+constexpr int TRD_SMALL_MAX = 192, TRD_SMALL_MAX_Z = 128;    // rows in one workgroup's registers
+constexpr int DC_SMALL_MAX = 128;                            // eigenvectors in one workgroup's LDS
+constexpr int BACK_SMALL_MAX = 768, BACK_SMALL_MAX_Z = 384;  // rows in the registers of one wavefront
+// Each takes nb blocks of at most nmax rows: `one` when list is null (nb = 1),
+// else the device array list.  trd_small overwrites A: reflector j (v_0 = 1)
+// in column j below the diagonal and in row j right of it; rows_only: in row
+// j, with zeros in its other columns.  back_small reads such rows.
+void trd_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, void* A, double* d,
+               double* e, void* tau, bool rows_only);
+void dc_small(tn_ctx* c, int nmax, int nb, const SmallEig& one, const SmallEig* list, const double* d, const double* e,
+              double* Q, double* lam);
+void back_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, const void* A,
+                const void* tau, const double* Q, void* V);
+// Hermitian p x p complex128 (interleaved, 1 <= p <= 16384): complex Householder
 // reduction to a real tridiagonal, the same divide and conquer, complex
 // back-transformation; Vt rows receive the conjugated eigenvectors
 void sym_eig_dc_z(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, std::vector<double>& w);
