@@ -1,20 +1,22 @@
-// Double-buffered MFMA GEMMs for the large contractions of the hot path.
+// Double-buffered MFMA GEMMs.
 //
-//  * gemm_fast<T, TA, TB>: FP64 (v_mfma_f64_16x16x4_f64) or FP32
-//    (v_mfma_f32_32x32x2_f32), 128 x 128 tiles, 4 wavefronts of 64 x 64.
+//  * gemm_fast<T, TA, TB, tile>: FP64 (v_mfma_f64_16x16x4_f64), FP32
+//    (v_mfma_f32_32x32x2_f32) or complex FP64 (four f64 MFMAs per product),
+//    square tiles of 128, 64 or 32, 4 wavefronts (2 x 2) of a quarter tile.
 //    Each operand is staged with 16-byte loads along its contiguous
 //    dimension into an LDS tile that keeps the global orientation
 //    (A: [m][k] if k is contiguous, [k][m] if m is; B: [k][n] or [n][k]),
 //    so staging never transposes; the MFMA fragment reads adapt instead.
 //    Two LDS stages: the next tile is fetched into registers while the
 //    current one feeds the MFMAs, then written to the other stage; one
-//    barrier per K tile.
+//    barrier per K tile.  The same loop runs over a list of K segments, for
+//    the grouped and the block-sparse products.
 //  * gemm_bf16x3_nt: C = A * B^T with A (M x K) and B (N x K) given as bf16
 //    hi/lo pairs (k contiguous, pre-split by split_bf16_*).  Each 32x32x16
 //    step issues lo*hi + hi*lo + hi*hi with FP32 accumulation.
-// Row strides must be multiples of the 16-byte vector width and bases
-// 16-byte aligned; the dispatcher in gemm.hip checks this and otherwise
-// uses the generic kernels.
+// Operands whose rows are 16-byte aligned with whole vectors take vector
+// loads, others element loads; any size and stride whose tile extents fit a
+// 32-bit byte offset runs here, the rest in gemm.hip.
 #include <map>
 #include <mutex>
 
@@ -22,6 +24,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace tn {
 namespace {
@@ -37,6 +40,7 @@ struct FArgs {
   const void* B; long ldb; long sB; long wB;
   void* C; long ldc; long sC;
   double alpha, beta;
+  int cA, cB;  // complex: conjugated operands
 };
 
 __device__ __forceinline__ void tile_coords2(int ntm, int ntn, int& tm, int& tn) {
@@ -54,10 +58,6 @@ __device__ __forceinline__ void tile_coords2(int ntm, int ntn, int& tm, int& tn)
   tm = first_m + (in_group % gsz);
   tn = in_group / gsz;
 }
-
-template <typename T> struct Vec;
-template <> struct Vec<double> { typedef double2 type; static constexpr int n = 2; };
-template <> struct Vec<float> { typedef float4 type; static constexpr int n = 4; };
 
 // ---------------------------------------------------------------------------
 // Tile loads through buffer resources.  A resource covers the rows of one
@@ -94,7 +94,7 @@ __device__ __forceinline__ unsigned voff(int rr, long c, long ld, long cols, int
 template <typename T, int AL>
 __device__ __forceinline__ uint4 ldvec(Rsrc r, int rr, long c, long ld, long cols) {
   constexpr int ES = (int)sizeof(T);
-  if constexpr (AL) {
+  if constexpr (AL || ES == 16) {
     return ld16(r, voff(rr, c, ld, cols, ES));
   } else if constexpr (ES == 8) {
     uint4 v;
@@ -115,11 +115,44 @@ __device__ __forceinline__ uint4 ldvec(Rsrc r, int rr, long c, long ld, long col
   }
 }
 
-template <typename T, int TA, int TB>
-struct FastCfg {
-  static constexpr int BM = 128, BN = 128;
-  static constexpr int BK = (sizeof(T) == 8) ? 16 : 32;
-  static constexpr int VN = Vec<T>::n;
+// ---------------------------------------------------------------------------
+// bf16 hi/lo split: hi = rne(x), lo = rne(x - hi); from FP64 or FP32 sources
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ unsigned short f2bf(float x) {
+  unsigned int u = __float_as_uint(x);
+  u += 0x7FFFu + ((u >> 16) & 1u);
+  return (unsigned short)(u >> 16);
+}
+__device__ __forceinline__ float bf2f_(unsigned short h) { return __uint_as_float(((unsigned int)h) << 16); }
+
+template <typename T>
+__device__ __forceinline__ void split1(T x, unsigned short& h, unsigned short& l) {
+  h = f2bf((float)x);
+  l = f2bf((float)(x - (T)bf2f_(h)));
+}
+
+// ---------------------------------------------------------------------------
+// One output tile.  T: float, double or double2 (complex).
+// Tile sizes: BM x BM outputs, K tiles of BK.  128 x 128 keeps the MFMAs busy
+// with two workgroups per CU; launch bounds of two wavefronts per SIMD keep
+// the 128 accumulator registers of the FP64 tile in place (without them the
+// compiler moved them between the two register files in every K tile: 4096^3
+// FP64 at 47 TF/s, with them 63).  64 and 32 put four and sixteen times the
+// workgroups on products with fewer tiles than CUs; they are bound by the
+// latency of a K tile, so theirs are longer.
+// ---------------------------------------------------------------------------
+template <typename T> struct Acc;
+template <> struct Acc<double> { typedef d4 type; static constexpr int MB = 16, NR = 4; };
+template <> struct Acc<float> { typedef f16v type; static constexpr int MB = 32, NR = 16; };
+struct Z4 {
+  d4 re, im;
+};
+template <> struct Acc<double2> { typedef Z4 type; static constexpr int MB = 16, NR = 4; };
+
+template <typename T, int TA, int TB, int BM_, int BK_>
+struct TileCfg {
+  static constexpr int BM = BM_, BN = BM_, BK = BK_;
+  static constexpr int VN = 16 / (int)sizeof(T);
   static constexpr int PAD = VN;  // keeps 16-byte alignment of every LDS row
   // A stage: [BM][BK+PAD] if TA == 0 else [BK][BM+PAD]
   static constexpr int A_ROWS = TA ? BK : BM, A_COLS = TA ? BM : BK, A_LD = A_COLS + PAD;
@@ -127,50 +160,73 @@ struct FastCfg {
   static constexpr int A_VECS = A_ROWS * A_COLS / VN / 256;  // per thread
   static constexpr int B_VECS = B_ROWS * B_COLS / VN / 256;
   static constexpr int A_ELEMS = A_ROWS * A_LD, B_ELEMS = B_ROWS * B_LD;
+  static constexpr int WT = BM / 2, F = WT / Acc<T>::MB;  // wave tile, MFMA blocks per side
+  static constexpr size_t LDS = 2 * (size_t)(A_ELEMS + B_ELEMS) * sizeof(T);
+  static_assert(A_VECS * VN * 256 == A_ROWS * A_COLS && B_VECS * VN * 256 == B_ROWS * B_COLS, "whole vectors");
 };
+// K tile of a tile size: 128 holds two 35 KB stages per operand pair, the
+// small tiles trade LDS for fewer barriers
+template <typename T> constexpr int tile_bk(int bm) {
+  return sizeof(T) == 8 ? (bm == 128 ? 16 : 32) : sizeof(T) == 4 ? (bm == 128 ? 32 : 32) : 16;
+}
 
-template <typename T, int TA, int TB, int AL>
-__global__ __launch_bounds__(256) void gemm_fast_kernel(FArgs a) {
-  using CF = FastCfg<T, TA, TB>;
-  constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, VN = CF::VN;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T* As = reinterpret_cast<T*>(smem);                 // 2 stages
+// acc += sum over the K segments of seg of A_s (rows m0..) * B_s (columns
+// n0..).  Seg: done(), next() and the current A, B, K, wA, wB, weight w
+// (SCALE: A_s is multiplied by w).  SPLIT: FP32 fragments as bf16 hi/lo parts.
+template <class CF, typename T, int TA, int TB, int AL, bool SCALE, bool SPLIT, class Seg>
+__device__ __forceinline__ void tile_product(Seg& seg, long M, long N, long m0, long n0, long lda, long ldb, int cA,
+                                             int cB, T* smem, typename Acc<T>::type (&acc)[CF::F][CF::F]) {
+  constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, VN = CF::VN, F = CF::F, MB = Acc<T>::MB, ES = (int)sizeof(T);
+  T* As = smem;  // 2 stages
   T* Bs = As + 2 * CF::A_ELEMS;
-
-  const int ntm = (int)((a.M + BM - 1) / BM), ntn = (int)((a.N + BN - 1) / BN);
-  int tm, tn;
-  tile_coords2(ntm, ntn, tm, tn);
-  const long m0 = (long)tm * BM, n0 = (long)tn * BN;
-  const long bz = blockIdx.z;
-  const T* A = reinterpret_cast<const T*>(a.A) + bz * a.sA;
-  const T* B = reinterpret_cast<const T*>(a.B) + bz * a.sB;
-  T* C = reinterpret_cast<T*>(a.C) + bz * a.sC;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  constexpr int ES = (int)sizeof(T);
+  const int wm = (wave >> 1) * CF::WT, wn = (wave & 1) * CF::WT;
   uint4 ra[CF::A_VECS], rb[CF::B_VECS];
-  // tile k0 of A: rows m (TA = 0, k contiguous) or rows k (TA = 1, m contiguous);
-  // a k0 past the end loads zeros (the unconditional prefetch of the last step)
-  auto gload = [&](long k0) {
-    const Rsrc ra_r = TA ? tile_rsrc(A, k0, a.K, BK, a.lda, a.wA, ES) : tile_rsrc(A, m0, a.M, BM, a.lda, a.wA, ES);
-    const Rsrc rb_r = TB ? tile_rsrc(B, n0, a.N, BN, a.ldb, a.wB, ES) : tile_rsrc(B, k0, a.K, BK, a.ldb, a.wB, ES);
+  long k0 = 0;
+  double w = 1.0;
+  // the next K tile of the current segment: rows m (TA = 0, k contiguous) or rows k (TA = 1, m contiguous)
+  auto gload = [&]() {
+    const T* A = reinterpret_cast<const T*>(seg.A);
+    const T* B = reinterpret_cast<const T*>(seg.B);
+    const Rsrc ar = TA ? tile_rsrc(A, k0, seg.K, BK, lda, seg.wA, ES) : tile_rsrc(A, m0, M, BM, lda, seg.wA, ES);
+    const Rsrc br = TB ? tile_rsrc(B, n0, N, BN, ldb, seg.wB, ES) : tile_rsrc(B, k0, seg.K, BK, ldb, seg.wB, ES);
 #pragma unroll
     for (int i = 0; i < CF::A_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::A_COLS / VN), cc = (idx % (CF::A_COLS / VN)) * VN;
-      ra[i] = TA ? ldvec<T, AL>(ra_r, rr, m0 + cc, a.lda, a.wA) : ldvec<T, AL>(ra_r, rr, k0 + cc, a.lda, a.wA);
+      ra[i] = ldvec<T, AL>(ar, rr, (TA ? m0 : k0) + cc, lda, seg.wA);
     }
 #pragma unroll
     for (int i = 0; i < CF::B_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::B_COLS / VN), cc = (idx % (CF::B_COLS / VN)) * VN;
-      rb[i] = TB ? ldvec<T, AL>(rb_r, rr, k0 + cc, a.ldb, a.wB) : ldvec<T, AL>(rb_r, rr, n0 + cc, a.ldb, a.wB);
+      rb[i] = ldvec<T, AL>(br, rr, (TB ? k0 : n0) + cc, ldb, seg.wB);
+    }
+    if constexpr (SCALE) w = seg.w;
+    k0 += BK;
+    if (k0 >= seg.K) {
+      k0 = 0;
+      seg.next();
     }
   };
   auto sstore = [&](int st) {
     T* as = As + st * CF::A_ELEMS;
     T* bs = Bs + st * CF::B_ELEMS;
+    if constexpr (SCALE) {
+#pragma unroll
+      for (int i = 0; i < CF::A_VECS; ++i) {
+        double2 v = __builtin_bit_cast(double2, ra[i]);
+        v.x *= w;
+        v.y *= w;
+        ra[i] = __builtin_bit_cast(uint4, v);
+      }
+    }
+    if constexpr (ES == 16) {  // conjugated operands: the sign of the imaginary part
+#pragma unroll
+      for (int i = 0; i < CF::A_VECS; ++i) ra[i].w ^= cA ? 0x80000000u : 0u;
+#pragma unroll
+      for (int i = 0; i < CF::B_VECS; ++i) rb[i].w ^= cB ? 0x80000000u : 0u;
+    }
 #pragma unroll
     for (int i = 0; i < CF::A_VECS; ++i) {
       const int idx = tid + i * 256;
@@ -187,105 +243,292 @@ __global__ __launch_bounds__(256) void gemm_fast_kernel(FArgs a) {
   // element (m, k) of the A stage and (k, n) of the B stage
   auto Ael = [&](const T* as, int m, int k) -> T { return TA ? as[k * CF::A_LD + m] : as[m * CF::A_LD + k]; };
   auto Bel = [&](const T* bs, int k, int n) -> T { return TB ? bs[n * CF::B_LD + k] : bs[k * CF::B_LD + n]; };
-
-  const long nk = (a.K + BK - 1) / BK;
-  if constexpr (sizeof(T) == 8) {
-    constexpr int FM = 4, FN = 4;  // 64x64 wave tile of 16x16 blocks
-    d4 acc[FM][FN];
+  auto compute = [&](int st) {
+    const T* as = As + st * CF::A_ELEMS;
+    const T* bs = Bs + st * CF::B_ELEMS;
+    if constexpr (SPLIT) {
+      // lane: row / column lane % 32, the 8 k values 8 (lane / 32) .. + 7 of every 16
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+      for (int kk = 0; kk < BK; kk += 16) {
+        const int kb = kk + 8 * (lane >> 5);
+        bf8 ah[F], al[F], bh[F], bl[F];
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = d4{0, 0, 0, 0};
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (long t = 0; t < nk; ++t) {
-      gload((t + 1) * BK);
-      __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
-      const T* as = As + (t & 1) * CF::A_ELEMS;
-      const T* bs = Bs + (t & 1) * CF::B_ELEMS;
+        for (int i = 0; i < F; ++i) {
+          us8 h, l;
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        const int kr = kk + (lane >> 4);
-        double fa[FM], fb[FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) fa[i] = Ael(as, wm * 64 + i * 16 + (lane & 15), kr);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) fb[j] = Bel(bs, kr, wn * 64 + j * 16 + (lane & 15));
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      sstore((t + 1) & 1);
-      __syncthreads();
-    }
-    // v_mfma_f64_16x16x4f64 output: register r of lane -> row lane/16 + 4r, column lane%16
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const long m = m0 + wm * 64 + i * 16 + (lane >> 4) + 4 * r;
-          const long n = n0 + wn * 64 + j * 16 + (lane & 15);
-          if (m < a.M && n < a.N) {
-            double v = a.alpha * acc[i][j][r];
-            if (a.beta != 0.0) v += a.beta * C[m * a.ldc + n];
-            C[m * a.ldc + n] = (T)v;
+          for (int q = 0; q < 8; ++q) {
+            unsigned short hq, lq;
+            split1<float>(Ael(as, wm + i * MB + (lane & 31), kb + q), hq, lq);
+            h[q] = hq;
+            l[q] = lq;
           }
+          ah[i] = __builtin_bit_cast(bf8, h);
+          al[i] = __builtin_bit_cast(bf8, l);
         }
-  } else {
-    constexpr int FM = 2, FN = 2;  // 64x64 wave tile of 32x32 blocks
-    f16v acc[FM][FN];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+        for (int j = 0; j < F; ++j) {
+          us8 h, l;
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = f16v{};
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (long t = 0; t < nk; ++t) {
-      gload((t + 1) * BK);
-      __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
-      const T* as = As + (t & 1) * CF::A_ELEMS;
-      const T* bs = Bs + (t & 1) * CF::B_ELEMS;
+          for (int q = 0; q < 8; ++q) {
+            unsigned short hq, lq;
+            split1<float>(Bel(bs, kb + q, wn + j * MB + (lane & 31)), hq, lq);
+            h[q] = hq;
+            l[q] = lq;
+          }
+          bh[j] = __builtin_bit_cast(bf8, h);
+          bl[j] = __builtin_bit_cast(bf8, l);
+        }
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+          }
+      }
+    } else if constexpr (ES == 4) {
 #pragma unroll
       for (int kk = 0; kk < BK; kk += 2) {
         const int kr = kk + (lane >> 5);
-        float fa[FM], fb[FN];
+        float fa[F], fb[F];
 #pragma unroll
-        for (int i = 0; i < FM; ++i) fa[i] = Ael(as, wm * 64 + i * 32 + (lane & 31), kr);
+        for (int i = 0; i < F; ++i) fa[i] = Ael(as, wm + i * MB + (lane & 31), kr);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) fb[j] = Bel(bs, kr, wn * 64 + j * 32 + (lane & 31));
+        for (int j = 0; j < F; ++j) fb[j] = Bel(bs, kr, wn + j * MB + (lane & 31));
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < F; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+          for (int j = 0; j < F; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      sstore((t + 1) & 1);
-      __syncthreads();
+    } else if constexpr (ES == 8) {
+#pragma unroll
+      for (int kk = 0; kk < BK; kk += 4) {
+        const int kr = kk + (lane >> 4);
+        double fa[F], fb[F];
+#pragma unroll
+        for (int i = 0; i < F; ++i) fa[i] = Ael(as, wm + i * MB + (lane & 15), kr);
+#pragma unroll
+        for (int j = 0; j < F; ++j) fb[j] = Bel(bs, kr, wn + j * MB + (lane & 15));
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < BK; kk += 4) {
+        const int kr = kk + (lane >> 4);
+        double2 fa[F], fb[F];
+#pragma unroll
+        for (int i = 0; i < F; ++i) fa[i] = Ael(as, wm + i * MB + (lane & 15), kr);
+#pragma unroll
+        for (int j = 0; j < F; ++j) fb[j] = Bel(bs, kr, wn + j * MB + (lane & 15));
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j) {
+            acc[i][j].re = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].x, fb[j].x, acc[i][j].re, 0, 0, 0);
+            acc[i][j].im = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].x, fb[j].y, acc[i][j].im, 0, 0, 0);
+            acc[i][j].re = __builtin_amdgcn_mfma_f64_16x16x4f64(-fa[i].y, fb[j].y, acc[i][j].re, 0, 0, 0);
+            acc[i][j].im = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i].y, fb[j].x, acc[i][j].im, 0, 0, 0);
+          }
+      }
     }
-    // register r of lane -> row 8*(r/4) + 4*(lane/32) + r%4, column lane%32
+  };
+  if (seg.done()) return;
+  gload();
+  sstore(0);
+  __syncthreads();
+  for (int st = 0;; st ^= 1) {
+    const bool more = !seg.done();
+    if (more) gload();
+    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
+    compute(st);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!more) break;
+    sstore(st ^ 1);
+    __syncthreads();
+  }
+}
+
+// C tile = alpha acc + beta C.  Registers of an MFMA block: f64 (complex: re
+// and im alike) register r of a lane is row lane / 16 + 4 r, column lane %
+// 16; f32 row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32.
+template <class CF, typename T>
+__device__ __forceinline__ void tile_store(T* C, long ldc, long M, long N, long m0, long n0, double alpha, double beta,
+                                           const typename Acc<T>::type (&acc)[CF::F][CF::F]) {
+  constexpr int F = CF::F, MB = Acc<T>::MB, NR = Acc<T>::NR;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long mw = m0 + (wave >> 1) * CF::WT, nw = n0 + (wave & 1) * CF::WT;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < F; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const long m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          const long n = n0 + wn * 64 + j * 32 + (lane & 31);
-          if (m < a.M && n < a.N) {
-            float v = (float)a.alpha * acc[i][j][r];
-            if (a.beta != 0.0) v += (float)a.beta * C[m * a.ldc + n];
-            C[m * a.ldc + n] = v;
+      for (int r = 0; r < NR; ++r) {
+        const long m = mw + i * MB + (MB == 32 ? 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) : (lane >> 4) + 4 * r);
+        const long n = nw + j * MB + (lane & (MB - 1));
+        if (m < M && n < N) {
+          T* p = C + m * ldc + n;
+          if constexpr (std::is_same<T, double2>::value) {
+            double2 v = make_double2(alpha * acc[i][j].re[r], alpha * acc[i][j].im[r]);
+            if (beta != 0.0) {
+              const double2 o = *p;
+              v.x += beta * o.x;
+              v.y += beta * o.y;
+            }
+            *p = v;
+          } else {
+            T v = (T)alpha * acc[i][j][r];
+            if (beta != 0.0) v += (T)beta * *p;
+            *p = v;
           }
         }
+      }
+}
+
+template <class CF, typename T>
+__device__ __forceinline__ void tile_zero(typename Acc<T>::type (&acc)[CF::F][CF::F]) {
+#pragma unroll
+  for (int i = 0; i < CF::F; ++i)
+#pragma unroll
+    for (int j = 0; j < CF::F; ++j) acc[i][j] = typename Acc<T>::type{};
+}
+
+struct OneSeg {  // a plain product: one segment
+  const void* A;
+  const void* B;
+  long K, wA, wB;
+  bool end;
+  __device__ __forceinline__ bool done() const { return end; }
+  __device__ __forceinline__ void next() { end = true; }
+};
+
+template <typename T, int TA, int TB, int AL, int BM>
+__global__ __launch_bounds__(256, 2) void gemm_fast_kernel(FArgs a) {
+  using CF = TileCfg<T, TA, TB, BM, tile_bk<T>(BM)>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int ntm = (int)((a.M + BM - 1) / BM), ntn = (int)((a.N + BM - 1) / BM);
+  int tm, tn;
+  tile_coords2(ntm, ntn, tm, tn);
+  const long m0 = (long)tm * BM, n0 = (long)tn * BM, bz = blockIdx.z;
+  OneSeg seg{reinterpret_cast<const T*>(a.A) + bz * a.sA, reinterpret_cast<const T*>(a.B) + bz * a.sB, a.K, a.wA, a.wB,
+             a.K <= 0};
+  typename Acc<T>::type acc[CF::F][CF::F];
+  tile_zero<CF, T>(acc);
+  tile_product<CF, T, TA, TB, AL, false, false>(seg, a.M, a.N, m0, n0, a.lda, a.ldb, a.cA, a.cB,
+                                                reinterpret_cast<T*>(smem), acc);
+  tile_store<CF, T>(reinterpret_cast<T*>(a.C) + bz * a.sC, a.ldc, a.M, a.N, m0, n0, a.alpha, a.beta, acc);
+}
+
+// ---------------------------------------------------------------------------
+// Grouped FP64 GEMM: output group g (grid y) and batch z (grid z) accumulate
+// sum over the terms t of group g of w_t A_{ia_t} B_{ib_t}, every term an
+// M x N x K product; the output tile is written once (no read of C).  The
+// terms are the K segments of one tile loop, so the next term's first tile
+// is on its way while a term ends.
+// ---------------------------------------------------------------------------
+struct TermSeg {
+  const GroupedDesc& g;
+  const double* A0;
+  const double* B0;
+  const void* A;
+  const void* B;
+  long K, wA, wB;
+  double w;
+  int t, t1;
+  __device__ __forceinline__ void set() {
+    if (t < t1) {
+      A = A0 + (long)g.ia[t] * g.tsA;
+      B = B0 + (long)g.ib[t] * g.tsB;
+      w = g.w[t];
+    }
   }
+  __device__ __forceinline__ bool done() const { return t >= t1; }
+  __device__ __forceinline__ void next() {
+    ++t;
+    set();
+  }
+};
+
+template <int AL, int BM>
+__global__ __launch_bounds__(256, 2) void gemm_grouped_kernel(GroupedDesc d) {
+  using CF = TileCfg<double, 0, 0, BM, tile_bk<double>(BM)>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  int tm, tn;
+  tile_coords2((int)((d.M + BM - 1) / BM), (int)((d.N + BM - 1) / BM), tm, tn);
+  const long m0 = (long)tm * BM, n0 = (long)tn * BM, z = blockIdx.z;
+  const int g = blockIdx.y;
+  TermSeg seg{d, d.A + z * d.sA, d.B + z * d.sB, nullptr, nullptr, d.K, d.K, d.N, 0.0, d.off[g], d.off[g + 1]};
+  if (d.K <= 0) seg.t = seg.t1;
+  seg.set();
+  d4 acc[CF::F][CF::F];
+  tile_zero<CF, double>(acc);
+  tile_product<CF, double, 0, 0, AL, true, false>(seg, d.M, d.N, m0, n0, d.lda, d.ldb, 0, 0,
+                                                  reinterpret_cast<double*>(smem), acc);
+  tile_store<CF, double>(d.C + (long)g * d.gsC + z * d.sC, d.ldc, d.M, d.N, m0, n0, 1.0, 0.0, acc);
+}
+
+// ---------------------------------------------------------------------------
+// Block-sparse GEMM over uneven blocks (QN sectors): one launch covers a list
+// of output tiles; tile t belongs to task tiles[t].x, whose output block
+// C + c_off (M x N, ld ldc) is the sum over the task's K segments of
+// A_s (M x K_s, ld lda) * B_s (K_s x N, ld ldb), A_s = A + a_off, B_s = B +
+// b_off.  A task without segments writes zeros.  The tile list is laid out
+// XCD-major: workgroup id i runs list entry (i % 8) * per + i / 8, so the
+// contiguous run of tiles one XCD runs shares its tasks' A and B panels in
+// that XCD's L2; padding entries (task < 0) exit at once.  Blocks start at
+// any element, so the operands take element loads.
+// SPLIT (FP32 operands only): each FP32 fragment is split into bf16 hi/lo
+// parts in registers and the product accumulates lo*hi + hi*lo + hi*hi with
+// the bf16 MFMA 32x32x16.
+// ---------------------------------------------------------------------------
+struct BlockSeg {
+  const BsSeg* segs;
+  const char* A0;
+  const char* B0;
+  int es, tB;
+  long N;
+  const void* A;
+  const void* B;
+  long K, wA, wB;
+  int s, s1;
+  __device__ __forceinline__ void set() {
+    while (s < s1) {
+      const BsSeg g = segs[s];
+      A = A0 + g.a_off * es;
+      B = B0 + g.b_off * es;
+      K = wA = g.K;
+      wB = tB ? g.K : N;
+      if (K > 0) return;
+      ++s;
+    }
+  }
+  __device__ __forceinline__ bool done() const { return s >= s1; }
+  __device__ __forceinline__ void next() {
+    ++s;
+    set();
+  }
+};
+
+template <typename T, int TB, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void gemm_bs_kernel(BsDesc d) {
+  using CF = TileCfg<T, 0, TB, BS_TILE, SPLIT ? 16 : tile_bk<T>(BS_TILE)>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int4 tl = d.tiles[(long)(blockIdx.x % 8) * (d.ntiles / 8) + blockIdx.x / 8];
+  if (tl.x < 0) return;
+  const BsTask tk = d.tasks[tl.x];
+  BlockSeg seg{d.segs, reinterpret_cast<const char*>(d.A), reinterpret_cast<const char*>(d.B), (int)sizeof(T), TB,
+               tk.N, nullptr, nullptr, 0, 0, 0, tk.seg0, tk.seg0 + tk.nseg};
+  seg.set();
+  typename Acc<T>::type acc[CF::F][CF::F];
+  tile_zero<CF, T>(acc);
+  tile_product<CF, T, 0, TB, 0, false, SPLIT>(seg, tk.M, tk.N, tl.y, tl.z, d.lda, d.ldb, 0, 0,
+                                              reinterpret_cast<T*>(smem), acc);
+  tile_store<CF, T>(reinterpret_cast<T*>(d.C) + tk.c_off, d.ldc, tk.M, tk.N, tl.y, tl.z, d.alpha, 0.0, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -411,22 +654,6 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_nt_kernel(SArgs a) {
       }
 }
 
-// ---------------------------------------------------------------------------
-// bf16 hi/lo split: hi = rne(x), lo = rne(x - hi); from FP64 or FP32 sources
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ unsigned short f2bf(float x) {
-  unsigned int u = __float_as_uint(x);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
-__device__ __forceinline__ float bf2f_(unsigned short h) { return __uint_as_float(((unsigned int)h) << 16); }
-
-template <typename T>
-__device__ __forceinline__ void split1(T x, unsigned short& h, unsigned short& l) {
-  h = f2bf((float)x);
-  l = f2bf((float)(x - (T)bf2f_(h)));
-}
-
 // dst[r][c] (ld_dst) = split(src[r][c]); columns cols..ld_dst-1 zeroed
 template <typename T>
 __global__ __launch_bounds__(256) void split_rows_kernel(const T* __restrict__ src, long rows, long cols,
@@ -497,75 +724,158 @@ void raise_lds_limit(const void* fn, size_t bytes) {
 }
 static void allow_lds(const void* fn, size_t bytes) { raise_lds_limit(fn, bytes); }
 
-// operands whose rows are 16-byte aligned with a valid width of whole
-// vectors take the vector loads; any other operand takes element loads
 // readable row widths of A and B: the valid width, rounded up to whole
 // vectors for an operand the caller marks zero-padded
+static int vec_elems(Prec p) { return p == Prec::F64 ? 2 : p == Prec::Z64 ? 1 : 4; }
+static size_t elem_bytes(Prec p) { return p == Prec::F64 ? 8 : p == Prec::Z64 ? 16 : 4; }
 static long width_a(Prec p, const GemmDesc& g) {
-  const int vn = (p == Prec::F64) ? 2 : 4;
+  const int vn = vec_elems(p);
   if (g.tA) return g.M;
   return g.zpA ? (g.K + vn - 1) / vn * vn : g.K;
 }
 static long width_b(Prec p, const GemmDesc& g) {
-  const int vn = (p == Prec::F64) ? 2 : 4;
+  const int vn = vec_elems(p);
   if (g.tB) return g.K;
   return g.zpB ? (g.N + vn - 1) / vn * vn : g.N;
 }
+// operands whose rows are 16-byte aligned with a valid width of whole
+// vectors take the vector loads; any other operand takes element loads
 static bool fast_aligned(Prec p, const GemmDesc& g) {
-  const int vn = (p == Prec::F64) ? 2 : 4;
+  const int vn = vec_elems(p);
   auto al = [&](const void* ptr, long ld, long s, long cols) {
     return ((uintptr_t)ptr % 16 == 0) && (ld % vn == 0) && (s % vn == 0) && (cols % vn == 0) && cols <= ld;
   };
   return al(g.A, g.lda, g.sA, width_a(p, g)) && al(g.B, g.ldb, g.sB, width_b(p, g));
 }
 
-bool gemm_fast_ok(Prec p, const GemmDesc& g) {
-  if (p != Prec::F64 && p != Prec::F32) return false;
-  if (g.cA || g.cB) return false;
-  if (g.M < 128 || g.N < 128 || g.K < 16) return false;
-  const size_t es = (p == Prec::F64) ? 8 : 4;
-  // a 128-row tile must span less than 2^31 bytes (32-bit buffer offsets)
-  return (size_t)g.lda * es * 130 < ((size_t)1 << 31) && (size_t)g.ldb * es * 130 < ((size_t)1 << 31);
+// a tile of up to 128 rows must span less than 2^31 bytes (32-bit buffer offsets)
+static bool extent_ok(long ld, long rows, size_t es) {
+  return (size_t)ld * es * (size_t)(std::min(rows, 130L) + 1) < ((size_t)1 << 31);
 }
+
+bool gemm_fast_ok(Prec p, const GemmDesc& g) {
+  if (p != Prec::F64 && p != Prec::F32 && p != Prec::Z64) return false;
+  if (p == Prec::Z64 && ((uintptr_t)g.A % 16 != 0 || (uintptr_t)g.B % 16 != 0)) return false;
+  const size_t es = elem_bytes(p);
+  return extent_ok(g.lda, g.tA ? g.K : g.M, es) && extent_ok(g.ldb, g.tB ? g.N : g.K, es);
+}
+
+// Tile of an M x N product over a batch: the one with the least work on the
+// busiest CU, tiles / 256 rounds of b^2 outputs each, weighted by how well a
+// tile size keeps the MFMAs fed (measured on full grids: FP64 128 63 TF/s,
+// 64 55, 32 30; complex 64 about the same as 32 with a quarter of the loads).
+// Complex products and FP32 have no 128 / 32 tile respectively.
+static int pick_tile(Prec p, long M, long N, long batch) {
+  int best = 0;
+  double cost = 0.0;
+  for (int b : {128, 64, 32}) {
+    if ((p == Prec::Z64 && b == 128) || (p == Prec::F32 && b == 32)) continue;
+    const double eff = b == 128 ? 1.0 : b == 64 ? 0.87 : 0.5;
+    const long tiles = ((M + b - 1) / b) * ((N + b - 1) / b) * batch;
+    const double t = (double)((tiles + 255) / 256) * b * b / eff;
+    if (best == 0 || t < cost) {
+      best = b;
+      cost = t;
+    }
+  }
+  return best;
+}
+
+namespace {
+template <typename T, int TA, int TB, int AL, int BM>
+void launch_tile(tn_ctx* c, const FArgs& a, int batch) {
+  constexpr size_t shm = TileCfg<T, TA, TB, BM, tile_bk<T>(BM)>::LDS;
+  const long tiles = ((a.M + BM - 1) / BM) * ((a.N + BM - 1) / BM);
+  TN_REQUIRE(tiles < (1L << 31), TN_E_INVALID, "gemm: too many tiles");
+  allow_lds((const void*)gemm_fast_kernel<T, TA, TB, AL, BM>, shm);
+  hipLaunchKernelGGL((gemm_fast_kernel<T, TA, TB, AL, BM>), dim3((unsigned)tiles, 1, (unsigned)batch), dim3(256), shm,
+                     c->stream, a);
+}
+template <typename T, int TA, int TB, int AL>
+void launch_bm(tn_ctx* c, const FArgs& a, int batch, int bm) {
+  if constexpr (sizeof(T) != 16)
+    if (bm == 128) return launch_tile<T, TA, TB, AL, 128>(c, a, batch);
+  if constexpr (sizeof(T) != 4)
+    if (bm == 32) return launch_tile<T, TA, TB, AL, 32>(c, a, batch);
+  launch_tile<T, TA, TB, AL, 64>(c, a, batch);
+}
+template <typename T, int AL>
+void launch_ops(tn_ctx* c, const FArgs& a, const GemmDesc& g, int bm) {
+  if (!g.tA && !g.tB) launch_bm<T, 0, 0, AL>(c, a, g.batch, bm);
+  else if (g.tA && !g.tB) launch_bm<T, 1, 0, AL>(c, a, g.batch, bm);
+  else if (!g.tA && g.tB) launch_bm<T, 0, 1, AL>(c, a, g.batch, bm);
+  else launch_bm<T, 1, 1, AL>(c, a, g.batch, bm);
+}
+}  // namespace
 
 void gemm_fast(tn_ctx* c, Prec p, const GemmDesc& g) {
   FArgs a;
   a.M = g.M; a.N = g.N; a.K = g.K;
   const bool aligned = fast_aligned(p, g);
-  a.A = g.A; a.lda = g.lda; a.sA = g.sA;
-  a.B = g.B; a.ldb = g.ldb; a.sB = g.sB;
+  a.A = g.A; a.lda = g.lda; a.sA = g.sA; a.cA = g.cA;
+  a.B = g.B; a.ldb = g.ldb; a.sB = g.sB; a.cB = g.cB;
   // the vector kernel reads the padded widths; the element kernel the valid ones
   a.wA = aligned ? width_a(p, g) : (g.tA ? g.M : g.K);
   a.wB = aligned ? width_b(p, g) : (g.tB ? g.K : g.N);
   a.C = g.C; a.ldc = g.ldc; a.sC = g.sC;
   a.alpha = g.alpha; a.beta = g.beta;
-  const long ntm = (g.M + 127) / 128, ntn = (g.N + 127) / 128;
-  dim3 grid((unsigned)(ntm * ntn), 1, (unsigned)g.batch);
-#define TN_LAUNCH_FAST1(T, TA, TB, AL)                                                               \
-  do {                                                                                               \
-    using CF = FastCfg<T, TA, TB>;                                                                   \
-    const size_t shm = 2 * (size_t)(CF::A_ELEMS + CF::B_ELEMS) * sizeof(T);                          \
-    allow_lds((const void*)gemm_fast_kernel<T, TA, TB, AL>, shm);                                    \
-    hipLaunchKernelGGL((gemm_fast_kernel<T, TA, TB, AL>), grid, dim3(256), shm, c->stream, a);       \
-  } while (0)
-#define TN_LAUNCH_FAST(T, TA, TB)                 \
-  do {                                            \
-    if (aligned) TN_LAUNCH_FAST1(T, TA, TB, 1);   \
-    else TN_LAUNCH_FAST1(T, TA, TB, 0);           \
-  } while (0)
+  const int bm = pick_tile(p, g.M, g.N, g.batch);
+  if (p == Prec::Z64) launch_ops<double2, 1>(c, a, g, bm);
+  else if (p == Prec::F64 && aligned) launch_ops<double, 1>(c, a, g, bm);
+  else if (p == Prec::F64) launch_ops<double, 0>(c, a, g, bm);
+  else if (aligned) launch_ops<float, 1>(c, a, g, bm);
+  else launch_ops<float, 0>(c, a, g, bm);
+  TN_HIP(hipGetLastError());
+}
+
+void gemm_grouped_f64(tn_ctx* c, const GroupedDesc& d) {
+  if (d.M <= 0 || d.N <= 0 || d.ngroups <= 0 || d.batch <= 0) return;
+  TN_REQUIRE(d.ngroups <= 65535 && d.batch <= 65535, TN_E_INVALID, "grouped gemm: grid too large");
+  TN_REQUIRE(extent_ok(d.lda, d.M, 8) && extent_ok(d.ldb, d.K, 8), TN_E_INVALID, "grouped gemm: row stride too large");
+  const int bm = std::min(64, pick_tile(Prec::F64, d.M, d.N, (long)d.ngroups * d.batch));
+  const long tiles = ((d.M + bm - 1) / bm) * ((d.N + bm - 1) / bm);
+  TN_REQUIRE(tiles < (1L << 31), TN_E_INVALID, "grouped gemm: too many tiles");
+  const bool al = (uintptr_t)d.A % 16 == 0 && (uintptr_t)d.B % 16 == 0 &&
+                  ((d.lda | d.sA | d.tsA | d.K | d.ldb | d.sB | d.tsB | d.N) & 1) == 0;
+  const dim3 gr((unsigned)tiles, (unsigned)d.ngroups, (unsigned)d.batch);
+  auto launch = [&](auto kern, size_t shm) {
+    allow_lds((const void*)kern, shm);
+    hipLaunchKernelGGL(kern, gr, dim3(256), shm, c->stream, d);
+  };
+  constexpr size_t s64 = TileCfg<double, 0, 0, 64, tile_bk<double>(64)>::LDS;
+  constexpr size_t s32 = TileCfg<double, 0, 0, 32, tile_bk<double>(32)>::LDS;
+  if (bm == 64 && al) launch(gemm_grouped_kernel<1, 64>, s64);
+  else if (bm == 64) launch(gemm_grouped_kernel<0, 64>, s64);
+  else if (al) launch(gemm_grouped_kernel<1, 32>, s32);
+  else launch(gemm_grouped_kernel<0, 32>, s32);
+  TN_HIP(hipGetLastError());
+}
+
+void gemm_blocksparse(tn_ctx* c, Prec p, const BsDesc& d) {
+  if (d.ntiles <= 0) return;
+  TN_REQUIRE(p == Prec::F64 || p == Prec::F32 || p == Prec::BF16X3, TN_E_INVALID,
+             "block-sparse gemm: FP64, FP32 or BF16x3 (FP32 operands) only");
+  TN_REQUIRE(d.ntiles % 8 == 0 && d.ntiles < (1L << 31), TN_E_INVALID, "block-sparse gemm: bad tile list");
+  const size_t es = p == Prec::F64 ? 8 : 4;
+  TN_REQUIRE(extent_ok(d.lda, BS_TILE, es) && extent_ok(d.ldb, BS_TILE, es), TN_E_INVALID,
+             "block-sparse gemm: row stride too large");
+  auto launch = [&](auto kern, size_t shm) {
+    allow_lds((const void*)kern, shm);
+    hipLaunchKernelGGL(kern, dim3((unsigned)d.ntiles), dim3(256), shm, c->stream, d);
+  };
+#define TN_BS(T, TB, SPLIT) \
+  launch(gemm_bs_kernel<T, TB, SPLIT>, TileCfg<T, 0, TB, BS_TILE, SPLIT ? 16 : tile_bk<T>(BS_TILE)>::LDS)
   if (p == Prec::F64) {
-    if (!g.tA && !g.tB) TN_LAUNCH_FAST(double, 0, 0);
-    else if (g.tA && !g.tB) TN_LAUNCH_FAST(double, 1, 0);
-    else if (!g.tA && g.tB) TN_LAUNCH_FAST(double, 0, 1);
-    else TN_LAUNCH_FAST(double, 1, 1);
+    if (d.tB) TN_BS(double, 1, false);
+    else TN_BS(double, 0, false);
+  } else if (p == Prec::F32) {
+    if (d.tB) TN_BS(float, 1, false);
+    else TN_BS(float, 0, false);
   } else {
-    if (!g.tA && !g.tB) TN_LAUNCH_FAST(float, 0, 0);
-    else if (g.tA && !g.tB) TN_LAUNCH_FAST(float, 1, 0);
-    else if (!g.tA && g.tB) TN_LAUNCH_FAST(float, 0, 1);
-    else TN_LAUNCH_FAST(float, 1, 1);
+    if (d.tB) TN_BS(float, 1, true);
+    else TN_BS(float, 0, true);
   }
-#undef TN_LAUNCH_FAST
-#undef TN_LAUNCH_FAST1
+#undef TN_BS
   TN_HIP(hipGetLastError());
 }
 

@@ -265,7 +265,7 @@ struct GroupedDesc {
   int ngroups = 0, batch = 1;
 };
 void gemm_grouped_f64(tn_ctx* c, const GroupedDesc& d);
-// Block-sparse GEMM over uneven blocks (gemm.hip): task i writes the block
+// Block-sparse GEMM over uneven blocks (gemm_fast.hip): task i writes the block
 // C + c_off (M x N, ld ldc) = alpha * sum over its segments s of
 // (A + a_off_s)(M x K_s, ld lda) * (B + b_off_s)(K_s x N, ld ldb); a task
 // without segments writes zeros.  tiles (device) lists {task, m0, n0, 0} of
@@ -292,8 +292,8 @@ struct BsDesc {
   double alpha = 1.0;
 };
 void gemm_blocksparse(tn_ctx* c, Prec p, const BsDesc& d);
-// double-buffered FP64/FP32 kernels (gemm_fast.hip); gemm() uses them when
-// gemm_fast_ok() holds (shapes >= one tile, 16-byte aligned operand rows)
+// double-buffered kernels (gemm_fast.hip); gemm() uses them when
+// gemm_fast_ok() holds (tile extents below 2^31 bytes)
 bool gemm_fast_ok(Prec p, const GemmDesc& g);
 void gemm_fast(tn_ctx* c, Prec p, const GemmDesc& g);
 // C (M x N, float) = A * B^T with A (M x K) and B (N x K) as bf16 hi/lo
