@@ -5,6 +5,8 @@
 // gather / transpose kernels used by the truncated SVD.
 #include "tn_internal.h"
 
+#include <type_traits>
+
 #include <cmath>
 
 namespace tn {
@@ -109,129 +111,138 @@ __global__ __launch_bounds__(256) void wstep_vec_kernel(int G, int Gp, int D, in
   }
 }
 
-// The W step of a dense operator (a compressed MPO pair: every output row
-// mixes most of the (w, S) inputs) as an MFMA product per workgroup:
-// out[(g', S'), cols] = Op[(g', S'), (g, S)] * slab[(g, S), cols] for one A
-// index and WM_NB columns.  Op (Mp x Kp, zero-padded) and the input slab
-// (Kp x WM_NB) sit in LDS; each wave owns 32 output columns and all row
-// blocks (FP32: v_mfma_f32_32x32x2f32, FP64: v_mfma_f64_16x16x4f64).
-constexpr int WM_NB = 128;
+// The W step as an MFMA product: out[(g', S'), cols] = Op[(g', S'), (g, S)] *
+// in[(g, S), cols] for one A index and a strip of columns.  Bound by HBM (the
+// input read once, the output written once): the operator sits in LDS, and
+// each wavefront streams strips on its own, without barriers: input rows go
+// straight from global memory into MFMA operands (two columns per lane, five
+// K steps on their way while five are multiplied) and the results straight
+// out.  All output rows of a strip are accumulated at once (NMB blocks of 32
+// rows, v_mfma_f32_32x32x2f32, or 16, v_mfma_f64_16x16x4f64).  A sparse
+// operator costs its full M x K here and still stays under the HBM time.
+// K runs from the operator's last column to its first.  In place of a
+// workgroup per 128 columns that staged operator and input in LDS, with the
+// w = 20 pair operator: FP32 to bf16 pairs at chi = 2048 2.46 -> 0.85 ms
+// (1.4 -> 4.0 TB/s), FP32 at chi = 4096 8.0 -> 2.65 ms, FP64 at chi = 255 39 ->
+// 33 us (22 where pairs of columns are aligned).  In place of CSR rows from
+// LDS: w = 5 at chi = 16 6.4 -> 4.7 us.
+// SPLIT (T = float): the result goes out as bf16 hi/lo pairs (ohi, olo).
+// VEC: nB and all strides are even and the bases two-element aligned.
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int WM_PF = 5;  // K steps per group of loads
 
-// SPLIT (T = float): the result goes out as bf16 hi/lo pairs (ohi, olo).
-template <typename T, bool SPLIT>
-__global__ __launch_bounds__(256) void wstep_mfma_kernel(int G, int Gp, int D, int Dp, long nB,
-                                                         const T* __restrict__ in, long in_sg, long in_sA,
-                                                         long in_sS, T* __restrict__ out, long out_sg,
-                                                         long out_sA, long out_sS, const T* __restrict__ opd,
-                                                         int Mp, int Kp, unsigned short* __restrict__ ohi,
-                                                         unsigned short* __restrict__ olo, int vecin) {
+template <typename T>
+struct WmArgs {
+  int D, Dp, M, K, Kp;
+  long nA, nB;
+  unsigned nbt, strips;  // strips per A index, in all
+  const T* in; long in_sg, in_sA, in_sS;
+  T* out; long out_sg, out_sA, out_sS;
+  const T* opd;
+  unsigned short* ohi;
+  unsigned short* olo;
+};
+
+template <typename T, bool SPLIT, bool VEC, int NMB>
+__global__ __launch_bounds__(256, 2) void wstep_mfma_kernel(WmArgs<T> w) {
   constexpr bool F64 = sizeof(T) == 8;
-  constexpr int VN = 16 / (int)sizeof(T);  // elements per 16-byte vector
-  typedef T vec_t __attribute__((ext_vector_type(VN)));
-  extern __shared__ unsigned char smem_raw[];
-  const int M = Gp * Dp, K = G * D;
-  const int lda = Kp + 1;
-  T* Aop = reinterpret_cast<T*>(smem_raw);  // Mp x lda
-  T* slab = Aop + Mp * lda;                 // Kp x WM_NB
+  constexpr int MB = F64 ? 16 : 32, KS = F64 ? 4 : 2, NR = F64 ? 4 : 16, MP = NMB * MB;
+  typedef T vec2 __attribute__((ext_vector_type(2)));
+  typedef typename std::conditional<F64, d4, f16v>::type Acc;
+  extern __shared__ __attribute__((aligned(16))) unsigned char wm_smem[];
+  const int lda = w.Kp + 1;
+  long* ioff = reinterpret_cast<long*>(wm_smem);  // Kp: input row offsets
+  long* ooff = ioff + w.Kp;                       // MP: output row offsets
+  T* Aop = reinterpret_cast<T*>(ooff + MP);       // MP x lda
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const long Ai = blockIdx.y;
-  const long B0 = (long)blockIdx.x * WM_NB;
-  for (int t = tid; t < Mp * Kp; t += 256) {
-    const int m = t / Kp, k = t % Kp;
-    Aop[m * lda + k] = (m < M && k < K) ? opd[m * K + k] : T(0);
-  }
-  if (vecin) {  // 16-byte loads: strides, nB and the input base are whole vectors
-    for (int t = tid; t < Kp * (WM_NB / VN); t += 256) {
-      const int i = t / (WM_NB / VN), col = (t % (WM_NB / VN)) * VN;
-      vec_t v = (vec_t)(T(0));
-      if (i < K && B0 + col < nB) {
-        const int g = i / D, S = i % D;
-        v = *reinterpret_cast<const vec_t*>(in + g * in_sg + Ai * in_sA + S * in_sS + B0 + col);
-      }
-      *reinterpret_cast<vec_t*>(slab + i * WM_NB + col) = v;
-    }
-  } else {
-    for (int t = tid; t < Kp * WM_NB; t += 256) {
-      const int i = t / WM_NB, col = t % WM_NB;
-      T v = T(0);
-      if (i < K && B0 + col < nB) {
-        const int g = i / D, S = i % D;
-        v = in[g * in_sg + Ai * in_sA + S * in_sS + B0 + col];
-      }
-      slab[i * WM_NB + col] = v;
-    }
-  }
+  const int ln = lane & (MB - 1), kg = lane / MB;
+  const int nks = w.Kp / KS;
+  const unsigned step = gridDim.x * 4;
+  // offset of K index i's input row (the padding meets zero operator columns), a strip's
+  // first column and one K step of its input at row offset off: this lane's two
+  // columns, those past the end clamped (and not stored)
+  auto row_offset = [&](int i) -> long {
+    const int r = min(w.Kp - 1 - i, w.K - 1);
+    return (r / w.D) * w.in_sg + (r % w.D) * w.in_sS;
+  };
+  auto first_col = [&](unsigned s) -> long { return (long)(s % w.nbt) * (2 * MB); };
+  auto load = [&](unsigned s, long off) -> vec2 {
+    const T* p = w.in + (s / w.nbt) * w.in_sA + off;
+    const long c0 = first_col(s) + (VEC ? 2 * ln : ln);
+    if constexpr (VEC) return *reinterpret_cast<const vec2*>(p + min(c0, w.nB - 2));
+    else return vec2{p[min(c0, w.nB - 1)], p[min(c0 + MB, w.nB - 1)]};
+  };
+  // the first strip's first rows are on their way while the operator is staged
+  unsigned s = blockIdx.x * 4 + wave;
+  vec2 cur[WM_PF], nxt[WM_PF];
+#pragma unroll
+  for (int p = 0; p < WM_PF; ++p) cur[p] = load(min(s, w.strips - 1), row_offset(p * KS + kg));
+  for (int m = wave; m < MP; m += 4)
+    for (int k = lane; k < w.Kp; k += 64) Aop[m * lda + (w.Kp - 1 - k)] = (m < w.M && k < w.K) ? w.opd[m * w.K + k] : T(0);
+  for (int i = tid; i < w.Kp; i += 256) ioff[i] = row_offset(i);
+  for (int i = tid; i < MP; i += 256) ooff[i] = (i / w.Dp) * w.out_sg + (i % w.Dp) * w.out_sS;
   __syncthreads();
-  if constexpr (!F64) {
-    const int nmb = Mp / 32;  // <= 4
-    f16v acc[4];
+  const T* arow = Aop + ln * lda + kg;
+  for (; s < w.strips; s += step) {
+    const unsigned Ai = s / w.nbt;
+    const long c0 = first_col(s) + (VEC ? 2 * ln : ln), c1 = VEC ? c0 + 1 : c0 + MB;
+    Acc acc[NMB][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = f16v{};
-    for (int k0 = 0; k0 < Kp; k0 += 2) {
-      const int kr = k0 + (lane >> 5);
-      const float bv = slab[kr * WM_NB + wave * 32 + (lane & 31)];
+    for (int i = 0; i < NMB; ++i) acc[i][0] = acc[i][1] = Acc{};
+    for (int k0 = 0; k0 < nks; k0 += WM_PF) {
+      // the next group of rows, or the next strip's first
+      const bool last = k0 + WM_PF >= nks;
+      const unsigned sn = last ? min(s + step, w.strips - 1) : s;
+      const int kn = last ? 0 : k0 + WM_PF;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (i < nmb) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(Aop[(i * 32 + (lane & 31)) * lda + kr], bv,
-                                                                   acc[i], 0, 0, 0);
-    }
-    // register r of lane: row 8(r/4) + 4(lane/32) + r%4, column lane%32
+      for (int p = 0; p < WM_PF; ++p) nxt[p] = load(sn, ioff[(kn + p) * KS + kg]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i >= nmb) continue;
+      for (int p = 0; p < WM_PF; ++p) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const long col = B0 + wave * 32 + (lane & 31);
-        if (row < M && col < nB) {
-          const int gp = row / Dp, Sp = row % Dp;
-          const long off = gp * out_sg + Ai * out_sA + Sp * out_sS + col;
-          if constexpr (SPLIT) {
-            const float x = acc[i][r];
-            const unsigned short h = f2bf_rne(x);
-            ohi[off] = h;
-            olo[off] = f2bf_rne(x - __uint_as_float(((unsigned int)h) << 16));
+        for (int i = 0; i < NMB; ++i) {
+          const T av = arow[i * MB * lda + (k0 + p) * KS];
+          if constexpr (F64) {
+            acc[i][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, cur[p][0], acc[i][0], 0, 0, 0);
+            acc[i][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, cur[p][1], acc[i][1], 0, 0, 0);
           } else {
-            out[off] = acc[i][r];
+            acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, cur[p][0], acc[i][0], 0, 0, 0);
+            acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, cur[p][1], acc[i][1], 0, 0, 0);
           }
         }
       }
+#pragma unroll
+      for (int p = 0; p < WM_PF; ++p) cur[p] = nxt[p];
     }
-  } else {
-    const int nmb = Mp / 16;  // <= 8
-    d4 acc[8][2];
+    // register r of a lane: f64 row lane / 16 + 4 r; f32 row 8 (r / 4) + 4 (lane / 32) + r % 4
+    const long obase = Ai * w.out_sA;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i][0] = acc[i][1] = d4{0, 0, 0, 0};
-    for (int k0 = 0; k0 < Kp; k0 += 4) {
-      const int kr = k0 + (lane >> 4);
-      const double b0 = slab[kr * WM_NB + wave * 32 + (lane & 15)];
-      const double b1 = slab[kr * WM_NB + wave * 32 + 16 + (lane & 15)];
+    for (int i = 0; i < NMB; ++i)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (i >= nmb) continue;
-        const double av = Aop[(i * 16 + (lane & 15)) * lda + kr];
-        acc[i][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b0, acc[i][0], 0, 0, 0);
-        acc[i][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b1, acc[i][1], 0, 0, 0);
-      }
-    }
-    // register r of lane: row lane/16 + 4r, column lane%16
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i >= nmb) continue;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = i * 16 + (lane >> 4) + 4 * r;
-          const long col = B0 + wave * 32 + j * 16 + (lane & 15);
-          if (row < M && col < nB) {
-            const int gp = row / Dp, Sp = row % Dp;
-            out[gp * out_sg + Ai * out_sA + Sp * out_sS + col] = acc[i][j][r];
+      for (int r = 0; r < NR; ++r) {
+        const int row = i * MB + (F64 ? kg + 4 * r : 8 * (r >> 2) + 4 * kg + (r & 3));
+        const long off = ooff[row] + obase;
+        const T x0 = acc[i][0][r], x1 = acc[i][1][r];
+        if constexpr (SPLIT) {
+          const unsigned short h0 = f2bf_rne(x0), h1 = f2bf_rne(x1);
+          const unsigned short l0 = f2bf_rne(x0 - __uint_as_float(((unsigned int)h0) << 16));
+          const unsigned short l1 = f2bf_rne(x1 - __uint_as_float(((unsigned int)h1) << 16));
+          if constexpr (VEC) {
+            if (row < w.M && c0 < w.nB) {
+              *reinterpret_cast<unsigned int*>(w.ohi + off + c0) = (unsigned int)h0 | ((unsigned int)h1 << 16);
+              *reinterpret_cast<unsigned int*>(w.olo + off + c0) = (unsigned int)l0 | ((unsigned int)l1 << 16);
+            }
+          } else {
+            if (row < w.M && c0 < w.nB) { w.ohi[off + c0] = h0; w.olo[off + c0] = l0; }
+            if (row < w.M && c1 < w.nB) { w.ohi[off + c1] = h1; w.olo[off + c1] = l1; }
           }
+        } else if constexpr (VEC) {
+          if (row < w.M && c0 < w.nB) *reinterpret_cast<vec2*>(w.out + off + c0) = vec2{x0, x1};
+        } else {
+          if (row < w.M && c0 < w.nB) w.out[off + c0] = x0;
+          if (row < w.M && c1 < w.nB) w.out[off + c1] = x1;
         }
-    }
+      }
   }
 }
 
@@ -614,70 +625,93 @@ void build_sparse_op(SparseOp& op, int rows, int cols, const std::vector<double>
   op.rows = rows;
   op.cols = cols;
   op.nnz = (int)ci.size();
-  op.rowptr.ensure(rp.size() * sizeof(int));
-  op.colidx.ensure(std::max<size_t>(1, ci.size()) * sizeof(int));
-  op.vals.ensure(std::max<size_t>(1, v.size()) * sizeof(double));
-  TN_HIP(hipMemcpy(op.rowptr.p, rp.data(), rp.size() * sizeof(int), hipMemcpyHostToDevice));
-  if (!ci.empty()) {
-    TN_HIP(hipMemcpy(op.colidx.p, ci.data(), ci.size() * sizeof(int), hipMemcpyHostToDevice));
-    TN_HIP(hipMemcpy(op.vals.p, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
-  }
-  op.dense = rows <= 128 && cols <= 128 && op.nnz >= 8 * rows;
-  if (op.dense) {
-    std::vector<float> f(dense.begin(), dense.begin() + (size_t)rows * cols);
-    op.d64.ensure((size_t)rows * cols * sizeof(double));
-    op.d32.ensure((size_t)rows * cols * sizeof(float));
-    TN_HIP(hipMemcpy(op.d64.p, dense.data(), (size_t)rows * cols * sizeof(double), hipMemcpyHostToDevice));
-    TN_HIP(hipMemcpy(op.d32.p, f.data(), (size_t)rows * cols * sizeof(float), hipMemcpyHostToDevice));
-  }
+  op.mat = rows <= 128 && cols <= 128;
+  op.dense = op.mat && op.nnz >= 8 * rows;
+  // one allocation and one copy: values, FP64 matrix, FP32 matrix, row starts, columns
+  const size_t n = v.size(), nm = op.mat ? (size_t)rows * cols : 0;
+  op.o_d64 = n * sizeof(double);
+  op.o_d32 = op.o_d64 + nm * sizeof(double);
+  op.o_rp = op.o_d32 + nm * sizeof(float);
+  op.o_ci = op.o_rp + rp.size() * sizeof(int);
+  std::vector<unsigned char> h(op.o_ci + n * sizeof(int));
+  std::copy_n(v.data(), n, reinterpret_cast<double*>(h.data()));
+  std::copy_n(dense.data(), nm, reinterpret_cast<double*>(h.data() + op.o_d64));
+  std::copy_n(dense.data(), nm, reinterpret_cast<float*>(h.data() + op.o_d32));
+  std::copy_n(rp.data(), rp.size(), reinterpret_cast<int*>(h.data() + op.o_rp));
+  std::copy_n(ci.data(), n, reinterpret_cast<int*>(h.data() + op.o_ci));
+  op.buf.ensure(h.size());
+  TN_HIP(hipMemcpy(op.buf.p, h.data(), h.size(), hipMemcpyHostToDevice));
 }
+
+namespace {
+template <typename T, bool SPLIT, bool VEC, int NMB>
+void launch_wm(tn_ctx* c, const WmArgs<T>& a) {
+  constexpr int MP = NMB * (sizeof(T) == 8 ? 16 : 32);
+  const size_t shm = ((size_t)a.Kp + MP) * sizeof(long) + (size_t)MP * (a.Kp + 1) * sizeof(T);
+  raise_lds_limit((const void*)wstep_mfma_kernel<T, SPLIT, VEC, NMB>, shm);
+  // wavefronts take strips until all are done: enough workgroups for three per CU
+  const unsigned wg = std::min<unsigned>((a.strips + 3) / 4, 768);
+  hipLaunchKernelGGL((wstep_mfma_kernel<T, SPLIT, VEC, NMB>), dim3(wg), dim3(256), shm, c->stream, a);
+}
+template <typename T, bool SPLIT, bool VEC>
+void launch_wm_rows(tn_ctx* c, const WmArgs<T>& a) {
+  const int nmb = (a.M + (sizeof(T) == 8 ? 15 : 31)) / (sizeof(T) == 8 ? 16 : 32);
+  if constexpr (sizeof(T) == 8) {
+    if (nmb <= 2) launch_wm<T, SPLIT, VEC, 2>(c, a);
+    else if (nmb <= 4) launch_wm<T, SPLIT, VEC, 4>(c, a);
+    else if (nmb <= 5) launch_wm<T, SPLIT, VEC, 5>(c, a);
+    else if (nmb <= 6) launch_wm<T, SPLIT, VEC, 6>(c, a);
+    else launch_wm<T, SPLIT, VEC, 8>(c, a);
+  } else {
+    if (nmb <= 1) launch_wm<T, SPLIT, VEC, 1>(c, a);
+    else if (nmb <= 2) launch_wm<T, SPLIT, VEC, 2>(c, a);
+    else if (nmb <= 3) launch_wm<T, SPLIT, VEC, 3>(c, a);
+    else launch_wm<T, SPLIT, VEC, 4>(c, a);
+  }
+  TN_HIP(hipGetLastError());
+}
+template <typename T, bool SPLIT>
+void wstep_mfma(tn_ctx* c, const WStepDesc& w, const T* opd, bool vec, unsigned short* hi, unsigned short* lo) {
+  constexpr int CW = sizeof(T) == 8 ? 32 : 64, KG = (sizeof(T) == 8 ? 4 : 2) * WM_PF;
+  WmArgs<T> a;
+  a.D = w.D; a.Dp = w.Dp; a.M = w.Gp * w.Dp; a.K = w.G * w.D;
+  a.Kp = (a.K + KG - 1) / KG * KG;
+  a.nA = w.nA; a.nB = w.nB;
+  const long nbt = (w.nB + CW - 1) / CW;
+  TN_REQUIRE(nbt * w.nA < (1L << 31), TN_E_INVALID, "wstep: too many columns");
+  a.nbt = (unsigned)nbt; a.strips = (unsigned)(nbt * w.nA);
+  a.in = (const T*)w.in; a.in_sg = w.in_sg; a.in_sA = w.in_sA; a.in_sS = w.in_sS;
+  a.out = (T*)w.out; a.out_sg = w.out_sg; a.out_sA = w.out_sA; a.out_sS = w.out_sS;
+  a.opd = opd; a.ohi = hi; a.olo = lo;
+  if (vec) launch_wm_rows<T, SPLIT, true>(c, a);
+  else launch_wm_rows<T, SPLIT, false>(c, a);
+}
+}  // namespace
 
 static void wstep_launch(tn_ctx* c, bool fp32, bool split, const WStepDesc& w, unsigned short* hi,
                          unsigned short* lo) {
   TN_REQUIRE(w.op && w.op->rows == w.Gp * w.Dp && w.op->cols == w.G * w.D, TN_E_SHAPE,
              "wstep: operator shape mismatch");
   if (w.nA == 0 || w.nB == 0) return;
-  TN_REQUIRE(w.nA <= 65535L, TN_E_INVALID, "wstep: nA exceeds grid.y");
   const int K = w.G * w.D;
-  const int* rp = w.op->rowptr.as<int>();
-  const int* ci = w.op->colidx.as<int>();
-  const double* vv = w.op->vals.as<double>();
-  if (w.op->dense) {
-    // dense operator: MFMA product per workgroup when Op and the slab fit in LDS
-    const int mb = fp32 ? 32 : 16, ks = fp32 ? 2 : 4;
-    const int M = w.Gp * w.Dp;
-    const int Mp = (M + mb - 1) / mb * mb, Kp = (K + ks - 1) / ks * ks;
-    const size_t es = fp32 ? sizeof(float) : sizeof(double);
-    const size_t mshm = ((size_t)Mp * (Kp + 1) + (size_t)Kp * WM_NB) * es;
-    if (mshm <= 160 * 1024 && Mp <= 128) {
-      const long nbt = (w.nB + WM_NB - 1) / WM_NB;
-      const int vn = fp32 ? 4 : 2;
-      auto whole = [&](long x) { return x % vn == 0; };
-      const int vecin = whole(w.nB) && whole(w.in_sg) && whole(w.in_sA) && whole(w.in_sS) &&
-                        (uintptr_t)w.in % 16 == 0;
-      dim3 grid((unsigned)nbt, (unsigned)w.nA);
-      if (split) {
-        raise_lds_limit((const void*)wstep_mfma_kernel<float, true>, mshm);
-        hipLaunchKernelGGL((wstep_mfma_kernel<float, true>), grid, dim3(256), mshm, c->stream, w.G, w.Gp, w.D,
-                           w.Dp, w.nB, (const float*)w.in, w.in_sg, w.in_sA, w.in_sS, (float*)nullptr, w.out_sg,
-                           w.out_sA, w.out_sS, w.op->d32.as<float>(), Mp, Kp, hi, lo, vecin);
-      } else if (fp32) {
-        raise_lds_limit((const void*)wstep_mfma_kernel<float, false>, mshm);
-        hipLaunchKernelGGL((wstep_mfma_kernel<float, false>), grid, dim3(256), mshm, c->stream, w.G, w.Gp, w.D,
-                           w.Dp, w.nB, (const float*)w.in, w.in_sg, w.in_sA, w.in_sS, (float*)w.out, w.out_sg,
-                           w.out_sA, w.out_sS, w.op->d32.as<float>(), Mp, Kp, (unsigned short*)nullptr,
-                           (unsigned short*)nullptr, vecin);
-      } else {
-        raise_lds_limit((const void*)wstep_mfma_kernel<double, false>, mshm);
-        hipLaunchKernelGGL((wstep_mfma_kernel<double, false>), grid, dim3(256), mshm, c->stream, w.G, w.Gp, w.D,
-                           w.Dp, w.nB, (const double*)w.in, w.in_sg, w.in_sA, w.in_sS, (double*)w.out, w.out_sg,
-                           w.out_sA, w.out_sS, w.op->d64.as<double>(), Mp, Kp, (unsigned short*)nullptr,
-                           (unsigned short*)nullptr, vecin);
-      }
-      TN_HIP(hipGetLastError());
-      return;
-    }
+  const int* rp = w.op->rowptr();
+  const int* ci = w.op->colidx();
+  const double* vv = w.op->vals();
+  // the MFMA product, except for operators past its 128 rows or columns and
+  // for inputs with undefined values where the operator is zero
+  if (w.op->mat && !w.csr) {
+    auto even = [](long x) { return x % 2 == 0; };
+    const size_t es = fp32 ? sizeof(float) : sizeof(double), os = split ? 2 : es;
+    const void* out0 = split ? (const void*)hi : w.out;
+    const bool vec = even(w.nB) && even(w.in_sg) && even(w.in_sA) && even(w.in_sS) && even(w.out_sg) &&
+                     even(w.out_sA) && even(w.out_sS) && (uintptr_t)w.in % (2 * es) == 0 &&
+                     (uintptr_t)out0 % (2 * os) == 0 && (!split || (uintptr_t)lo % 4 == 0);
+    if (split) wstep_mfma<float, true>(c, w, w.op->d32(), vec, hi, lo);
+    else if (fp32) wstep_mfma<float, false>(c, w, w.op->d32(), vec, nullptr, nullptr);
+    else wstep_mfma<double, false>(c, w, w.op->d64(), vec, nullptr, nullptr);
+    return;
   }
+  TN_REQUIRE(w.nA <= 65535L, TN_E_INVALID, "wstep: nA exceeds grid.y");
   if (!split) {
     // 16-byte vectors along B when every offset allows them and the slab fits
     const int vec = fp32 ? 4 : 2;

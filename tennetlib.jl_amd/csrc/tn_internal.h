@@ -315,11 +315,17 @@ void split_bf16(tn_ctx* c, const void* src, bool src_f64, long rows, long cols, 
 // ---------------------------------------------------------------------------
 struct SparseOp {
   int rows = 0, cols = 0, nnz = 0;
-  DevBuf rowptr, colidx, vals;  // int, int, double
-  // row-major dense copies (FP64, FP32) for the MFMA W step, kept when the
-  // operator has at least 8 entries per row and at most 128 rows and columns
-  bool dense = false;
-  DevBuf d64, d32;
+  // CSR rows, and row-major dense copies (FP64, FP32) for the MFMA W step when
+  // the operator has at most 128 rows and columns (mat); dense: at least 8
+  // entries per row as well.  One buffer, parts at the byte offsets o_*
+  bool dense = false, mat = false;
+  DevBuf buf;
+  size_t o_d64 = 0, o_d32 = 0, o_rp = 0, o_ci = 0;
+  const double* vals() const { return buf.as<double>(); }
+  const double* d64() const { return reinterpret_cast<const double*>(buf.as<char>() + o_d64); }
+  const float* d32() const { return reinterpret_cast<const float*>(buf.as<char>() + o_d32); }
+  const int* rowptr() const { return reinterpret_cast<const int*>(buf.as<char>() + o_rp); }
+  const int* colidx() const { return reinterpret_cast<const int*>(buf.as<char>() + o_ci); }
 };
 struct WStepDesc {
   int G = 0, Gp = 0, D = 0, Dp = 0;
@@ -327,6 +333,8 @@ struct WStepDesc {
   const void* in = nullptr; long in_sg = 0, in_sA = 0, in_sS = 0;
   void* out = nullptr; long out_sg = 0, out_sA = 0, out_sS = 0;
   const SparseOp* op = nullptr;
+  // read the input only where the operator has entries (the rest may be undefined)
+  bool csr = false;
 };
 void wstep(tn_ctx* c, bool fp32, const WStepDesc& w);
 // W step from FP32 input writing the result as bf16 hi/lo pairs at the

@@ -937,6 +937,7 @@ void matvec_qn(tn_env* e, const QnMvPlan& qp, const Dom& D, const SparseOp& op, 
   ws.in = T1; ws.in_sg = chil * DD * chir; ws.in_sA = DD * chir; ws.in_sS = chir;
   ws.out = T2; ws.out_sg = chir; ws.out_sA = (long)DD * w2 * chir; ws.out_sS = (long)w2 * chir;
   ws.op = &op;
+  ws.csr = !op.dense;
   wstep(c, f32, ws);
   BsDesc g3;
   g3.A = T2; g3.lda = (long)DD * w2 * chir;

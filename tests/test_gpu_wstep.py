@@ -1,0 +1,67 @@
+"""H psi where the operator step changes kernels: operators of one to 128 rows
+and columns (blocks of 16 rows in FP64, 32 in FP32, K groups of 20 and 10),
+dense and sparse, with column counts at the edges of a strip (32 and 64), odd
+ones and one column, against the oracle's contraction."""
+
+import numpy as np
+import pytest
+
+from oracle import tn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (MPO bond, d, sites, chi left, chi right): rows and columns = bond * d^sites
+SIZES = [(1, 2, 1, 5, 1), (5, 2, 1, 16, 33), (8, 2, 1, 16, 64), (17, 1, 1, 9, 31), (5, 2, 2, 40, 64),
+         (8, 2, 2, 3, 66), (11, 3, 1, 7, 65), (4, 4, 2, 16, 30), (20, 2, 2, 33, 97), (24, 2, 2, 20, 32),
+         (7, 4, 2, 6, 34), (32, 2, 2, 37, 63), (8, 4, 2, 64, 128)]
+
+
+@pytest.fixture(scope="module")
+def T():
+    import tennetlib_amd
+    return tennetlib_amd
+
+
+def chain(w, d, chil, chir, fill, seed):
+    """Four sites with a random MPO of bond w around sites 2 and 3."""
+    rng = np.random.default_rng(seed)
+    wd = [1, w, w, w, 1]
+    cd = [1, min(chil, 8), chil, chir, 1]
+    Ws = []
+    for k in range(4):
+        W = rng.standard_normal((wd[k], d, d, wd[k + 1]))
+        Ws.append(W * (rng.random(W.shape) < fill))
+    A = [rng.standard_normal((cd[k], d, cd[k + 1])) for k in range(4)]
+    return Ws, A, rng
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "w%d_d%d_n%d_%dx%d" % s)
+@pytest.mark.parametrize("fill", [1.0, 0.15])
+def test_operator_step(T, size, fill):
+    w, d, nsite, chil, chir = size
+    Ws, A, rng = chain(w, d, chil, chir, fill, seed=w * 1000 + chir)
+    env, ref = T.StateEnvs(A, Ws), O.Envs(Ws)
+    ref.nsite = nsite
+    T.set_nsite_(env, nsite)
+    p = 2 if nsite == 2 else 3   # one site: both of its bonds are chil and chir wide
+    T.position_(env, p)
+    ref.position(A, p)
+    dims, _ = env.phi_dims()
+    psi = rng.standard_normal(tuple(dims) if nsite == 2 else (dims[0], dims[1], dims[3]))
+    want = ref.product(psi)
+    # rounding grows with the lengths of the sums and with the cancellation in
+    # them: bounded by eps times the product of the absolute values, whose norm
+    # is taken from the same contraction
+    cap = O.Envs([np.abs(W) for W in Ws])
+    cap.nsite = nsite
+    cap.position([np.abs(a) for a in A], p)
+    scale = np.linalg.norm(cap.product(np.abs(psi)))
+    # relative error of one sum of K products: K eps at the worst, sqrt(K) in
+    # practice; three sums of at most 4 * 128 terms follow each other in the
+    # environments and three in the product, and the precision's own input
+    # rounding (2^-24; bf16 pairs 2^-16, kept to 1e-4 elsewhere) is inside
+    for prec, tol in (("fp64", 6 * 512 * 2.0 ** -53), ("fp32", 3 * 512 * 2.0 ** -24), ("bf16x3", 1e-4)):
+        print("w step", size, fill, prec, flush=True)
+        got = T.product(env, psi, precision=prec).reshape(want.shape)
+        err = np.linalg.norm(got - want)
+        assert err <= tol * scale, (prec, err / max(scale, 1e-300))
