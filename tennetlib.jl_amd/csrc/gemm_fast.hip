@@ -161,6 +161,11 @@ struct TileCfg {
   static constexpr int B_VECS = B_ROWS * B_COLS / VN / 256;
   static constexpr int A_ELEMS = A_ROWS * A_LD, B_ELEMS = B_ROWS * B_LD;
   static constexpr int WT = BM / 2, F = WT / Acc<T>::MB;  // wave tile, MFMA blocks per side
+  // K tiles on their way in registers: one where the MFMAs of a tile cover a
+  // load, more where they do not (a 32 x 32 FP64 tile multiplies 32 rows of K
+  // in 0.2 us): 370 x 185 x 925 FP64 20.2 us with one, 17.4 with four.  64 x 64
+  // FP64 and complex tiles gained nothing (40.4 and 40.7 us, 35.3 and 36.6).
+  static constexpr int PF = BM == 128 || (BM == 64 && sizeof(T) >= 8) ? 1 : (A_VECS + B_VECS) <= 4 ? 4 : 2;
   static constexpr size_t LDS = 2 * (size_t)(A_ELEMS + B_ELEMS) * sizeof(T);
   static_assert(A_VECS * VN * 256 == A_ROWS * A_COLS && B_VECS * VN * 256 == B_ROWS * B_COLS, "whole vectors");
 };
@@ -181,11 +186,13 @@ __device__ __forceinline__ void tile_product(Seg& seg, long M, long N, long m0, 
   T* Bs = As + 2 * CF::A_ELEMS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * CF::WT, wn = (wave & 1) * CF::WT;
-  uint4 ra[CF::A_VECS], rb[CF::B_VECS];
+  constexpr int PF = CF::PF;
+  uint4 ra[PF][CF::A_VECS], rb[PF][CF::B_VECS];
   long k0 = 0;
-  double w = 1.0;
+  double w[PF];
   // the next K tile of the current segment: rows m (TA = 0, k contiguous) or rows k (TA = 1, m contiguous)
-  auto gload = [&]() {
+  auto gload = [&](auto slot) {
+    constexpr int Q = decltype(slot)::value;
     const T* A = reinterpret_cast<const T*>(seg.A);
     const T* B = reinterpret_cast<const T*>(seg.B);
     const Rsrc ar = TA ? tile_rsrc(A, k0, seg.K, BK, lda, seg.wA, ES) : tile_rsrc(A, m0, M, BM, lda, seg.wA, ES);
@@ -194,50 +201,51 @@ __device__ __forceinline__ void tile_product(Seg& seg, long M, long N, long m0, 
     for (int i = 0; i < CF::A_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::A_COLS / VN), cc = (idx % (CF::A_COLS / VN)) * VN;
-      ra[i] = ldvec<T, AL>(ar, rr, (TA ? m0 : k0) + cc, lda, seg.wA);
+      ra[Q][i] = ldvec<T, AL>(ar, rr, (TA ? m0 : k0) + cc, lda, seg.wA);
     }
 #pragma unroll
     for (int i = 0; i < CF::B_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::B_COLS / VN), cc = (idx % (CF::B_COLS / VN)) * VN;
-      rb[i] = ldvec<T, AL>(br, rr, (TB ? k0 : n0) + cc, ldb, seg.wB);
+      rb[Q][i] = ldvec<T, AL>(br, rr, (TB ? k0 : n0) + cc, ldb, seg.wB);
     }
-    if constexpr (SCALE) w = seg.w;
+    if constexpr (SCALE) w[Q] = seg.w;
     k0 += BK;
     if (k0 >= seg.K) {
       k0 = 0;
       seg.next();
     }
   };
-  auto sstore = [&](int st) {
+  auto sstore = [&](auto slot, int st) {
+    constexpr int Q = decltype(slot)::value;
     T* as = As + st * CF::A_ELEMS;
     T* bs = Bs + st * CF::B_ELEMS;
     if constexpr (SCALE) {
 #pragma unroll
       for (int i = 0; i < CF::A_VECS; ++i) {
-        double2 v = __builtin_bit_cast(double2, ra[i]);
-        v.x *= w;
-        v.y *= w;
-        ra[i] = __builtin_bit_cast(uint4, v);
+        double2 v = __builtin_bit_cast(double2, ra[Q][i]);
+        v.x *= w[Q];
+        v.y *= w[Q];
+        ra[Q][i] = __builtin_bit_cast(uint4, v);
       }
     }
     if constexpr (ES == 16) {  // conjugated operands: the sign of the imaginary part
 #pragma unroll
-      for (int i = 0; i < CF::A_VECS; ++i) ra[i].w ^= cA ? 0x80000000u : 0u;
+      for (int i = 0; i < CF::A_VECS; ++i) ra[Q][i].w ^= cA ? 0x80000000u : 0u;
 #pragma unroll
-      for (int i = 0; i < CF::B_VECS; ++i) rb[i].w ^= cB ? 0x80000000u : 0u;
+      for (int i = 0; i < CF::B_VECS; ++i) rb[Q][i].w ^= cB ? 0x80000000u : 0u;
     }
 #pragma unroll
     for (int i = 0; i < CF::A_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::A_COLS / VN), cc = (idx % (CF::A_COLS / VN)) * VN;
-      *reinterpret_cast<uint4*>(&as[rr * CF::A_LD + cc]) = ra[i];
+      *reinterpret_cast<uint4*>(&as[rr * CF::A_LD + cc]) = ra[Q][i];
     }
 #pragma unroll
     for (int i = 0; i < CF::B_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::B_COLS / VN), cc = (idx % (CF::B_COLS / VN)) * VN;
-      *reinterpret_cast<uint4*>(&bs[rr * CF::B_LD + cc]) = rb[i];
+      *reinterpret_cast<uint4*>(&bs[rr * CF::B_LD + cc]) = rb[Q][i];
     }
   };
   // element (m, k) of the A stage and (k, n) of the B stage
@@ -339,18 +347,59 @@ __device__ __forceinline__ void tile_product(Seg& seg, long M, long N, long m0, 
     }
   };
   if (seg.done()) return;
-  gload();
-  sstore(0);
-  __syncthreads();
-  for (int st = 0;; st ^= 1) {
-    const bool more = !seg.done();
-    if (more) gload();
-    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
-    compute(st);
-    __builtin_amdgcn_sched_barrier(0);
-    if (!more) break;
-    sstore(st ^ 1);
+  using S0 = std::integral_constant<int, 0>;
+  if constexpr (PF == 1) {
+    gload(S0{});
+    sstore(S0{}, 0);
     __syncthreads();
+    for (int st = 0;; st ^= 1) {
+      const bool more = !seg.done();
+      if (more) gload(S0{});
+      __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
+      compute(st);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!more) break;
+      sstore(S0{}, st ^ 1);
+      __syncthreads();
+    }
+  } else {
+    // PF tiles ahead in registers: slot q holds tiles q, q + PF, ...
+    using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, PF == 4 ? 2 : 0>;
+    using S3 = std::integral_constant<int, PF == 4 ? 3 : 1>;
+    int ahead = 1;  // tiles loaded and not yet multiplied
+    gload(S0{});
+    auto fetch = [&](auto slot) {
+      if (!seg.done()) {
+        gload(slot);
+        ++ahead;
+      }
+    };
+    fetch(S1{});
+    if constexpr (PF == 4) {
+      fetch(S2{});
+      fetch(S3{});
+    }
+    sstore(S0{}, 0);
+    fetch(S0{});
+    __syncthreads();
+    // one tile: multiply it from stage st, then move the next one (slot) to the other stage
+    auto step = [&](int st, auto slot) -> bool {
+      compute(st);
+      if (--ahead == 0) return false;
+      sstore(slot, st ^ 1);
+      fetch(slot);
+      __syncthreads();
+      return true;
+    };
+    while (true) {
+      if (!step(0, S1{})) break;
+      if (!step(1, S2{})) break;
+      if constexpr (PF == 4) {
+        if (!step(0, S3{})) break;
+        if (!step(1, S0{})) break;
+      }
+    }
   }
 }
 
