@@ -1158,24 +1158,25 @@ __global__ __launch_bounds__(256) void adjoint_z_kernel(const double2* __restric
 // ---------------------------------------------------------------------------
 // 2. divide and conquer
 // ---------------------------------------------------------------------------
-// Zero the two off-diagonal sub-blocks of each merge block, so that every
-// column of the block is explicit over all n rows.
 struct MergeDev {
-  int a, n1, n;    // block [a, a + n), split at a + n1
+  int a, n1, n;    // block: entries [a, a + n) of the stacked vectors, split at a + n1
   int k;           // non-deflated roots
   int koff;        // offset into the packed root arrays
   int roff, nrot;  // deflation rotations
+  long q, ldq;     // its first element and row stride in Q
   long uoff;       // offset of this merge's U^T (k x k) in the packed buffer
+  long toff;       // offset of its n x n columns in the gather buffer
   double rho;      // > 0
 };
 
-__global__ __launch_bounds__(256) void dc_zero_off_kernel(double* __restrict__ Q, long ldq,
-                                                          const MergeDev* __restrict__ md) {
+// Zero the two off-diagonal sub-blocks of each merge block, so that every
+// column of the block is explicit over all n rows.
+__global__ __launch_bounds__(256) void dc_zero_off_kernel(double* __restrict__ Q, const MergeDev* __restrict__ md) {
   const MergeDev m = md[blockIdx.y];
   const long tot = (long)m.n * m.n;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < tot; i += (long)gridDim.x * 256) {
     const int r = (int)(i / m.n), c = (int)(i % m.n);
-    if ((r < m.n1) != (c < m.n1)) Q[(long)(m.a + r) * ldq + (m.a + c)] = 0.0;
+    if ((r < m.n1) != (c < m.n1)) Q[m.q + r * m.ldq + c] = 0.0;
   }
 }
 
@@ -1184,13 +1185,12 @@ struct Rot {
   double c, s;
 };
 // deflation rotations, in order, on the rows of each merge block
-__global__ __launch_bounds__(256) void dc_givens_kernel(double* __restrict__ Q, long ldq,
-                                                        const MergeDev* __restrict__ md,
+__global__ __launch_bounds__(256) void dc_givens_kernel(double* __restrict__ Q, const MergeDev* __restrict__ md,
                                                         const Rot* __restrict__ rots) {
   const MergeDev m = md[blockIdx.y];
   const int r = blockIdx.x * 256 + threadIdx.x;
   if (r >= m.n || m.nrot == 0) return;
-  double* row = Q + (long)(m.a + r) * ldq + m.a;
+  double* row = Q + m.q + r * m.ldq;
   for (int t = 0; t < m.nrot; ++t) {
     const Rot R = rots[m.roff + t];
     const double x = row[R.ca], y = row[R.cb];
@@ -1363,32 +1363,32 @@ __global__ __launch_bounds__(256) void dc_evec_kernel(const MergeDev* __restrict
 }
 
 // z of each merge: last row of its left block, first row of its right block
-__global__ __launch_bounds__(256) void dc_zgather_kernel(const double* __restrict__ Q, long ldq,
-                                                         const int* __restrict__ zl, double* __restrict__ z) {
-  const int a = zl[3 * blockIdx.y], n1 = zl[3 * blockIdx.y + 1], n = zl[3 * blockIdx.y + 2];
-  for (int t = threadIdx.x; t < n; t += 256) {
-    const long r = (t < n1) ? (a + n1 - 1) : (a + n1);
-    z[a + t] = Q[r * ldq + (a + t)];
-  }
+__global__ __launch_bounds__(256) void dc_zgather_kernel(const double* __restrict__ Q,
+                                                         const MergeDev* __restrict__ md, double* __restrict__ z) {
+  const MergeDev m = md[blockIdx.x];
+  for (int t = threadIdx.x; t < m.n; t += 256) z[m.a + t] = Q[m.q + (t < m.n1 ? m.n1 - 1 : m.n1) * m.ldq + t];
 }
 
-// new column order of a merge block: tmp[:, t] = Q[:, a + src[t]] (n x n, ld n)
-__global__ __launch_bounds__(256) void dc_gather_cols_kernel(const double* __restrict__ Q, long ldq, int a, int n,
+// new column order of each merge block: tmp[:, t] = Q[:, src[t]] (n x n, ld n)
+__global__ __launch_bounds__(256) void dc_gather_cols_kernel(const double* __restrict__ Q,
+                                                             const MergeDev* __restrict__ md,
                                                              const int* __restrict__ src, double* __restrict__ tmp) {
-  const long tot = (long)n * n;
+  const MergeDev m = md[blockIdx.y];
+  const long tot = (long)m.n * m.n;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < tot; i += (long)gridDim.x * 256) {
-    const int r = (int)(i / n), t = (int)(i % n);
-    tmp[i] = Q[(long)(a + r) * ldq + (a + src[t])];
+    const int r = (int)(i / m.n), t = (int)(i % m.n);
+    tmp[m.toff + i] = Q[m.q + r * m.ldq + src[m.a + t]];
   }
 }
-// Q[a + r][a + t] = tmp[r][t] for t in [t0, n)
-__global__ __launch_bounds__(256) void dc_put_cols_kernel(double* __restrict__ Q, long ldq, int a, int n, int t0,
+// the deflated columns, after the roots: Q[r][t] = tmp[r][t] for t in [k, n)
+__global__ __launch_bounds__(256) void dc_put_cols_kernel(double* __restrict__ Q, const MergeDev* __restrict__ md,
                                                           const double* __restrict__ tmp) {
-  const int w = n - t0;
-  const long tot = (long)n * w;
+  const MergeDev m = md[blockIdx.y];
+  const int w = m.n - m.k;
+  const long tot = (long)m.n * w;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < tot; i += (long)gridDim.x * 256) {
-    const int r = (int)(i / w), t = t0 + (int)(i % w);
-    Q[(long)(a + r) * ldq + (a + t)] = tmp[(long)r * n + t];
+    const int r = (int)(i / w), t = m.k + (int)(i % w);
+    Q[m.q + r * m.ldq + t] = tmp[m.toff + (long)r * m.n + t];
   }
 }
 
@@ -1540,113 +1540,129 @@ struct EigStages {
   }
 };
 
-static size_t level_bytes(long p) {
-  return (size_t)p * (5 * 8 + 6 * 4) + (size_t)p * sizeof(MergeDev) + (size_t)p * sizeof(Rot) + 1024;
-}
+// One tridiagonal of a forest: n entries from a on in the stacked vectors, its
+// eigenvectors at q in Q (row stride ldq).
+struct Tree {
+  int a, n;
+  long q, ldq;
+};
 
-// Divide and conquer on the symmetric tridiagonal (d, e), p >= 2: Q (p x p,
-// ld p) receives the eigenvectors as columns; returns their eigenvalues.
-static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<double>& d, const std::vector<double>& e,
-                                      double* Q, EigStages& stage) {
-  const int P = (int)p;
-  const size_t lvb = level_bytes(p);
-  char* hs = (char*)c->host_stage(lvb + 8 * (size_t)p * sizeof(double) + 256);
-  double* hx = (double*)(hs + ((lvb + 255) & ~(size_t)255));
-  // ---- 2. divide and conquer on (d, e)
-  struct Blk { int a, n; };
+// Divide and conquer on the symmetric tridiagonals of a forest (d, e device
+// vectors of T entries in all): the trees' eigenvectors go to Q as columns;
+// returns the eigenvalues, stacked as d is.  The leaves of all trees are one
+// launch, the merges of one level one sequence of launches: a tree more costs
+// a product per merge and hardly more latency.
+static std::vector<double> dc_forest(tn_ctx* c, int T, const std::vector<Tree>& trees, const double* d_d,
+                                     const double* d_e, double* Q, EigStages& stage) {
+  struct Blk { int a, n, t; };
   std::vector<Blk> blocks;
-  {  // ceil(P / LEAF) leaves of nearly equal size (the slowest leaf sets the time)
-    const int nl = (P + LEAF - 1) / LEAF;
-    for (int b = 0, a = 0; b < nl; ++b) {
-      const int nb = P / nl + (b < P % nl ? 1 : 0);
-      blocks.push_back(Blk{a, nb});
-      a += nb;
+  std::vector<SmallEig> leaves;
+  long nn = 0;  // entries of all trees' matrices
+  int nmax = 0;
+  for (size_t t = 0; t < trees.size(); ++t) {
+    // ceil(n / LEAF) leaves of nearly equal size (the slowest leaf sets the time)
+    const Tree& tr = trees[t];
+    const int nl = (tr.n + LEAF - 1) / LEAF;
+    nn += (long)tr.n * tr.n;
+    for (int b = 0, o = 0; b < nl; ++b) {
+      const int nb = tr.n / nl + (b < tr.n % nl ? 1 : 0);
+      blocks.push_back(Blk{tr.a + o, nb, (int)t});
+      leaves.push_back(SmallEig{nb, tr.a + o, 0, 0, tr.q + o * tr.ldq + o, tr.ldq, 0, 0,
+                                (b > 0 ? SE_TEAR_L : 0) | (b + 1 < nl ? SE_TEAR_R : 0)});
+      nmax = std::max(nmax, nb);
+      o += nb;
     }
   }
-  std::vector<double> dt = d;  // torn diagonal
-  for (size_t b = 1; b < blocks.size(); ++b) {
-    const int k = blocks[b].a;
-    dt[k - 1] -= e[k - 1];
-    dt[k] -= e[k - 1];
+  const bool merges = leaves.size() > trees.size();
+  // level tables, packed: dK, zK, zh, tau (T doubles each), org, root_merge,
+  // src (T ints each), rotations, merge descriptors, z rows; a merge joins at
+  // least two leaves of more than LEAF / 2 rows
+  const long nmerge = T / LEAF + 1;
+  const size_t tab = (size_t)T * (5 * sizeof(double) + 3 * sizeof(int) + sizeof(Rot)) + nmerge * sizeof(MergeDev) + 64;
+  const size_t lvb = std::max(tab, leaves.size() * sizeof(SmallEig));
+  char* hs = (char*)c->host_stage(((lvb + 255) & ~(size_t)255) + (size_t)2 * T * sizeof(double));
+  double* hx = (double*)(hs + ((lvb + 255) & ~(size_t)255));  // eigenvalues, e
+  char* lv = (char*)c->workspace(WS_DC_LEVEL, lvb);
+  double* d_lam = (double*)c->workspace(WS_DC_SMALL, (size_t)T * sizeof(double));
+  const bool one = leaves.size() == 1;
+  if (!one) {
+    std::copy(leaves.begin(), leaves.end(), (SmallEig*)hs);
+    TN_HIP(hipMemcpyAsync(lv, hs, leaves.size() * sizeof(SmallEig), hipMemcpyHostToDevice, c->stream));
   }
-  const long ldq = p;
-  double* small = (double*)c->workspace(WS_DC_SMALL, (size_t)3 * p * sizeof(double) + blocks.size() * sizeof(SmallEig));
-  double* d_dt = small;
-  double* d_e = d_dt + p;
-  double* d_lam = d_e + p;
-  SmallEig* d_leaf = (SmallEig*)(d_lam + p);
-  {
-    // mirror of the `small` layout: dt, e, lam (p doubles each), leaves
-    std::copy(dt.begin(), dt.end(), hx);
-    std::copy(e.begin(), e.end(), hx + p);
-    SmallEig* hl = (SmallEig*)(hx + 3 * p);
-    int nmax = 0;
-    for (size_t b = 0; b < blocks.size(); ++b) {
-      const int a = blocks[b].a;
-      hl[b] = SmallEig{blocks[b].n, a, 0, 0, (long)a * ldq + a, ldq, 0, 0};
-      nmax = std::max(nmax, blocks[b].n);
-    }
-    TN_HIP(hipMemcpyAsync(small, hx, (size_t)3 * p * sizeof(double) + blocks.size() * sizeof(SmallEig),
-                          hipMemcpyHostToDevice, c->stream));
-    dc_small(c, nmax, (int)blocks.size(), SmallEig{}, d_leaf, d_dt, d_e, Q, d_lam);
-  }
-  TN_HIP(hipMemcpyAsync(hx + 2 * p, d_lam, p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  dc_small(c, nmax, (int)leaves.size(), leaves[0], one ? nullptr : (const SmallEig*)lv, d_d, d_e, Q, d_lam);
+  TN_HIP(hipMemcpyAsync(hx, d_lam, (size_t)T * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (merges) TN_HIP(hipMemcpyAsync(hx + T, d_e, (size_t)T * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   stage("leaves");
   TN_HIP(hipStreamSynchronize(c->stream));
-  std::vector<double> D(hx + 2 * p, hx + 3 * p);  // eigenvalues per block, block-local column order
+  std::vector<double> D(hx, hx + T);  // eigenvalues per block, block-local column order
+  if (!merges) return D;
+  const std::vector<double> e(hx + T, hx + 2 * T);
 
-  double* tmp = (double*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double));
-  double* Utb = (double*)c->workspace(WS_DC_UT, (size_t)p * p * sizeof(double));
-  // packed per-level device arrays: dK, zK, zh, tau (p doubles each), org,
-  // root_merge, src (p ints each), merge descriptors and rotations
-  char* lv = (char*)c->workspace(WS_DC_LEVEL, lvb);
+  double* tmp = (double*)c->workspace(WS_DC_TMP, (size_t)nn * sizeof(double));
+  double* Utb = (double*)c->workspace(WS_DC_UT, (size_t)nn * sizeof(double));
   auto H = [&](const void* dev) { return hs + ((const char*)dev - lv); };  // host mirror of a level table
   double* d_dK = (double*)lv;
-  double* d_zK = d_dK + p;
-  double* d_zh = d_zK + p;
-  double* d_tau = d_zh + p;
-  int* d_org = (int*)(d_tau + p);
-  int* d_rm = d_org + p;
-  int* d_src = d_rm + p;
-  MergeDev* d_md = (MergeDev*)(((uintptr_t)(d_src + p) + 15) & ~(uintptr_t)15);
-  Rot* d_rot = (Rot*)(((uintptr_t)(d_md + p) + 15) & ~(uintptr_t)15);
-  double* d_zrow = (double*)(((uintptr_t)(d_rot + p) + 15) & ~(uintptr_t)15);
-  int* d_zl = (int*)(d_zrow + p);  // 3 ints per merge
+  double* d_zK = d_dK + T;
+  double* d_zh = d_zK + T;
+  double* d_tau = d_zh + T;
+  int* d_org = (int*)(d_tau + T);
+  int* d_rm = d_org + T;
+  int* d_src = d_rm + T;
+  auto up16 = [](void* x) { return (char*)(((uintptr_t)x + 15) & ~(uintptr_t)15); };
+  Rot* d_rot = (Rot*)up16(d_src + T);
+  MergeDev* d_md = (MergeDev*)up16(d_rot + T);
+  double* d_zrow = (double*)up16(d_md + nmerge);
 
-  while (blocks.size() > 1) {
+  while (true) {
+    // pairs of neighbours within a tree
     std::vector<Blk> nb;
+    std::vector<MergeDev> mds;
     std::vector<HostMerge> hms;
-    // z of every merge: last row of the left block, first row of the right block
-    int* hzl = (int*)H(d_zl);  // (a, n1, n) per merge
-    int nzm = 0;
-    for (size_t i = 0; i + 1 < blocks.size(); i += 2, ++nzm) {
-      hzl[3 * nzm] = blocks[i].a;
-      hzl[3 * nzm + 1] = blocks[i].n;
-      hzl[3 * nzm + 2] = blocks[i].n + blocks[i + 1].n;
+    long toff = 0;
+    for (size_t i = 0; i < blocks.size(); ++i) {
+      const Blk b1 = blocks[i];
+      if (i + 1 == blocks.size() || blocks[i + 1].t != b1.t) {
+        nb.push_back(b1);
+        continue;
+      }
+      const Tree& tr = trees[b1.t];
+      MergeDev md{};
+      md.a = b1.a;
+      md.n1 = b1.n;
+      md.n = b1.n + blocks[i + 1].n;
+      md.q = tr.q + (b1.a - tr.a) * (tr.ldq + 1);
+      md.ldq = tr.ldq;
+      md.toff = toff;
+      toff += (long)md.n * md.n;
+      mds.push_back(md);
+      nb.push_back(Blk{b1.a, md.n, b1.t});
+      ++i;
     }
-    TN_HIP(hipMemcpyAsync(d_zl, hzl, 3 * nzm * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(dc_zgather_kernel, dim3(1, nzm), dim3(256), 0, c->stream, Q, ldq, d_zl, d_zrow);
-    TN_HIP(hipMemcpyAsync(H(d_zrow), d_zrow, p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const int nm = (int)mds.size();
+    if (nm == 0) break;
+    TN_REQUIRE(nm <= nmerge, TN_E_INVALID, "divide and conquer: merge table");
+    std::copy(mds.begin(), mds.end(), (MergeDev*)H(d_md));
+    TN_HIP(hipMemcpyAsync(d_md, H(d_md), nm * sizeof(MergeDev), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(dc_zgather_kernel, dim3(nm), dim3(256), 0, c->stream, Q, d_md, d_zrow);
+    TN_HIP(hipMemcpyAsync(H(d_zrow), d_zrow, (size_t)T * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     TN_HIP(hipStreamSynchronize(c->stream));
     const double* zrow = (const double*)H(d_zrow);
-    std::vector<MergeDev> mds;
     std::vector<Rot> allrot;
     std::vector<double> hdK, hzK;
-    std::vector<int> hrm, hsrc;
+    std::vector<int> hrm;
     long uoff = 0;
-    for (size_t i = 0; i + 1 < blocks.size(); i += 2) {
-      const Blk b1 = blocks[i], b2 = blocks[i + 1];
+    int maxn = 0, maxdefl = 0;
+    for (int mi = 0; mi < nm; ++mi) {
+      MergeDev& md = mds[mi];
       HostMerge hm;
-      hm.a = b1.a;
-      hm.n1 = b1.n;
-      hm.n = b1.n + b2.n;
+      hm.a = md.a;
+      hm.n1 = md.n1;
+      hm.n = md.n;
       std::vector<double> Dm(D.begin() + hm.a, D.begin() + hm.a + hm.n);
       std::vector<double> zm(zrow + hm.a, zrow + hm.a + hm.n);
       const double is2 = 1.0 / std::sqrt(2.0);
       for (double& v : zm) v *= is2;
-      deflate(hm, Dm, zm, e[b2.a - 1]);
-      MergeDev md;
-      md.a = hm.a; md.n1 = hm.n1; md.n = hm.n;
+      deflate(hm, Dm, zm, e[hm.a + hm.n1 - 1]);
       md.k = (int)hm.K.size();
       md.koff = (int)hdK.size();
       md.roff = (int)allrot.size();
@@ -1654,17 +1670,15 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
       md.uoff = uoff;
       md.rho = hm.rho;
       uoff += (long)md.k * md.k;
-      for (int t = 0; t < md.k; ++t) hrm.push_back((int)mds.size());
+      maxn = std::max(maxn, md.n);
+      maxdefl = std::max(maxdefl, md.n - md.k);
+      hrm.insert(hrm.end(), md.k, mi);
       hdK.insert(hdK.end(), hm.dK.begin(), hm.dK.end());
       hzK.insert(hzK.end(), hm.zK.begin(), hm.zK.end());
       allrot.insert(allrot.end(), hm.rots.begin(), hm.rots.end());
-      mds.push_back(md);
       hms.push_back(std::move(hm));
-      nb.push_back(Blk{b1.a, b1.n + b2.n});
     }
-    if (blocks.size() % 2) nb.push_back(blocks.back());
     const int nroots = (int)hdK.size();
-    const int nm = (int)mds.size();
     // all tables of the level in one upload through the pinned mirror
     std::copy(mds.begin(), mds.end(), (MergeDev*)H(d_md));
     std::copy(allrot.begin(), allrot.end(), (Rot*)H(d_rot));
@@ -1673,21 +1687,17 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
     std::copy(hrm.begin(), hrm.end(), (int*)H(d_rm));
     {
       int* hsrc = (int*)H(d_src);  // new column order of every merge block: [roots..., deflated...]
-      for (int mi = 0; mi < nm; ++mi) {
-        const HostMerge& hm = hms[mi];
+      for (const HostMerge& hm : hms) {
         std::copy(hm.K.begin(), hm.K.end(), hsrc + hm.a);
         std::copy(hm.defl.begin(), hm.defl.end(), hsrc + hm.a + hm.K.size());
       }
     }
     TN_HIP(hipMemcpyAsync(lv, hs, (size_t)((char*)d_zrow - lv), hipMemcpyHostToDevice, c->stream));
-    int maxn = 0;
-    for (auto& m : mds) maxn = std::max(maxn, m.n);
     // explicit zeros off the two diagonal sub-blocks, then the deflation rotations
-    hipLaunchKernelGGL(dc_zero_off_kernel, dim3(grid_for((long)maxn * maxn, 1024), nm), dim3(256), 0, c->stream, Q,
-                       ldq, d_md);
+    const dim3 mgrid(grid_for((long)maxn * maxn, 1024), nm);
+    hipLaunchKernelGGL(dc_zero_off_kernel, mgrid, dim3(256), 0, c->stream, Q, d_md);
     if (!allrot.empty())
-      hipLaunchKernelGGL(dc_givens_kernel, dim3((maxn + 255) / 256, nm), dim3(256), 0, c->stream, Q, ldq, d_md,
-                         d_rot);
+      hipLaunchKernelGGL(dc_givens_kernel, dim3((maxn + 255) / 256, nm), dim3(256), 0, c->stream, Q, d_md, d_rot);
     if (nroots > 0) {
       hipLaunchKernelGGL(dc_secular_kernel, dim3((unsigned)((nroots + 3) / 4)), dim3(256), 0, c->stream, d_md, d_rm,
                          d_dK, d_zK, nroots, d_org, d_tau);
@@ -1696,31 +1706,26 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
       hipLaunchKernelGGL(dc_evec_kernel, dim3((unsigned)nroots), dim3(256), 0, c->stream, d_md, d_rm, d_dK, d_zh,
                          d_org, d_tau, Utb);
     }
+    // Q_blk[:, :k] = Q_K U of every merge, deflated columns after the roots
+    hipLaunchKernelGGL(dc_gather_cols_kernel, mgrid, dim3(256), 0, c->stream, Q, d_md, d_src, tmp);
     TN_HIP(hipGetLastError());
-    // per merge: Q_blk[:, :k] = Q_K U, deflated columns after the roots
-    for (int mi = 0; mi < nm; ++mi) {
-      const HostMerge& hm = hms[mi];
-      const MergeDev& md = mds[mi];
-      int* d_s = d_src + hm.a;
-      hipLaunchKernelGGL(dc_gather_cols_kernel, dim3(grid_for((long)hm.n * hm.n)), dim3(256), 0, c->stream, Q, ldq,
-                         hm.a, hm.n, d_s, tmp);
-      if (md.k > 0) {
-        GemmDesc g;
-        g.M = hm.n; g.N = md.k; g.K = md.k;
-        g.A = tmp; g.lda = hm.n;
-        g.B = Utb + md.uoff; g.ldb = md.k; g.tB = 1;
-        g.C = Q + (long)hm.a * ldq + hm.a; g.ldc = ldq;
-        gemm(c, Prec::F64, g);
-      }
-      if (md.k < hm.n)
-        hipLaunchKernelGGL(dc_put_cols_kernel, dim3(grid_for((long)hm.n * (hm.n - md.k))), dim3(256), 0, c->stream,
-                           Q, ldq, hm.a, hm.n, md.k, tmp);
-      TN_HIP(hipGetLastError());
+    for (const MergeDev& md : mds) {
+      if (md.k == 0) continue;
+      GemmDesc g;
+      g.M = md.n; g.N = md.k; g.K = md.k;
+      g.A = tmp + md.toff; g.lda = md.n;
+      g.B = Utb + md.uoff; g.ldb = md.k; g.tB = 1;
+      g.C = Q + md.q; g.ldc = md.ldq;
+      gemm(c, Prec::F64, g);
     }
+    if (maxdefl > 0)
+      hipLaunchKernelGGL(dc_put_cols_kernel, dim3(grid_for((long)maxn * maxdefl, 1024), nm), dim3(256), 0, c->stream,
+                         Q, d_md, tmp);
+    TN_HIP(hipGetLastError());
     // eigenvalues of the merged blocks (host), in the new column order
-    // tau (p doubles) and org (p ints) are adjacent: one download
+    // tau (T doubles) and org (T ints) are adjacent: one download
     if (nroots > 0)
-      TN_HIP(hipMemcpyAsync(H(d_tau), d_tau, (size_t)p * sizeof(double) + (size_t)nroots * sizeof(int),
+      TN_HIP(hipMemcpyAsync(H(d_tau), d_tau, (size_t)T * sizeof(double) + (size_t)nroots * sizeof(int),
                             hipMemcpyDeviceToHost, c->stream));
     TN_HIP(hipStreamSynchronize(c->stream));
     const int* horg = (const int*)H(d_org);
@@ -1735,7 +1740,6 @@ static std::vector<double> dc_tridiag(tn_ctx* c, long p, const std::vector<doubl
     blocks.swap(nb);
     stage("merge level");
   }
-
   return D;
 }
 
@@ -1754,36 +1758,136 @@ constexpr int TRD_BLOCKED_MIN = 3072;
 // launches per column instead of one)
 constexpr int TRD_TILE_MIN = 1024;
 
+// columns [0, j0) of a p x p matrix, one fused launch each: reflector 0, then
+// the update with one reflector and the next one together, then the last
+// update.  scratch: 9 p + 2048 doubles.
+static void trd_columns(tn_ctx* c, double* G, int P, long ldg, int j0, double* dv, double* ev, double* tauv,
+                        double* scratch) {
+  if (j0 < 1) return;
+  const long p = P;
+  double* y = scratch;
+  double* part = y + p;
+  double* vA = scratch + 3 * p + 512;
+  double* vB = vA + p;
+  double* yB = vB + p;
+  double* pB = yB + p;  // >= 512 + p / 4 entries
+  raise_lds_limit((const void*)trd_reflect_kernel, (size_t)p * sizeof(double));
+  raise_lds_limit((const void*)trd_step_kernel, 3 * (size_t)(P - 1) * sizeof(double));
+  const int m = P - 1;
+  const int np0 = (m + HR - 1) / HR;
+  hipLaunchKernelGGL(trd_reflect_kernel, dim3(np0), dim3(256), (size_t)m * sizeof(double), c->stream, G, ldg, P, 0, y,
+                     part, dv, ev, tauv, vA);
+  double *cv = vA, *cy = y, *cp = part, *nv = vB, *ny = yB, *npart = pB;
+  int cnp = np0;
+  for (int j = 0; j + 2 <= j0; ++j) {
+    const int mj = P - j - 1, mn = mj - 1;
+    const int nwg = std::min(256, (mn + 3) / 4);
+    hipLaunchKernelGGL(trd_step_kernel, dim3(nwg), dim3(256), 3 * (size_t)mj * sizeof(double), c->stream, G, ldg, P, j,
+                       cv, cy, cp, cnp, nv, ny, npart, dv, ev, tauv);
+    std::swap(cv, nv);
+    std::swap(cy, ny);
+    std::swap(cp, npart);
+    cnp = nwg;
+  }
+  const unsigned tiles = (unsigned)((P - j0 + 63) / 64);
+  hipLaunchKernelGGL(trd_update_kernel, dim3(tiles, tiles), dim3(256), 0, c->stream, G, ldg, P, j0 - 1, cy, cp, cnp,
+                     tauv);
+  TN_HIP(hipGetLastError());
+}
+
+void sym_eig_blocks(tn_ctx* c, std::vector<SmallEig> blk, double* G, double* V, std::vector<double>& w) {
+  const int nb = (int)blk.size();
+  if (nb == 0) return;
+  int T = 0;
+  long nn = 0, nrows = 0;
+  for (SmallEig& b : blk) {
+    TN_REQUIRE(b.n >= 1 && b.n <= BACK_SMALL_MAX, TN_E_INVALID, "sym_eig_blocks: size out of range");
+    b.de = T;
+    b.q = nn;
+    b.ldq = b.n;
+    T += b.n;
+    nn += (long)b.n * b.n;
+    if (b.n > TRD_SMALL_MAX) nrows += (long)b.n * b.n;
+  }
+  // largest first: they set the time of a launch, and its size classes are runs
+  std::stable_sort(blk.begin(), blk.end(), [](const SmallEig& x, const SmallEig& y) { return x.n > y.n; });
+  const int nmax = blk[0].n;
+  EigStages stage(c, nmax);
+  double* dv = (double*)c->workspace(WS_DC_VEC, ((size_t)3 * T + 9 * nmax + 2048) * sizeof(double));
+  double* ev = dv + T;
+  double* tauv = ev + T;
+  double* Q = (double*)c->workspace(WS_DC_Q, (size_t)nn * sizeof(double));
+  // ---- 1. tridiagonalisation: the last TRD_SMALL_MAX columns of every block in one launch
+  std::vector<SmallEig> lists;
+  for (const SmallEig& b : blk) {
+    const int jt = std::max(0, b.n - TRD_SMALL_MAX);
+    trd_columns(c, G + b.a, b.n, b.lda, jt, dv + b.de, ev + b.de, tauv + b.de, tauv + T);
+    lists.push_back(SmallEig{b.n - jt, b.de + jt, b.a + jt * (b.lda + 1), b.lda, 0, 0, 0, 0, jt == 0 ? SE_ROWS : 0});
+  }
+  // the list of the back-transformation: blocks with columns reduced one by one read rows collected at the end
+  std::vector<Tree> trees;
+  long ro = 0;
+  for (const SmallEig& b : blk) {
+    SmallEig t = b;
+    if (b.n > TRD_SMALL_MAX) {
+      t.a = ro;
+      t.lda = b.n;
+      ro += (long)b.n * b.n;
+    }
+    lists.push_back(t);
+    trees.push_back(Tree{b.de, b.n, b.q, b.ldq});
+  }
+  const SmallEig* dl = nullptr;
+  if (nb > 1) {
+    dl = (const SmallEig*)c->workspace(WS_DC_LIST, lists.size() * sizeof(SmallEig));
+    TN_HIP(hipMemcpyAsync((void*)dl, lists.data(), lists.size() * sizeof(SmallEig), hipMemcpyHostToDevice, c->stream));
+  }
+  trd_small(c, false, lists[0].n, nb, lists[0], dl, G, dv, ev, tauv);
+  stage("tridiagonal");
+  // ---- 2. divide and conquer
+  w = dc_forest(c, T, trees, dv, ev, Q, stage);
+  // ---- 3. back-transformation, a launch per class of registers
+  double* rows = nullptr;
+  if (nrows > 0) rows = (double*)c->workspace(WS_DC_TMP, (size_t)nrows * sizeof(double));
+  static constexpr int cls[] = {128, TRD_SMALL_MAX, 256, 512, BACK_SMALL_MAX};
+  for (int i = 0; i < nb;) {
+    const int top = *std::lower_bound(std::begin(cls), std::end(cls), blk[i].n);
+    int j = i;
+    for (; j < nb && *std::lower_bound(std::begin(cls), std::end(cls), blk[j].n) == top; ++j) {
+      if (top <= TRD_SMALL_MAX) continue;
+      const unsigned nt = (unsigned)((blk[j].n + 31) / 32);
+      hipLaunchKernelGGL(reflector_rows_kernel<double>, dim3(nt, nt), dim3(256), 0, c->stream, G + blk[j].a,
+                         blk[j].lda, blk[j].n, rows + lists[nb + j].a);
+    }
+    TN_HIP(hipGetLastError());
+    back_small(c, false, blk[i].n, j - i, lists[nb + i], dl ? dl + nb + i : nullptr, top <= TRD_SMALL_MAX ? G : rows,
+               tauv, Q, V);
+    i = j;
+  }
+  stage("back-transform");
+  TN_HIP(hipStreamSynchronize(c->stream));  // the host lists go out of scope
+}
+
 void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, std::vector<double>& w) {
   TN_REQUIRE(p >= 1 && p <= 16384, TN_E_INVALID, "sym_eig_dc: size out of range");
   const int P = (int)p;
+  if (P <= BACK_SMALL_MAX) {
+    sym_eig_blocks(c, {SmallEig{P, 0, 0, ldg, 0, 0, 0, ldv, 0}}, G, Vt, w);
+    return;
+  }
   EigStages stage(c, p);
   // ---- 1. tridiagonalisation
   double* vecs = (double*)c->workspace(WS_DC_VEC, (size_t)(12 * p + 2048) * sizeof(double));
   double* dv = vecs;
   double* ev = dv + p;
   double* tauv = ev + p;
-  if (P <= DC_SMALL_MAX) {  // one workgroup holds the block: three launches, one read-back
-    double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
-    double* lam = tauv + p;
-    const SmallEig one{P, 0, 0, ldg, 0, p, 0, ldv};
-    trd_small(c, false, P, 1, one, nullptr, G, dv, ev, tauv, true);
-    dc_small(c, P, 1, one, nullptr, dv, ev, Q, lam);
-    back_small(c, false, P, 1, one, nullptr, G, tauv, Q, Vt);
-    double* hx = (double*)c->host_stage((size_t)p * sizeof(double));
-    TN_HIP(hipMemcpyAsync(hx, lam, (size_t)p * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    TN_HIP(hipStreamSynchronize(c->stream));
-    w.assign(hx, hx + p);
-    stage("one workgroup");
-    return;
-  }
   double* y = tauv + p;
-  double* part = y + p;  // <= ceil(p / HR) entries
   // panels of NBT columns (one pass over the trailing block per column) from
   // p = TRD_BLOCKED_MIN on; below it one fused launch per column
-  const int jt = std::max(0, P - TRD_SMALL_MAX);  // columns jt.. are reduced by one workgroup
-  bool done = false;
-  if (jt >= 1 && P >= TRD_BLOCKED_MIN) {
+  const int jt = P - TRD_SMALL_MAX;  // columns jt.. are reduced by one workgroup
+  if (P < TRD_BLOCKED_MIN) {
+    trd_columns(c, G, P, ldg, jt, dv, ev, tauv, tauv + p);
+  } else {
     const int nAmax = (P + RCHUNK - 1) / RCHUNK;
     const int nBmax = (P + 7) / 8;
     const long ntmax = (p + SYT - 1) / SYT + 1;
@@ -1863,76 +1967,12 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
         gemm(c, Prec::F64, g);
       }
     }
-    done = true;
   }
-  if (!done) {
-    const size_t lds_bytes = (size_t)p * sizeof(double);
-    raise_lds_limit((const void*)trd_reflect_kernel, (size_t)lds_bytes);
-    const int j0 = jt;
-    if (j0 >= 1 && P <= 6000) {
-      // fused path: reflector 0, then one launch per column, then the update of step j0 - 1
-      double* vA = vecs + 6 * p + 512;
-      double* vB = vA + p;
-      double* yB = vB + p;
-      double* pB = yB + p;  // >= 512 + p / 4 entries
-      const size_t step_lds_max = 3 * (size_t)(P - 1) * sizeof(double);
-      raise_lds_limit((const void*)trd_step_kernel, step_lds_max);
-      const int m = P - 1;
-      const int np0 = (m + HR - 1) / HR;
-      hipLaunchKernelGGL(trd_reflect_kernel, dim3(np0), dim3(256), (size_t)m * sizeof(double), c->stream, G, ldg, P,
-                         0, y, part, dv, ev, tauv, vA);
-      double *cv = vA, *cy = y, *cp = part, *nv = vB, *ny = yB, *npart = pB;
-      int cnp = np0;
-      for (int j = 0; j + 2 <= j0; ++j) {
-        const int mj = P - j - 1, mn = mj - 1;
-        const int nwg = std::min(256, (mn + 3) / 4);
-        hipLaunchKernelGGL(trd_step_kernel, dim3(nwg), dim3(256), 3 * (size_t)mj * sizeof(double), c->stream, G, ldg,
-                           P, j, cv, cy, cp, cnp, nv, ny, npart, dv, ev, tauv);
-        std::swap(cv, nv);
-        std::swap(cy, ny);
-        std::swap(cp, npart);
-        cnp = nwg;
-      }
-      const int mlast = P - j0;
-      const unsigned tiles = (unsigned)((mlast + 63) / 64);
-      hipLaunchKernelGGL(trd_update_kernel, dim3(tiles, tiles), dim3(256), 0, c->stream, G, ldg, P, j0 - 1, cy, cp,
-                         cnp, tauv);
-    } else {
-      for (int j = 0; j < j0; ++j) {
-        const int m = P - j - 1;
-        const int nparts = (m + HR - 1) / HR;
-        hipLaunchKernelGGL(trd_reflect_kernel, dim3(nparts), dim3(256), (size_t)m * sizeof(double), c->stream, G,
-                           ldg, P, j, y, part, dv, ev, tauv, (double*)nullptr);
-        const unsigned tiles = (unsigned)((m + 63) / 64);
-        hipLaunchKernelGGL(trd_update_kernel, dim3(tiles, tiles), dim3(256), 0, c->stream, G, ldg, P, j, y, part,
-                           nparts, tauv);
-      }
-    }
-  }
-  trd_small(c, false, P - jt, 1, SmallEig{P - jt, jt, (long)jt * ldg + jt, ldg, 0, 0, 0, 0}, nullptr, G, dv, ev, tauv,
-            false);
-  TN_HIP(hipGetLastError());
-  // d, e to the host through the pinned staging buffer
-  double* hx = (double*)c->host_stage(2 * (size_t)p * sizeof(double));
-  TN_HIP(hipMemcpyAsync(hx, dv, (2 * p - 1) * sizeof(double), hipMemcpyDeviceToHost, c->stream));  // d, e
-  TN_HIP(hipStreamSynchronize(c->stream));
-  std::vector<double> d(hx, hx + p), e(hx + p, hx + 2 * p - 1);
+  trd_small(c, false, P - jt, 1, SmallEig{P - jt, jt, (long)jt * ldg + jt, ldg, 0, 0, 0, 0, 0}, nullptr, G, dv, ev, tauv);
   stage("tridiagonal");
   double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
   const long ldq = p;
-  std::vector<double> D = dc_tridiag(c, p, d, e, Q, stage);
-  if (P <= BACK_SMALL_MAX) {
-    // ---- 3. back-transformation with the reflectors as rows
-    double* rows = (double*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double));
-    const unsigned nt = (unsigned)((P + 31) / 32);
-    hipLaunchKernelGGL(reflector_rows_kernel<double>, dim3(nt, nt), dim3(256), 0, c->stream, G, ldg, P, rows);
-    TN_HIP(hipGetLastError());
-    back_small(c, false, P, 1, SmallEig{P, 0, 0, p, 0, ldq, 0, ldv}, nullptr, rows, tauv, Q, Vt);
-    stage("back-transform");
-    w.assign(D.begin(), D.end());
-    TN_HIP(hipStreamSynchronize(c->stream));
-    return;
-  }
+  std::vector<double> D = dc_forest(c, P, {Tree{0, P, 0, p}}, dv, ev, Q, stage);
   double* tmp = (double*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double));
 
   // ---- 3. back-transformation Q <- H Q, H = H_0 ... H_{p-3}
@@ -2002,8 +2042,8 @@ void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv
   if (P <= std::min(DC_SMALL_MAX, TRD_SMALL_MAX_Z)) {
     double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
     double* lam = (double*)yz;
-    const SmallEig one{P, 0, 0, ldg, 0, p, 0, ldv};
-    trd_small(c, true, P, 1, one, nullptr, G, dv, ev, tauz, true);
+    const SmallEig one{P, 0, 0, ldg, 0, p, 0, ldv, SE_ROWS};
+    trd_small(c, true, P, 1, one, nullptr, G, dv, ev, tauz);
     dc_small(c, P, 1, one, nullptr, dv, ev, Q, lam);
     back_small(c, true, P, 1, one, nullptr, G, tauz, Q, Vt);
     double* hx = (double*)c->host_stage((size_t)p * sizeof(double));
@@ -2027,23 +2067,18 @@ void sym_eig_dc_z(tn_ctx* c, double* Gd, long p, long ldg, double* Vtd, long ldv
     hipLaunchKernelGGL(trdz_update_kernel, dim3(tiles, tiles), dim3(256), 0, c->stream, G, ldg, P, j, yz, partz,
                        nparts, tauz);
   }
-  trd_small(c, true, P - j0, 1, SmallEig{P - j0, j0, (long)j0 * ldg + j0, ldg, 0, 0, 0, 0}, nullptr, G, dv, ev, tauz,
-            false);
-  TN_HIP(hipGetLastError());
-  double* hx = (double*)c->host_stage(2 * (size_t)p * sizeof(double));
-  TN_HIP(hipMemcpyAsync(hx, dv, (2 * p - 1) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  TN_HIP(hipStreamSynchronize(c->stream));
-  std::vector<double> d(hx, hx + p), e(hx + p, hx + 2 * p - 1);
+  trd_small(c, true, P - j0, 1, SmallEig{P - j0, j0, (long)j0 * ldg + j0, ldg, 0, 0, 0, 0, 0}, nullptr, G, dv, ev,
+            tauz);
   stage("tridiagonal");
   // ---- 2. real divide and conquer
   double* Q = (double*)c->workspace(WS_DC_Q, (size_t)p * p * sizeof(double));
-  std::vector<double> D = dc_tridiag(c, p, d, e, Q, stage);
+  std::vector<double> D = dc_forest(c, P, {Tree{0, P, 0, p}}, dv, ev, Q, stage);
   if (P <= BACK_SMALL_MAX_Z) {
     double2* rows = (double2*)c->workspace(WS_DC_TMP, (size_t)p * p * sizeof(double2));
     const unsigned nt = (unsigned)((P + 31) / 32);
     hipLaunchKernelGGL(reflector_rows_kernel<double2>, dim3(nt, nt), dim3(256), 0, c->stream, G, ldg, P, rows);
     TN_HIP(hipGetLastError());
-    back_small(c, true, P, 1, SmallEig{P, 0, 0, p, 0, p, 0, ldv}, nullptr, rows, tauz, Q, Vt);
+    back_small(c, true, P, 1, SmallEig{P, 0, 0, p, 0, p, 0, ldv, 0}, nullptr, rows, tauz, Q, Vt);
     stage("back-transform");
     w.assign(D.begin(), D.end());
     TN_HIP(hipStreamSynchronize(c->stream));

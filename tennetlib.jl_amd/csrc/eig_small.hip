@@ -98,7 +98,7 @@ __device__ __forceinline__ double sum4(double x) {
 // and the dot product for itself.  Nothing is stored to global memory inside
 // the loop (a barrier would wait for the stores): column j of the block is
 // dead after step j and keeps the reflector, as does row j.
-// rows_only: row j of A receives the reflector right of the diagonal and
+// SE_ROWS: row j of A receives the reflector right of the diagonal and
 // zeros elsewhere.
 // Measured: 32 rows 13 us, 64 rows 64 us, 192 rows 416 us (136 rows in LDS
 // with 256 threads: 504 us; the same registers over 1024 threads: 910 us, the
@@ -107,8 +107,7 @@ __device__ __forceinline__ double sum4(double x) {
 template <bool CX, int GR, int GC, int NR, int NC>
 __global__ __launch_bounds__(GR* GC) void trd_reg_kernel(SmallEig one, const SmallEig* __restrict__ list,
                                                          void* __restrict__ Abase, double* __restrict__ dbase,
-                                                         double* __restrict__ ebase, void* __restrict__ taubase,
-                                                         int rows_only) {
+                                                         double* __restrict__ ebase, void* __restrict__ taubase) {
   typedef El<CX> E;
   typedef typename E::T T;
   constexpr int NT = GR * GC, NM = GR * NR, NP = NM + 2, NW = (NM + 63) / 64, SEG = GC;
@@ -256,7 +255,7 @@ __global__ __launch_bounds__(GR* GC) void trd_reg_kernel(SmallEig one, const Sma
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const int r = tr + GR * i, c = tc + GC * j;
-      if (r < n && c < n) A[(long)r * S.lda + c] = (rows_only && c <= r) ? E::zero() : a[i][j];
+      if (r < n && c < n) A[(long)r * S.lda + c] = ((S.flags & SE_ROWS) && c <= r) ? E::zero() : a[i][j];
     }
   T* tauv = reinterpret_cast<T*>(taubase) + S.de;
   for (int t = tid; t < n; t += NT) {
@@ -500,7 +499,9 @@ __global__ __launch_bounds__(4 * NM) void dc_small_kernel(SmallEig one, const Sm
   for (int i = tid; i < n * LD; i += NT) Q[i] = 0.0;
   // scaled by a power of two to entries of at most one: nothing below leaves the normal range
   double big = 0.0;
-  for (int t = lane; t < n; t += 64) big = fmax(big, fmax(fabs(d[t]), t < n - 1 ? fabs(e[t]) : 0.0));
+  const double tl = (S.flags & SE_TEAR_L) ? e[-1] : 0.0, tr = (S.flags & SE_TEAR_R) ? e[n - 1] : 0.0;
+  auto diag = [&](int t) { return d[t] - (t == 0 ? tl : 0.0) - (t == n - 1 ? tr : 0.0); };
+  for (int t = lane; t < n; t += 64) big = fmax(big, fmax(fabs(diag(t)), t < n - 1 ? fabs(e[t]) : 0.0));
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
   int ex = 0;
@@ -510,14 +511,14 @@ __global__ __launch_bounds__(4 * NM) void dc_small_kernel(SmallEig one, const Sm
   if (tid < n) {
     const int t = tid, lf = leaf_of(t), a = bnd(lf), sz = bnd(lf + 1) - a;
     if (t == a) {
-      double p = ldexp(d[t], -ex) - (t > 0 ? fabs(ee[t - 1]) : 0.0);
+      double p = ldexp(diag(t), -ex) - (t > 0 ? fabs(ee[t - 1]) : 0.0);
       if (sz == 1) {
         if (t < n - 1) p -= fabs(ee[t]);
         D[t] = p;
         Q[t * LD + t] = 1.0;
       } else {
         const double g = ee[t];
-        const double q = ldexp(d[t + 1], -ex) - (t + 1 < n - 1 ? fabs(ee[t + 1]) : 0.0);
+        const double q = ldexp(diag(t + 1), -ex) - (t + 1 < n - 1 ? fabs(ee[t + 1]) : 0.0);
         double c = 1.0, s = 0.0, tt = 0.0;
         if (g != 0.0) {
           const double zeta = (q - p) / (2.0 * g);
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(4 * NM) void dc_small_kernel(SmallEig one, const Sm
   }
   if (L == 0 && tid == 0) {  // n = 1
     Qg[0] = 1.0;
-    lam[0] = d[0];
+    lam[0] = diag(0);
   }
   __syncthreads();
   // four lanes per column (root)
@@ -833,13 +834,13 @@ __global__ __launch_bounds__(64) void back_small_kernel(SmallEig one, const Smal
 
 template <bool CX, int GR, int GC, int NR, int NC>
 void launch_trd(tn_ctx* c, int nb, const SmallEig& one, const SmallEig* list, void* A, double* d, double* e,
-                void* tau, bool rows_only) {
+                void* tau) {
   constexpr int NM = GR * NR;
   constexpr size_t es = CX ? 16 : 8;
   const size_t shm = ((size_t)GR * (NM + 2) + 4 * NM) * es + 2 * (size_t)NM * sizeof(double);
   raise_lds_limit((const void*)trd_reg_kernel<CX, GR, GC, NR, NC>, shm);
   hipLaunchKernelGGL((trd_reg_kernel<CX, GR, GC, NR, NC>), dim3((unsigned)nb), dim3(GR * GC), shm, c->stream, one,
-                     list, A, d, e, tau, rows_only ? 1 : 0);
+                     list, A, d, e, tau);
 }
 
 template <int NM>
@@ -853,17 +854,17 @@ void launch_dc(tn_ctx* c, int nb, const SmallEig& one, const SmallEig* list, con
 }  // namespace
 
 void trd_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, void* A, double* d,
-               double* e, void* tau, bool rows_only) {
+               double* e, void* tau) {
   TN_REQUIRE(nmax >= 1 && nmax <= (cplx ? TRD_SMALL_MAX_Z : TRD_SMALL_MAX), TN_E_INVALID, "trd_small: size");
   if (!cplx) {
-    if (nmax <= 32) launch_trd<false, 8, 8, 4, 4>(c, nb, one, list, A, d, e, tau, rows_only);
-    else if (nmax <= 64) launch_trd<false, 16, 16, 4, 4>(c, nb, one, list, A, d, e, tau, rows_only);
-    else if (nmax <= 128) launch_trd<false, 16, 16, 8, 8>(c, nb, one, list, A, d, e, tau, rows_only);
-    else launch_trd<false, 16, 32, 12, 6>(c, nb, one, list, A, d, e, tau, rows_only);
+    if (nmax <= 32) launch_trd<false, 8, 8, 4, 4>(c, nb, one, list, A, d, e, tau);
+    else if (nmax <= 64) launch_trd<false, 16, 16, 4, 4>(c, nb, one, list, A, d, e, tau);
+    else if (nmax <= 128) launch_trd<false, 16, 16, 8, 8>(c, nb, one, list, A, d, e, tau);
+    else launch_trd<false, 16, 32, 12, 6>(c, nb, one, list, A, d, e, tau);
   } else {
-    if (nmax <= 32) launch_trd<true, 8, 8, 4, 4>(c, nb, one, list, A, d, e, tau, rows_only);
-    else if (nmax <= 64) launch_trd<true, 16, 16, 4, 4>(c, nb, one, list, A, d, e, tau, rows_only);
-    else launch_trd<true, 16, 32, 8, 4>(c, nb, one, list, A, d, e, tau, rows_only);
+    if (nmax <= 32) launch_trd<true, 8, 8, 4, 4>(c, nb, one, list, A, d, e, tau);
+    else if (nmax <= 64) launch_trd<true, 16, 16, 4, 4>(c, nb, one, list, A, d, e, tau);
+    else launch_trd<true, 16, 32, 8, 4>(c, nb, one, list, A, d, e, tau);
   }
   TN_HIP(hipGetLastError());
 }

@@ -209,7 +209,7 @@ enum WsSlot {
   WS_DC_VEC, WS_DC_Q, WS_DC_SMALL, WS_DC_TMP, WS_DC_UT, WS_DC_LEVEL, WS_DC_W, WS_PROJ_X, WS_PROJ_Y, WS_PROJ_C,
   WS_QR_X, WS_QR_V, WS_QR_Q, WS_QR_R, WS_QR_S, WS_QR_W, WS_TTN_A, WS_TTN_S, WS_TTN_G, WS_TTN_P, WS_TTN_F,
   WS_GEMM_SPLIT, WS_BOND, WS_PHI2, WS_TTNP_0, WS_TTNP_1, WS_TTNP_2, WS_TTNP_3, WS_DC_PANEL,
-  WS_QN_M, WS_QN_V, WS_QN_W, WS_QN_IDX, WS_QN_T, WS_QN_RHO, WS_QN_PLAN, WS_SLOTS
+  WS_DC_LIST, WS_QN_M, WS_QN_V, WS_QN_IDX, WS_QN_T, WS_QN_RHO, WS_QN_PLAN, WS_SLOTS
 };
 
 // scoped phase timer (HIP events on the context stream)
@@ -460,24 +460,33 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
 // Blocks that one workgroup holds (eig_small.hip).  Offsets in elements from
 // the base pointers of a call: d, e, tau and eigenvalues at de, the matrix at
 // a (row stride lda), the tridiagonal's eigenvectors (columns, real) at q,
-// the block's eigenvectors (rows, conjugated when complex) at v.
+// the block's eigenvectors (rows, conjugated when complex) at v.  flags:
+// trd_small leaves reflectors as rows (SE_ROWS); dc_small tears the coupling
+// to the rows before or after the block off its ends (SE_TEAR_L, SE_TEAR_R).
 struct SmallEig {
   int n, de;
   long a, lda, q, ldq, v, ldv;
+  int flags;
 };
+constexpr int SE_ROWS = 1, SE_TEAR_L = 2, SE_TEAR_R = 4;
 constexpr int TRD_SMALL_MAX = 192, TRD_SMALL_MAX_Z = 128;    // rows in one workgroup's registers
 constexpr int DC_SMALL_MAX = 128;                            // eigenvectors in one workgroup's LDS
 constexpr int BACK_SMALL_MAX = 768, BACK_SMALL_MAX_Z = 384;  // rows in the registers of one wavefront
 // Each takes nb blocks of at most nmax rows: `one` when list is null (nb = 1),
 // else the device array list.  trd_small overwrites A: reflector j (v_0 = 1)
-// in column j below the diagonal and in row j right of it; rows_only: in row
-// j, with zeros in its other columns.  back_small reads such rows.
+// in column j below the diagonal and in row j right of it; SE_ROWS: in row j,
+// with zeros in its other columns.  back_small reads such rows.
 void trd_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, void* A, double* d,
-               double* e, void* tau, bool rows_only);
+               double* e, void* tau);
 void dc_small(tn_ctx* c, int nmax, int nb, const SmallEig& one, const SmallEig* list, const double* d, const double* e,
               double* Q, double* lam);
 void back_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, const void* A,
                 const void* tau, const double* Q, void* V);
+// Symmetric blocks of at most BACK_SMALL_MAX rows together: block i (n x n at
+// a, row stride lda in G, overwritten) leaves its eigenvectors as rows at v
+// (row stride ldv) in V; w receives the eigenvalues, block after block.  de, q,
+// ldq and flags are the function's own.
+void sym_eig_blocks(tn_ctx* c, std::vector<SmallEig> blk, double* G, double* V, std::vector<double>& w);
 // Hermitian p x p complex128 (interleaved, 1 <= p <= 16384): complex Householder
 // reduction to a real tridiagonal, the same divide and conquer, complex
 // back-transformation; Vt rows receive the conjugated eigenvectors
@@ -486,13 +495,6 @@ void sym_eig_dc_z(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, 
 void gather_rows_T_z(tn_ctx* c, const double* src, long ld_src, const int* perm, const double* scale,
                      long kcount, long L, double* out, bool conj);
 
-// QN blocks of the factorisation (qn.hip).  qn_block_eig: nblk density-matrix
-// blocks, each at most pmax <= QN_JACOBI_MAX rows, stacked in R (ld
-// QN_RHO_LD); blk_dev[4b..4b+3] = {row offset in R, size p, offset of the p
-// eigenvalues in w, offset of the p eigenvectors (rows of length p) in V}.
-constexpr int QN_JACOBI_MAX = 96;
-constexpr int QN_RHO_LD = 96;
-void qn_block_eig(tn_ctx* c, const double* R, const int* blk_dev, int nblk, int pmax, double* w, double* V);
 // qn_scatter: column j of out (rows x k, ld ldo; its transpose when trans)
 // receives eigenvector col[4j+2] (stored at V + col[4j] as rows of length
 // col[4j+3]) on the rows rows[col[4j+1] ..]; out must be zero elsewhere

@@ -1894,9 +1894,9 @@ void replacebond(tn_env* e, int b, const double* phi, bool ortho_left, long maxd
 // semantics, upstream ITensors/NDTensors; called at update_site.jl:64-76):
 // the density matrix of the kept side is block diagonal in the QN of its
 // combined (link, site) index.  Rows of M (ortho left; columns, through the
-// transpose, for ortho right) are gathered sector by sector; blocks up to 32
-// rows are formed and diagonalised in one launch (one wavefront each), larger
-// ones one by one (gram_eig: divide and conquer).  All weights go through
+// transpose, for ortho right) are gathered sector by sector; blocks of at most
+// BACK_SMALL_MAX rows are formed by one block-sparse product and diagonalised
+// together, larger ones one by one.  All weights go through
 // truncate!!; each block keeps its weights above docut (whole multiplets split
 // across blocks are dropped together, exact zeros go).  The new link lists
 // the kept sectors in ascending QN order, weights descending within each.
@@ -1936,13 +1936,11 @@ void replacebond_qn(tn_env* e, int b, const double* phi, bool ortho_left, long m
     psz.push_back((int)kv.second.size());
     perm.insert(perm.end(), kv.second.begin(), kv.second.end());
   }
-  // eigenvalue / eigenvector slots of every block
-  std::vector<long> woff(ns), voff(ns);
-  long wtot = 0, vtot = 0;
+  // eigenvector slots of every block
+  std::vector<long> voff(ns);
+  long vtot = 0;
   for (int i = 0; i < ns; ++i) {
-    woff[i] = wtot;
     voff[i] = vtot;
-    wtot += psz[i];
     vtot += (long)psz[i] * psz[i];
   }
   TN_REQUIRE(vtot < (1L << 31), TN_E_UNSUPPORTED, "QN-conserving factorisation: blocks too large");
@@ -1960,41 +1958,33 @@ void replacebond_qn(tn_env* e, int b, const double* phi, bool ortho_left, long m
     Gsrc = Mt;
   }
   gather_rows(c, Gsrc, L, dperm, dones, p, L, Gp);
-  double* Wd = (double*)c->workspace(WS_QN_W, (size_t)wtot * sizeof(double));
   double* Vd = (double*)c->workspace(WS_QN_V, (size_t)std::max<long>(vtot, 1) * sizeof(double));
-  // Blocks of a size class (up to 32, 64, 96 rows) go to one batched Jacobi
-  // launch when the block-size histogram says it is cheaper than the dense
-  // eigensolver block by block: measured on MI355X, a launch of class c
-  // takes about qn_batch_ms[c] (set by its largest block, all blocks run
-  // side by side) and one block of p rows through the dense eigensolver
-  // about 0.35 + 0.005 p ms (launch-latency bound below 136 rows).  The
-  // batched blocks' rho_q = G_q G_q^T come from one block-sparse GEMM
-  // launch into a stack (ld QN_RHO_LD); the rest use the dense eigensolver.
-  static constexpr double qn_batch_ms[3] = {0.25, 1.2, 4.0};
-  double serial_ms[3] = {0.0, 0.0, 0.0};
-  for (int i = 0; i < ns; ++i)
-    if (psz[i] <= QN_JACOBI_MAX) serial_ms[(psz[i] + 31) / 32 - 1] += (psz[i] < 3 ? 0.05 : 0.35 + 0.005 * psz[i]);
-  bool batch_cls[3];
-  for (int cl = 0; cl < 3; ++cl) batch_cls[cl] = serial_ms[cl] > qn_batch_ms[cl];
+  // rho_q = G_q G_q^T of every block that the batched eigensolver takes, by one
+  // block-sparse product into a stack.  A step of the eigensolver lasts as long
+  // as its largest block takes: H psi and this factorisation with sectors of
+  // 292, 4 x 188, 4 x 121, 4 x 46 and 15 more of at most 29 rows took 9.2 ms
+  // with the blocks above 96 rows one by one and batched Jacobi rotations below
+  // (17.1 ms when each block also took more launches), together 2.7 ms.
+  std::vector<std::vector<double>> w(ns);
   std::vector<long> soff(ns, -1);
-  long srows = 0;
+  std::vector<SmallEig> blk;
+  long srows = 0, ldr = 0;
   for (int i = 0; i < ns; ++i)
-    if (psz[i] <= QN_JACOBI_MAX && batch_cls[(psz[i] + 31) / 32 - 1]) {
+    if (psz[i] <= BACK_SMALL_MAX) {
       soff[i] = srows;
       srows += psz[i];
+      ldr = std::max<long>(ldr, (psz[i] + 1) / 2 * 2);
     }
   std::vector<BsTask> gt;
   std::vector<BsSeg> gs;
   std::vector<int4> gtl;
-  std::vector<int> meta;
   std::vector<char> host;  // staging of the block plan, alive until the stream is synchronised
-  int cls_n[3] = {0, 0, 0};
   if (srows > 0) {
-    double* Rst = (double*)c->workspace(WS_QN_RHO, (size_t)srows * QN_RHO_LD * sizeof(double));
+    double* Rst = (double*)c->workspace(WS_QN_RHO, (size_t)srows * ldr * sizeof(double));
     for (int i = 0; i < ns; ++i) {
       if (soff[i] < 0) continue;
       BsTask t;
-      t.c_off = soff[i] * QN_RHO_LD;
+      t.c_off = soff[i] * ldr;
       t.M = t.N = psz[i];
       t.seg0 = (int)gs.size();
       t.nseg = 1;
@@ -2003,37 +1993,31 @@ void replacebond_qn(tn_env* e, int b, const double* phi, bool ortho_left, long m
       gt.push_back(t);
     }
     pad_tiles(gtl);
-    // size classes 32, 64, 96: metadata of class 0, then 1, then 2
-    for (int cl = 0; cl < 3; ++cl)
-      for (int i = 0; i < ns; ++i) {
-        if (soff[i] < 0 || (psz[i] + 31) / 32 - 1 != cl) continue;
-        meta.insert(meta.end(), {(int)soff[i], psz[i], (int)woff[i], (int)voff[i]});
-        ++cls_n[cl];
-      }
     auto al = [](size_t x) { return (x + 15) / 16 * 16; };
     const size_t b_t = al(gt.size() * sizeof(BsTask)), b_s = al(gs.size() * sizeof(BsSeg));
-    const size_t b_l = al(gtl.size() * sizeof(int4)), b_m = al(meta.size() * sizeof(int));
-    host.assign(b_t + b_s + b_l + b_m, 0);
+    const size_t b_l = gtl.size() * sizeof(int4);
+    host.assign(b_t + b_s + b_l, 0);
     std::memcpy(host.data(), gt.data(), gt.size() * sizeof(BsTask));
     std::memcpy(host.data() + b_t, gs.data(), gs.size() * sizeof(BsSeg));
     std::memcpy(host.data() + b_t + b_s, gtl.data(), gtl.size() * sizeof(int4));
-    std::memcpy(host.data() + b_t + b_s + b_l, meta.data(), meta.size() * sizeof(int));
     char* dplan = (char*)c->workspace(WS_QN_PLAN, host.size());
     TN_HIP(hipMemcpyAsync(dplan, host.data(), host.size(), hipMemcpyHostToDevice, c->stream));
     BsDesc g;
     g.A = Gp; g.lda = L;
     g.B = Gp; g.ldb = L; g.tB = 1;
-    g.C = Rst; g.ldc = QN_RHO_LD;
+    g.C = Rst; g.ldc = ldr;
     g.tasks = (const BsTask*)dplan;
     g.segs = (const BsSeg*)(dplan + b_t);
     g.tiles = (const int4*)(dplan + b_t + b_s);
     g.ntiles = (long)gtl.size();
     gemm_blocksparse(c, Prec::F64, g);
-    const int* dm = (const int*)(dplan + b_t + b_s + b_l);
-    for (int cl = 0, o = 0; cl < 3; o += cls_n[cl], ++cl)
-      qn_block_eig(c, Rst, dm + 4 * o, cls_n[cl], 32 * (cl + 1), Wd, Vd);
+    for (int i = 0; i < ns; ++i)
+      if (soff[i] >= 0) blk.push_back(SmallEig{psz[i], 0, soff[i] * ldr, ldr, 0, 0, voff[i], psz[i], 0});
+    std::vector<double> hw;
+    sym_eig_blocks(c, blk, Rst, Vd, hw);
+    for (int i = 0; i < ns; ++i)
+      if (soff[i] >= 0) w[i].assign(hw.begin() + soff[i], hw.begin() + soff[i] + psz[i]);
   }
-  std::vector<std::vector<double>> w(ns);
   // large blocks: the dense eigensolver, one block at a time
   for (int i = 0; i < ns; ++i) {
     if (soff[i] >= 0) continue;
@@ -2042,13 +2026,6 @@ void replacebond_qn(tn_env* e, int b, const double* phi, bool ortho_left, long m
     w[i] = ge.w;
     TN_HIP(hipMemcpy2DAsync(Vd + voff[i], (size_t)psz[i] * sizeof(double), ge.Vt, (size_t)ge.ppad * sizeof(double),
                             (size_t)psz[i] * sizeof(double), (size_t)psz[i], hipMemcpyDeviceToDevice, c->stream));
-  }
-  if (srows > 0) {
-    std::vector<double> hw(wtot);
-    TN_HIP(hipMemcpyAsync(hw.data(), Wd, wtot * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    TN_HIP(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < ns; ++i)
-      if (soff[i] >= 0) w[i].assign(hw.begin() + woff[i], hw.begin() + woff[i] + psz[i]);
   }
   // weights of every block in descending order, then NDTensors' block rule
   std::vector<std::vector<int>> ord(ns);

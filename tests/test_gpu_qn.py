@@ -87,10 +87,9 @@ def test_qn_replacebond_matches_oracle(T, ortho):
 
 @pytest.mark.parametrize("ortho", ["left", "right"])
 def test_qn_replacebond_block_size_classes(T, ortho):
-    """U(1) blocks of 10 to 120 rows.  ortho left: 2, 6 and 6 blocks in the
-    size classes up to 32, 64 and 96 rows, enough for each class to take the
-    batched Jacobi launch; ortho right: blocks of 60 and 120 rows through the
-    dense eigensolver.  Kept weights to 1e-13 of the oracle's (numpy eigh per
+    """U(1) blocks of 10 to 120 rows, diagonalised together.  ortho left: 2, 6
+    and 6 blocks of up to 32, 64 and 96 rows; ortho right: blocks of 60 and 120
+    rows.  Kept weights to 1e-13 of the oracle's (numpy eigh per
     block), the new site orthonormal to 1e-13, the product of the two new
     sites to 1e-12."""
     sizes_l = dict(zip(range(-12, 13, 2), [10, 40, 40, 40, 20, 40, 40, 40, 20, 40, 40, 40, 10]))
