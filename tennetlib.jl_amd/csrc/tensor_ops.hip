@@ -338,15 +338,6 @@ __global__ void scaled_copy_kernel(double* __restrict__ y, const double* __restr
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     y[i] = a * x[i];
 }
-// y = x / sqrt(max(0, *r2)) with r2 read from device memory (the squared
-// norm a Krylov step left there), so the next basis vector needs no host trip
-__global__ void scale_rnorm_kernel(double* __restrict__ y, const double* __restrict__ x,
-                                   const double* __restrict__ r2, long n) {
-  const double a = 1.0 / sqrt(fmax(0.0, *r2));
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    y[i] = a * x[i];
-}
-
 // ---------------------------------------------------------------------------
 // Krylov: multi-dot (first stage + fixed-order second stage)
 // part[v * nblk + blk] = partial sum of <basis_v, x> over the block's slice.
@@ -418,103 +409,372 @@ __global__ __launch_bounds__(256) void multidot_stage2(const double* __restrict_
   }
 }
 
-// x -= sum_v coef[v] * basis_v (real or complex coefficients)
-template <bool CPLX>
-__global__ __launch_bounds__(256) void multi_axpy_kernel(const double* __restrict__ basis, long ld, int count,
-                                                         const double* __restrict__ coef, double* __restrict__ x,
-                                                         long n, int sub) {
-  const long stride = (long)gridDim.x * blockDim.x;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += stride) {
-    if (!CPLX) {
-      double acc = 0.0;
-      for (int v = 0; v < count; ++v) acc = fma(coef[v], basis[v * ld + i], acc);
-      x[i] = sub ? x[i] - acc : acc;
-    } else {
-      double ar = 0.0, ai = 0.0;
-      for (int v = 0; v < count; ++v) {
-        const double cr = coef[2 * v], ci = coef[2 * v + 1];
-        const double br = basis[v * ld + 2 * i], bi = basis[v * ld + 2 * i + 1];
-        ar = fma(cr, br, fma(-ci, bi, ar));
-        ai = fma(cr, bi, fma(ci, br, ai));
-      }
-      if (sub) { x[2 * i] -= ar; x[2 * i + 1] -= ai; }
-      else { x[2 * i] = ar; x[2 * i + 1] = ai; }
+// ---------------------------------------------------------------------------
+// Krylov steps: w <- w - V (V^H w) twice over K basis vectors, |w|^2, and the
+// next basis vector w / |w|.  Short vectors: one workgroup with w in
+// registers.  Others: a launch per pass over V -- dots; update and the second
+// pass's dots, from one read of V; update and norm; scaling -- where every
+// workgroup sums the previous launch's partial sums for itself, in a fixed
+// order.  Bound by launches and load latency up to about 10^6 elements (n = 1.4
+// 10^5, 10 vectors: V is 11 MB, 3 us), so all loads of a tile are issued before
+// the first is used.  A solve of 7 steps at n = 137k took 750 us with nine
+// launches a step (dots and their sums, update, twice; norm and its sum;
+// scaling) and the start's norm read by the host, with four 580 us; two-site
+// sweeps of 20 spins, mostly short vectors, 58 -> 49 ms.
+// ---------------------------------------------------------------------------
+constexpr int KS_THREADS = 1024;  // one-workgroup step
+constexpr int KP_TILE = 512;      // elements per tile of the others, two a thread
+constexpr int KP_BLOCKS = 1024;
+constexpr long KS_MAX = 4L * KS_THREADS;
+
+// n <= EP * blockDim elements.  hout (mapped host memory) receives the passes'
+// coefficients at 0 and 128 (pairs when CX) and |w|^2 at 256.  K = 0: norm and
+// scaling only, w stays as it is.
+template <bool CX, int EP>
+__global__ __launch_bounds__(KS_THREADS) void krylov_small_kernel(const double* __restrict__ basis, long ld, int K,
+                                                                  double* __restrict__ w, int n,
+                                                                  double* __restrict__ vnext,
+                                                                  double* __restrict__ hout) {
+  constexpr int C = CX ? 2 : 1;
+  constexpr int KS_CH = EP == 1 ? 8 : 4;  // basis vectors whose loads are in flight at once
+  __shared__ double part[KS_THREADS / 64][128];
+  __shared__ double cf[128];  // zero past the last vector, as far as whole chunks reach
+  __shared__ double red[KS_THREADS / 64];
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+  const int nacc = C * K;
+  double x[EP][C];
+  int idx[EP];
+#pragma unroll
+  for (int e = 0; e < EP; ++e) {
+    const int j = tid + nt * e;
+    idx[e] = C * min(j, n - 1);
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+      const double t = w[idx[e] + q];
+      x[e][q] = j < n ? t : 0.0;
     }
   }
-}
-
-// A whole Krylov orthogonalisation step for a short vector in one
-// workgroup: two passes of w <- w - V (V^H w) over the K basis vectors, then
-// |w|^2.  The pass coefficients go to coef[0..) and coef[128..) (complex
-// pairs when cplx) and |w|^2 to coef[256], each also to hout (mapped host
-// memory) at the same offsets.  Dots: one wave per basis vector (DPP sums).
-constexpr int KS_THREADS = 1024;
-template <bool CPLX>
-__global__ __launch_bounds__(KS_THREADS) void krylov_ortho_small_kernel(const double* __restrict__ basis, long ld,
-                                                                        int K, double* __restrict__ w, long n,
-                                                                        double* __restrict__ coef,
-                                                                        double* __restrict__ hout) {
-  __shared__ double cf[128];
-  __shared__ double red[KS_THREADS / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int NW = KS_THREADS / 64;
-  for (int pass = 0; pass < 2; ++pass) {
-    for (int i = wave; i < K; i += NW) {
-      const double* v = basis + (long)i * ld;
-      double re = 0.0, im = 0.0;
-      if (!CPLX) {
-        for (long j = lane; j < n; j += 64) re = fma(v[j], w[j], re);
-      } else {
-        for (long j = lane; j < n; j += 64) {
-          const double vr = v[2 * j], vi = v[2 * j + 1], wr = w[2 * j], wi = w[2 * j + 1];
-          re = fma(vr, wr, fma(vi, wi, re));
-          im = fma(vr, wi, fma(-vi, wr, im));
+  for (int pass = 0; pass < 2 && K > 0; ++pass) {
+    for (int v0 = 0; v0 < K; v0 += KS_CH) {
+      double b[KS_CH][EP][C], acc[KS_CH][C];
+#pragma unroll
+      for (int u = 0; u < KS_CH; ++u)
+#pragma unroll
+        for (int e = 0; e < EP; ++e)
+#pragma unroll
+          for (int q = 0; q < C; ++q) b[u][e][q] = basis[min(v0 + u, K - 1) * ld + idx[e] + q];
+#pragma unroll
+      for (int u = 0; u < KS_CH; ++u) {
+#pragma unroll
+        for (int q = 0; q < C; ++q) acc[u][q] = 0.0;
+#pragma unroll
+        for (int e = 0; e < EP; ++e) {
+          acc[u][0] = fma(b[u][e][0], x[e][0], acc[u][0]);
+          if constexpr (CX) {
+            acc[u][0] = fma(b[u][e][1], x[e][1], acc[u][0]);
+            acc[u][1] = fma(b[u][e][0], x[e][1], fma(-b[u][e][1], x[e][0], acc[u][1]));
+          }
         }
+#pragma unroll
+        for (int q = 0; q < C; ++q) acc[u][q] = wave_sum64(acc[u][q]);
       }
-      re = wave_sum64(re);
-      if (CPLX) im = wave_sum64(im);
       if (lane == 0) {
-        if (CPLX) { cf[2 * i] = re; cf[2 * i + 1] = im; }
-        else cf[i] = re;
+#pragma unroll
+        for (int u = 0; u < KS_CH; ++u)
+#pragma unroll
+          for (int q = 0; q < C; ++q) part[wave][C * (v0 + u) + q] = acc[u][q];
       }
     }
     __syncthreads();
-    for (long j = tid; j < n; j += KS_THREADS) {
-      if (!CPLX) {
-        double acc = 0.0;
-        for (int v = 0; v < K; ++v) acc = fma(cf[v], basis[v * ld + j], acc);
-        w[j] -= acc;
-      } else {
-        double ar = 0.0, ai = 0.0;
-        for (int v = 0; v < K; ++v) {
-          const double cr = cf[2 * v], ci = cf[2 * v + 1];
-          const double br = basis[v * ld + 2 * j], bi = basis[v * ld + 2 * j + 1];
-          ar = fma(cr, br, fma(-ci, bi, ar));
-          ai = fma(cr, bi, fma(ci, br, ai));
-        }
-        w[2 * j] -= ar;
-        w[2 * j + 1] -= ai;
+    for (int t = tid; t < 128; t += nt) {
+      double s = 0.0;
+      if (t < nacc) {
+        for (int k = 0; k < nw; ++k) s += part[k][t];
+        hout[128 * pass + t] = s;
       }
+      cf[t] = s;
     }
-    const int nc = CPLX ? 2 * K : K;
-    for (int i = tid; i < nc; i += KS_THREADS) {
-      coef[128 * pass + i] = cf[i];
-      hout[128 * pass + i] = cf[i];
+    __syncthreads();
+    double sub[EP][C];
+#pragma unroll
+    for (int e = 0; e < EP; ++e)
+#pragma unroll
+      for (int q = 0; q < C; ++q) sub[e][q] = 0.0;
+    for (int v0 = 0; v0 < K; v0 += KS_CH) {
+      double b[KS_CH][EP][C];
+#pragma unroll
+      for (int u = 0; u < KS_CH; ++u)
+#pragma unroll
+        for (int e = 0; e < EP; ++e)
+#pragma unroll
+          for (int q = 0; q < C; ++q) b[u][e][q] = basis[min(v0 + u, K - 1) * ld + idx[e] + q];
+#pragma unroll
+      for (int u = 0; u < KS_CH; ++u)
+#pragma unroll
+        for (int e = 0; e < EP; ++e) {
+          const double cr = cf[C * (v0 + u)];
+          if constexpr (CX) {
+            const double ci = cf[C * (v0 + u) + 1];
+            sub[e][0] = fma(cr, b[u][e][0], fma(-ci, b[u][e][1], sub[e][0]));
+            sub[e][1] = fma(cr, b[u][e][1], fma(ci, b[u][e][0], sub[e][1]));
+          } else {
+            sub[e][0] = fma(cr, b[u][e][0], sub[e][0]);
+          }
+        }
     }
-    __syncthreads();  // w complete and cf read before the next pass rewrites cf
+#pragma unroll
+    for (int e = 0; e < EP; ++e)
+#pragma unroll
+      for (int q = 0; q < C; ++q) x[e][q] = tid + nt * e < n ? x[e][q] - sub[e][q] : 0.0;
   }
-  const long nd = CPLX ? 2 * n : n;
   double s = 0.0;
-  for (long j = tid; j < nd; j += KS_THREADS) s = fma(w[j], w[j], s);
+#pragma unroll
+  for (int e = 0; e < EP; ++e)
+#pragma unroll
+    for (int q = 0; q < C; ++q) s = fma(x[e][q], x[e][q], s);
   s = wave_sum64(s);
   if (lane == 0) red[wave] = s;
   __syncthreads();
-  if (tid == 0) {
-    double t = 0.0;
-    for (int i = 0; i < NW; ++i) t += red[i];
-    coef[256] = t;
-    hout[256] = t;
+  double r2 = 0.0;
+  for (int k = 0; k < nw; ++k) r2 += red[k];
+  if (tid == 0) hout[256] = r2;
+  const double a = 1.0 / sqrt(fmax(0.0, r2));
+#pragma unroll
+  for (int e = 0; e < EP; ++e)
+#pragma unroll
+    for (int q = 0; q < C; ++q)
+      if (tid + nt * e < n) {
+        if (K > 0) w[idx[e] + q] = x[e][q];
+        vnext[idx[e] + q] = a * x[e][q];
+      }
+}
+
+// sums of the previous launch's partial results: 16 threads per value
+__device__ __forceinline__ double sum_parts16(const double* __restrict__ pin, int np) {
+  const int l = threadIdx.x & 15;
+  double s = 0.0;
+  for (int i = l; i < np; i += 16) s += pin[i];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
+  return s;
+}
+
+// PHASE 0: dots of w with the basis vectors.  PHASE 1: their sums, w updated,
+// dots of the new w.  PHASE 2: sums, update, |w|^2.  NV >= K, or 16 (then the
+// dots of PHASE 1 read V once more).  Partial results of workgroup g at
+// pout[value * gridDim.x + g]; hout: the coefficients of this phase.
+template <bool CX, int PHASE, int NV>
+__global__ __launch_bounds__(256) void krylov_pass_kernel(const double* __restrict__ basis, long ld, int K,
+                                                          double* __restrict__ w, long n,
+                                                          const double* __restrict__ pin, double* __restrict__ pout,
+                                                          double* __restrict__ hout) {
+  constexpr int C = CX ? 2 : 1;
+  __shared__ double cf[128];
+  __shared__ double red[4][C * NV];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nblk = gridDim.x;
+  const int nacc = C * K;
+  if constexpr (PHASE > 0) {
+    if (tid < 128) cf[tid] = 0.0;
+    __syncthreads();
+    for (int v = tid >> 4; v < nacc; v += 16) {
+      const double s = sum_parts16(pin + (long)v * nblk, nblk);
+      if ((tid & 15) == 0) {
+        cf[v] = s;
+        if (blockIdx.x == 0) hout[v] = s;
+      }
+    }
+    __syncthreads();
   }
+  double acc[NV][C];
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+#pragma unroll
+    for (int q = 0; q < C; ++q) acc[u][q] = 0.0;
+  double nrm = 0.0;
+  auto load = [&](int v0, const long (&o)[2], double (&b)[NV][2][C]) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int q = 0; q < C; ++q) b[u][e][q] = basis[min(v0 + u, K - 1) * ld + o[e] + q];
+  };
+  auto dots = [&](const double (&b)[NV][2][C], const double (&x)[2][C]) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        acc[u][0] = fma(b[u][e][0], x[e][0], acc[u][0]);
+        if constexpr (CX) {
+          acc[u][0] = fma(b[u][e][1], x[e][1], acc[u][0]);
+          acc[u][1] = fma(b[u][e][0], x[e][1], fma(-b[u][e][1], x[e][0], acc[u][1]));
+        }
+      }
+  };
+  auto offsets = [&](long i0, long (&o)[2]) {
+    o[0] = C * min(i0 + tid, n - 1);
+    o[1] = C * min(i0 + tid + 256, n - 1);
+  };
+  auto read = [&](long i0, const long (&o)[2], double (&x)[2][C]) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const double t = w[o[e] + q];
+        x[e][q] = i0 + tid + 256 * e < n ? t : 0.0;
+      }
+  };
+  auto flush = [&](int v0) {  // this workgroup's sums of the dots with vectors v0 ..
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const double s = wave_sum64(acc[u][q]);
+        if (lane == 0) red[wave][C * u + q] = s;
+        acc[u][q] = 0.0;
+      }
+    __syncthreads();
+    for (int t = tid; t < C * NV; t += 256)
+      if (C * v0 + t < nacc)
+        pout[(long)(C * v0 + t) * nblk + blockIdx.x] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+    __syncthreads();
+  };
+  const long step = (long)nblk * KP_TILE;
+  const bool one = K <= NV;
+  if (PHASE > 0 || one) {
+    for (long i0 = (long)blockIdx.x * KP_TILE; i0 < n; i0 += step) {
+      long o[2];
+      double x[2][C], b[NV][2][C];
+      offsets(i0, o);
+      read(i0, o, x);
+      if constexpr (PHASE == 0) {
+        load(0, o, b);
+      } else {
+        double sub[2][C];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int q = 0; q < C; ++q) sub[e][q] = 0.0;
+        for (int v0 = 0; v0 < K; v0 += NV) {
+          load(v0, o, b);
+#pragma unroll
+          for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const double cr = cf[C * (v0 + u)];
+              if constexpr (CX) {
+                const double ci = cf[C * (v0 + u) + 1];
+                sub[e][0] = fma(cr, b[u][e][0], fma(-ci, b[u][e][1], sub[e][0]));
+                sub[e][1] = fma(cr, b[u][e][1], fma(ci, b[u][e][0], sub[e][1]));
+              } else {
+                sub[e][0] = fma(cr, b[u][e][0], sub[e][0]);
+              }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int q = 0; q < C; ++q)
+            if (i0 + tid + 256 * e < n) {
+              x[e][q] -= sub[e][q];
+              w[o[e] + q] = x[e][q];
+            }
+      }
+      if constexpr (PHASE == 2) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int q = 0; q < C; ++q) nrm = fma(x[e][q], x[e][q], nrm);
+      } else if (one) {
+        dots(b, x);
+      }
+    }
+  }
+  if constexpr (PHASE < 2) {
+    if (one) {
+      flush(0);
+    } else {
+      for (int v0 = 0; v0 < K; v0 += NV) {
+        for (long i0 = (long)blockIdx.x * KP_TILE; i0 < n; i0 += step) {
+          long o[2];
+          double x[2][C], b[NV][2][C];
+          offsets(i0, o);
+          read(i0, o, x);
+          load(v0, o, b);
+          dots(b, x);
+        }
+        flush(v0);
+      }
+    }
+  } else {
+    nrm = wave_sum64(nrm);
+    if (lane == 0) red[wave][0] = nrm;
+    __syncthreads();
+    if (tid == 0) pout[blockIdx.x] = (red[0][0] + red[1][0]) + (red[2][0] + red[3][0]);
+  }
+}
+
+// out = sum_v co[v] V_v (pairs when CX); norm: with the partial sums of |out|^2
+struct KryCoef {
+  double c[128];
+};
+template <bool CX>
+__global__ __launch_bounds__(256) void krylov_combine_kernel(const double* __restrict__ basis, long ld, int K,
+                                                             KryCoef co, double* __restrict__ out, long n,
+                                                             double* __restrict__ pout) {
+  constexpr int C = CX ? 2 : 1;
+  __shared__ double red[4];
+  double nrm = 0.0;
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+    double a[C];
+#pragma unroll
+    for (int q = 0; q < C; ++q) a[q] = 0.0;
+    for (int v = 0; v < K; ++v) {
+      const double* b = basis + v * ld + C * i;
+      if constexpr (CX) {
+        const double br = b[0], bi = b[1], cr = co.c[2 * v], ci = co.c[2 * v + 1];
+        a[0] = fma(cr, br, fma(-ci, bi, a[0]));
+        a[1] = fma(cr, bi, fma(ci, br, a[1]));
+      } else {
+        a[0] = fma(co.c[v], b[0], a[0]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+      out[C * i + q] = a[q];
+      nrm = fma(a[q], a[q], nrm);
+    }
+  }
+  if (!pout) return;  // uniform over the grid
+  nrm = wave_sum64(nrm);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = nrm;
+  __syncthreads();
+  if (threadIdx.x == 0) pout[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+__global__ __launch_bounds__(256) void krylov_norm_kernel(const double* __restrict__ x, long nd,
+                                                          double* __restrict__ pout) {
+  __shared__ double red[4];
+  double s = 0.0;
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < nd; i += gridDim.x * 256L) s = fma(x[i], x[i], s);
+  s = wave_sum64(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) pout[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+// y = x / |x| from the partial sums of |x|^2 (y may be x)
+__global__ __launch_bounds__(256) void krylov_scale_kernel(double* y, const double* x, long nd,
+                                                           const double* __restrict__ pin, int np,
+                                                           double* __restrict__ hout) {
+  __shared__ double red[4];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < np; i += 256) s += pin[i];
+  s = wave_sum64(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  const double r2 = (red[0] + red[1]) + (red[2] + red[3]);
+  if (hout && blockIdx.x == 0 && threadIdx.x == 0) *hout = r2;
+  const double a = 1.0 / sqrt(fmax(0.0, r2));
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < nd; i += gridDim.x * 256L) y[i] = a * x[i];
 }
 
 // row sums of squares: one block per row
@@ -837,12 +1097,6 @@ void scaled_copy(tn_ctx* c, double* y, const double* x, double a, long n) {
   hipLaunchKernelGGL(scaled_copy_kernel, dim3(grid1d(n)), dim3(256), 0, c->stream, y, x, a, n);
   TN_HIP(hipGetLastError());
 }
-void scale_rnorm(tn_ctx* c, double* y, const double* x, const double* r2_dev, long n) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(scale_rnorm_kernel, dim3(grid1d(n)), dim3(256), 0, c->stream, y, x, r2_dev, n);
-  TN_HIP(hipGetLastError());
-}
-
 void multi_dot(tn_ctx* c, const double* basis, long ld, int count, const double* x, long n, bool cplx,
                double* out_dev, double* out_host) {
   TN_REQUIRE(count >= 1, TN_E_INVALID, "multi_dot: count");
@@ -898,40 +1152,82 @@ void add_scaled_dev(tn_ctx* c, double* y, const double* x, const double* coef_de
   TN_HIP(hipGetLastError());
 }
 
-bool krylov_ortho_small(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, bool cplx,
-                        double* coef_dev, double* hout) {
-  if (n > 4L * KS_THREADS || K < 1 || K > 61) return false;
-  if (cplx)
-    hipLaunchKernelGGL(krylov_ortho_small_kernel<true>, dim3(1), dim3(KS_THREADS), 0, c->stream, basis, ld, K, w,
-                       n, coef_dev, hout);
+// |x|^2 partial sums per workgroup, and workgroups of a scaling
+static int krylov_blocks(long n) { return (int)std::min<long>(KP_BLOCKS, std::max<long>(1, (n + KP_TILE - 1) / KP_TILE)); }
+
+template <bool CX>
+static bool krylov_small(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, double* vnext,
+                         double* hout) {
+  if (n > KS_MAX) return false;
+  // one element a thread, or four
+  if (n <= KS_THREADS)
+    hipLaunchKernelGGL((krylov_small_kernel<CX, 1>), dim3(1), dim3((unsigned)((n + 63) / 64 * 64)), 0, c->stream, basis,
+                       ld, K, w, (int)n, vnext, hout);
   else
-    hipLaunchKernelGGL(krylov_ortho_small_kernel<false>, dim3(1), dim3(KS_THREADS), 0, c->stream, basis, ld, K, w,
-                       n, coef_dev, hout);
+    hipLaunchKernelGGL((krylov_small_kernel<CX, 4>), dim3(1), dim3(KS_THREADS), 0, c->stream, basis, ld, K, w, (int)n,
+                       vnext, hout);
   TN_HIP(hipGetLastError());
   return true;
 }
 
-void multi_axpy_sub(tn_ctx* c, const double* basis, long ld, int count, const double* coef_dev, double* x,
-                    long n, bool cplx) {
-  if (n <= 0 || count <= 0) return;
-  if (cplx)
-    hipLaunchKernelGGL(multi_axpy_kernel<true>, dim3(grid1d(n)), dim3(256), 0, c->stream, basis, ld, count,
-                       coef_dev, x, n, 1);
-  else
-    hipLaunchKernelGGL(multi_axpy_kernel<false>, dim3(grid1d(n)), dim3(256), 0, c->stream, basis, ld, count,
-                       coef_dev, x, n, 1);
+template <bool CX, int NV>
+static void krylov_passes(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, double* p1, double* p2,
+                          double* p3, double* hout) {
+  const dim3 g(krylov_blocks(n)), b(256);
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 0, NV>), g, b, 0, c->stream, basis, ld, K, w, n, nullptr, p1, nullptr);
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 1, NV>), g, b, 0, c->stream, basis, ld, K, w, n, p1, p2, hout);
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 2, NV>), g, b, 0, c->stream, basis, ld, K, w, n, p2, p3, hout + 128);
   TN_HIP(hipGetLastError());
 }
 
-void lincomb(tn_ctx* c, const double* basis, long ld, int count, const double* coef_dev, double* out, long n,
-             bool cplx) {
-  if (n <= 0) return;
-  if (cplx)
-    hipLaunchKernelGGL(multi_axpy_kernel<true>, dim3(grid1d(n)), dim3(256), 0, c->stream, basis, ld, count,
-                       coef_dev, out, n, 0);
-  else
-    hipLaunchKernelGGL(multi_axpy_kernel<false>, dim3(grid1d(n)), dim3(256), 0, c->stream, basis, ld, count,
-                       coef_dev, out, n, 0);
+template <bool CX>
+static void krylov_step_t(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, double* vnext,
+                          double* hout) {
+  if (krylov_small<CX>(c, basis, ld, K, w, n, vnext, hout)) return;
+  const int nb = krylov_blocks(n), nacc = CX ? 2 * K : K;
+  const long nd = CX ? 2 * n : n;
+  double* p1 = (double*)c->workspace(WS_KRY_PART, (size_t)(2 * nacc + 1) * nb * sizeof(double));
+  double* p2 = p1 + (size_t)nacc * nb;
+  double* p3 = p2 + (size_t)nacc * nb;
+  if (K <= 4) krylov_passes<CX, 4>(c, basis, ld, K, w, n, p1, p2, p3, hout);
+  else if (K <= 8) krylov_passes<CX, 8>(c, basis, ld, K, w, n, p1, p2, p3, hout);
+  else krylov_passes<CX, 16>(c, basis, ld, K, w, n, p1, p2, p3, hout);
+  hipLaunchKernelGGL(krylov_scale_kernel, dim3(grid1d(nd)), dim3(256), 0, c->stream, vnext, (const double*)w, nd,
+                     (const double*)p3, nb, hout + 256);
+  TN_HIP(hipGetLastError());
+}
+
+void krylov_step(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, bool cplx, double* vnext,
+                 double* hout) {
+  TN_REQUIRE(K >= 1 && K <= KRY_MAX && n >= 1, TN_E_INVALID, "Krylov step: basis size");
+  if (cplx) krylov_step_t<true>(c, basis, ld, K, w, n, vnext, hout);
+  else krylov_step_t<false>(c, basis, ld, K, w, n, vnext, hout);
+}
+
+void krylov_normalize(tn_ctx* c, double* y, const double* x, long nd, double* hout) {
+  // the one-workgroup step without basis vectors leaves x as it is
+  if (krylov_small<false>(c, nullptr, 0, 0, const_cast<double*>(x), nd, y, hout - 256)) return;
+  const int nb = krylov_blocks(nd);
+  double* p = (double*)c->workspace(WS_KRY_PART, (size_t)nb * sizeof(double));
+  hipLaunchKernelGGL(krylov_norm_kernel, dim3(nb), dim3(256), 0, c->stream, x, nd, p);
+  hipLaunchKernelGGL(krylov_scale_kernel, dim3(grid1d(nd)), dim3(256), 0, c->stream, y, x, nd, (const double*)p, nb,
+                     hout);
+  TN_HIP(hipGetLastError());
+}
+
+void krylov_combine(tn_ctx* c, const double* basis, long ld, int K, const double* co, double* out, long n, bool cplx,
+                    bool normalize) {
+  TN_REQUIRE(K >= 1 && K <= KRY_MAX && n >= 1, TN_E_INVALID, "Krylov combination: basis size");
+  KryCoef kc{};
+  std::copy(co, co + (cplx ? 2 * K : K), kc.c);
+  const int nb = krylov_blocks(n);
+  const long nd = cplx ? 2 * n : n;
+  double* p = normalize ? (double*)c->workspace(WS_KRY_PART, (size_t)nb * sizeof(double)) : nullptr;
+  if (cplx) hipLaunchKernelGGL(krylov_combine_kernel<true>, dim3(nb), dim3(256), 0, c->stream, basis, ld, K, kc, out, n, p);
+  else hipLaunchKernelGGL(krylov_combine_kernel<false>, dim3(nb), dim3(256), 0, c->stream, basis, ld, K, kc, out, n, p);
+  if (normalize)
+    hipLaunchKernelGGL(krylov_scale_kernel, dim3(grid1d(nd)), dim3(256), 0, c->stream, out, (const double*)out, nd,
+                       (const double*)p, nb, (double*)nullptr);
   TN_HIP(hipGetLastError());
 }
 

@@ -372,24 +372,21 @@ void copy_f64(tn_ctx* c, double* dst, const double* src, long n);
 // been synchronised (no separate copy).
 void multi_dot(tn_ctx* c, const double* basis, long ld, int count, const double* x, long n,
                bool cplx, double* out_dev, double* out_host = nullptr);
-// x -= sum_i coef[i] * basis_i ; coef on device (real or complex pairs)
-void multi_axpy_sub(tn_ctx* c, const double* basis, long ld, int count, const double* coef_dev,
-                    double* x, long n, bool cplx);
-// out = sum_i coef[i] * basis_i ; coef on device
-void lincomb(tn_ctx* c, const double* basis, long ld, int count, const double* coef_dev,
-             double* out, long n, bool cplx);
 // x *= s (s real, on host)
 void scale_f64(tn_ctx* c, double* x, double s, long n);
 // y = a*x (a real), n doubles
 void scaled_copy(tn_ctx* c, double* y, const double* x, double a, long n);
-// one Krylov orthogonalisation step (two passes against K basis vectors, then
-// |w|^2) in a single launch for short vectors; coefficients at coef_dev[0..),
-// [128..), |w|^2 at [256], mirrored to hout.  Returns false (nothing queued)
-// when n or K is outside its range
-bool krylov_ortho_small(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, bool cplx,
-                        double* coef_dev, double* hout);
-// y = x / sqrt(max(0, *r2_dev)) (r2_dev: a device scalar)
-void scale_rnorm(tn_ctx* c, double* y, const double* x, const double* r2_dev, long n);
+constexpr int KRY_MAX = 62;  // basis vectors of a Krylov step (complex pairs fit in 128)
+// one Krylov step: w orthogonalised against K basis vectors twice, vnext = w /
+// |w|.  hout (mapped host memory) receives the coefficients of the two passes
+// at 0 and 128 (pairs when cplx) and |w|^2 at 256.
+void krylov_step(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, bool cplx, double* vnext,
+                 double* hout);
+// y = x / |x| (nd doubles; y may be x), |x|^2 to *hout (mapped host memory)
+void krylov_normalize(tn_ctx* c, double* y, const double* x, long nd, double* hout);
+// out = sum_v co[v] V_v (co on the host, pairs when cplx), normalised on request
+void krylov_combine(tn_ctx* c, const double* basis, long ld, int K, const double* co, double* out, long n, bool cplx,
+                    bool normalize);
 // row sum of squares of a (rows x L) row-major matrix into out[rows]
 void row_norms2(tn_ctx* c, const double* X, long rows, long L, long ld, double* out);
 // y += scale * coef_dev[0] * x (complex coefficient pair when cplx)

@@ -1223,21 +1223,9 @@ struct Krylov {
     for (hipEvent_t& ev : c->kry_ev)
       if (!ev) TN_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   }
-  // w <- w - V_{0..K-1} (V^H w), twice (queued; results in slot s)
+  // w <- w - V_{0..K-1} (V^H w), twice, and V(K) = w / |w| (queued; results in slot s)
   void orthogonalize_async(int K, int s) {
-    // coefficient scratch: pass 1 at [0, 2K), pass 2 at [128, 128+2K),
-    // |w|^2 at 256 (K <= 61 basis vectors, complex pairs fit in 128)
-    double* hd = c->pinned_dev + 512 * s;
-    if (krylov_ortho_small(c, base, nd, K, w, n, cx, coef, hd)) {
-      ensure_events();
-      TN_HIP(hipEventRecord(c->kry_ev[s], c->stream));
-      return;
-    }
-    multi_dot(c, base, nd, K, w, n, cx, coef, hd);
-    multi_axpy_sub(c, base, nd, K, coef, w, n, cx);
-    multi_dot(c, base, nd, K, w, n, cx, coef + 128, hd + 128);
-    multi_axpy_sub(c, base, nd, K, coef + 128, w, n, cx);
-    multi_dot(c, w, nd, 1, w, n, cx, coef + 256, hd + 256);
+    krylov_step(c, base, nd, K, w, n, cx, V(K), c->pinned_dev + 512 * s);
     ensure_events();
     TN_HIP(hipEventRecord(c->kry_ev[s], c->stream));
   }
@@ -1252,25 +1240,17 @@ struct Krylov {
     }
     nrm2 = hb[256];
   }
-  void orthogonalize(int K, std::vector<cplx>& h, double& nrm2) {
-    orthogonalize_async(K, 0);
-    orthogonalize_wait(K, 0, h, nrm2);
-  }
-  // V(i) = w / |w| with |w|^2 of the last queued step (device side)
-  void next_from_w(int i) { scale_rnorm(c, V(i), w, coef + 256, nd); }
-  // out = sum_i coefs[i] V_i
-  void combine(int K, const std::vector<cplx>& co, double* out) {
-    // the pinned upload area may still feed an earlier copy: drain the stream first
-    TN_HIP(hipStreamSynchronize(c->stream));
-    double* hc = c->pinned + 2048;
-    const int nc = cx ? 2 * K : K;
+  // V(0) = x / |x|, queued; |x|^2 is at start_norm2() once the first step has been waited for
+  void start(const double* x) { krylov_normalize(c, V(0), x, nd, c->pinned_dev + 1536); }
+  double start_norm2() const { return c->pinned[1536]; }
+  // out = sum_i coefs[i] V_i, normalised on request (queued)
+  void combine(int K, const std::vector<cplx>& co, double* out, bool normalize = false) {
+    double h[128];
     for (int i = 0; i < K; ++i) {
-      if (cx) { hc[2 * i] = co[i].real(); hc[2 * i + 1] = co[i].imag(); }
-      else hc[i] = co[i].real();
+      if (cx) { h[2 * i] = co[i].real(); h[2 * i + 1] = co[i].imag(); }
+      else h[i] = co[i].real();
     }
-    double* dc = coef + 512;  // [512, 512 + 2K)
-    TN_HIP(hipMemcpyAsync(dc, hc, nc * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    lincomb(c, base, nd, K, dc, out, n, cx);
+    krylov_combine(c, base, nd, K, h, out, n, cx, normalize);
   }
 };
 
@@ -1449,12 +1429,9 @@ double tn::krylov_eig_op(tn_ctx* c, bool cx, long n, const std::function<void(co
   Krylov K(c, cx, n, 2 * kdim + 2);
   tn_krylov_info inf{0, 0, 1, NAN};
   // v0 = x0 / |x0|
-  double b0;
   {
     PhaseTimer pt(c, PH_KRYLOV);
-    b0 = std::sqrt(K.norm2(phi));
-    TN_REQUIRE(std::isfinite(b0) && b0 > 0.0, TN_E_NUMERIC, "eig_solver: zero or non-finite start vector");
-    scaled_copy(K.c, K.V(0), phi, 1.0 / b0, K.nd);
+    K.start(phi);
   }
   std::vector<double> Hm((size_t)(kdim + 1) * (kdim + 1), 0.0);
   auto H = [&](int i, int j) -> double& { return Hm[(size_t)i * (kdim + 1) + j]; };
@@ -1473,10 +1450,6 @@ double tn::krylov_eig_op(tn_ctx* c, bool cx, long n, const std::function<void(co
     // step ends the cycle on an invariant subspace)
     const bool ahead = Kn < kdim;
     if (ahead) {
-      {
-        PhaseTimer pt(c, PH_KRYLOV);
-        K.next_from_w(Kn);
-      }
       apply(K.V(Kn), K.w);
       PhaseTimer pt(c, PH_KRYLOV);
       K.orthogonalize_async(Kn + 1, sl ^ 1);
@@ -1484,6 +1457,10 @@ double tn::krylov_eig_op(tn_ctx* c, bool cx, long n, const std::function<void(co
     {
       PhaseTimer pt(c, PH_KRYLOV);
       K.orthogonalize_wait(Kn, sl, h, r2);
+    }
+    if (inf.numops == 0) {
+      const double b0 = std::sqrt(K.start_norm2());
+      TN_REQUIRE(std::isfinite(b0) && b0 > 0.0, TN_E_NUMERIC, "eig_solver: zero or non-finite start vector");
     }
     inf.numops++;
     H(Kn - 1, Kn - 1) = h[Kn - 1].real();
@@ -1507,9 +1484,7 @@ double tn::krylov_eig_op(tn_ctx* c, bool cx, long n, const std::function<void(co
         PhaseTimer pt(c, PH_KRYLOV);
         std::vector<cplx> co(Kn);
         for (int i = 0; i < Kn; ++i) co[i] = U[(size_t)i * Kn + 0];
-        K.combine(Kn, co, phi);
-        const double ny = std::sqrt(K.norm2(phi));
-        scale_f64(K.c, phi, 1.0 / ny, K.nd);
+        K.combine(Kn, co, phi, true);  // after the step queued ahead, which is dropped
         if (info) *info = inf;
         return theta[0];
       }
@@ -1568,17 +1543,12 @@ void krylov_expm(tn_env* e, double* phi, cplx t, int kdim, int maxiter, double t
   double last = 1.0;       // last accepted sub-step
   std::vector<cplx> h;
   double r2;
-  while (remaining > 0.0 && inf.numiter < maxiter) {
+  bool zero = false;  // the vector vanished: nothing to propagate
+  while (!zero && remaining > 0.0 && inf.numiter < maxiter) {
     inf.numiter++;
-    double nx;
     {
       PhaseTimer pt(e->ctx, PH_KRYLOV);
-      nx = std::sqrt(K.norm2(phi));
-    }
-    if (nx == 0.0) break;
-    {
-      PhaseTimer pt(e->ctx, PH_KRYLOV);
-      scaled_copy(K.c, K.V(0), phi, 1.0 / nx, K.nd);
+      K.start(phi);
     }
     std::vector<double> Hm((size_t)(kdim + 1) * (kdim + 1), 0.0);
     auto H = [&](int i, int j) -> double& { return Hm[(size_t)i * (kdim + 1) + j]; };
@@ -1593,10 +1563,6 @@ void krylov_expm(tn_env* e, double* phi, cplx t, int kdim, int maxiter, double t
     }
     while (true) {
       if (Kn + 1 < kdim) {
-        {
-          PhaseTimer pt(e->ctx, PH_KRYLOV);
-          K.next_from_w(Kn + 1);
-        }
         apply_op(e, K.V(Kn + 1), K.w, prec);
         PhaseTimer pt(e->ctx, PH_KRYLOV);
         K.orthogonalize_async(Kn + 2, sl ^ 1);
@@ -1604,6 +1570,11 @@ void krylov_expm(tn_env* e, double* phi, cplx t, int kdim, int maxiter, double t
       {
         PhaseTimer pt(e->ctx, PH_KRYLOV);
         K.orthogonalize_wait(Kn + 1, sl, h, r2);
+      }
+      const double nx = std::sqrt(K.start_norm2());
+      if (nx == 0.0) {
+        zero = true;
+        break;
       }
       inf.numops++;
       H(Kn, Kn) = h[Kn].real();
@@ -1634,7 +1605,7 @@ void krylov_expm(tn_env* e, double* phi, cplx t, int kdim, int maxiter, double t
       if (err <= tol * remaining || beta <= 1e-14 * hmax) {
         PhaseTimer pt(e->ctx, PH_KRYLOV);
         for (auto& v : y) v *= nx;
-        K.combine(Kn, y, phi);  // waits for the step queued ahead, then drops it
+        K.combine(Kn, y, phi);  // after the step queued ahead, which is dropped
         remaining = 0.0;
         break;
       }
