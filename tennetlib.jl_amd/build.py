@@ -32,7 +32,7 @@ OBJ = HERE / "_build"
 OUT = HERE / "libtnhip.so"
 OBJ_HARDENED = HERE / "_build_hardened"
 OUT_HARDENED = HERE / "libtnhip_hardened.so"
-SOURCES = ["gemm.hip", "gemm_fast.hip", "tensor_ops.hip", "svd.hip", "eig_dc.hip", "eig_small.hip", "qr.hip", "tnhip_api.hip",
+SOURCES = ["gemm.hip", "gemm_fast.hip", "tensor_ops.hip", "svd.hip", "eig_dc.hip", "eig_small.hip", "mv_small.hip", "qr.hip", "tnhip_api.hip",
            "ttn.hip", "qn.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -336,6 +336,11 @@ struct WStepDesc {
   // read the input only where the operator has entries (the rest may be undefined)
   bool csr = false;
 };
+// H psi in FP64 (complex128 when cplx) in one launch (mv_small.hip): L[(w0
+// a'), a], psi[a, S, b], op, R[(w2 b), b'] to out[a', S', b'].  false (nothing
+// queued) for sizes that its workgroups do not take; timed: as PH_MV_GEMM.
+bool mv_small(tn_ctx* c, bool cplx, const SparseOp& op, const void* L, const void* v, const void* R, void* out, int w0,
+              int w2, int DD, long chil, long chir, bool timed);
 void wstep(tn_ctx* c, bool fp32, const WStepDesc& w);
 // W step from FP32 input writing the result as bf16 hi/lo pairs at the
 // positions w.out_* would address (w.out is ignored)

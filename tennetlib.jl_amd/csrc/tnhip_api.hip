@@ -1080,6 +1080,7 @@ void matvec_mpo(tn_env* e, const void* v, void* out, int prec) {
   if (prec == TN_PREC_FP64) P = cx ? Prec::Z64 : Prec::F64;
   else if (prec == TN_PREC_FP32) { P = Prec::F32; f32 = true; }
   else throw Error(TN_E_INVALID, "unknown precision");
+  if (!f32 && mv_small(c, cx, op, L.buf.p, v, R.buf.p, out, w0, w2, DD, chil, chir, true)) return;
   const size_t es = f32 ? 4 : e->esz;
   const int m2 = cx ? 2 : 1;
   // FP32 operands are copies of ours: their rows are padded to 16 bytes so the
@@ -1406,6 +1407,7 @@ void matvec_noalloc(tn_env* e, const void* v, void* out) {
   TN_REQUIRE(need <= NOALLOC_SCRATCH_BYTES, TN_E_INVALID,
              "allocation-free product needs " + std::to_string(need) + " bytes of scratch, more than the fixed " +
                  std::to_string(NOALLOC_SCRATCH_BYTES));
+  if (mv_small(c, cx, op, L.buf.p, v, R.buf.p, out, w0, w2, DD, chil, chir, false)) return;
   g1.split_ws = g3.split_ws = base + align256(t1) + align256(t2);
   g1.split_cap = g3.split_cap = split;
   gemm(c, P, g1);
