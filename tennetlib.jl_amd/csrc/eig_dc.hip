@@ -227,26 +227,15 @@ __global__ __launch_bounds__(256) void trd_step_kernel(double* __restrict__ A, l
   double* wj = vj + mj;
   double* vn = wj + mj;
   const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // issue the loads of row j+1 and of this wave's first own row up front, so
-  // their latency overlaps the vector set-up (rows up to 6144 / 1024 long)
-  constexpr int OV = 24, RV = 16;
+  // issue the loads of row j+1 up front, so their latency overlaps the vector
+  // set-up (rows up to 6144 long)
+  constexpr int OV = 24;
   const double* orow = A + (long)(j + 1) * ld + (j + 2);
   double ov[OV];
 #pragma unroll
   for (int u = 0; u < OV; ++u) {
     const int t = tid + 256 * u;
     ov[u] = (t < mn) ? orow[t] : 0.0;
-  }
-  const int rr0 = g * 4 + wave;
-  const bool pre = (mn <= 64 * RV) && (rr0 < mn);
-  double rv[RV];
-  {
-    const double* row0 = A + (long)(j + 2 + (pre ? rr0 : 0)) * ld + (j + 2);
-#pragma unroll
-    for (int u = 0; u < RV; ++u) {
-      const int t = lane + 64 * u;
-      rv[u] = (pre && t < mn) ? row0[t] : 0.0;
-    }
   }
   // v_j and y_j (up to 1024 entries) are loaded before the reduction of the
   // partial sums, so both global round trips overlap
@@ -322,26 +311,14 @@ __global__ __launch_bounds__(256) void trd_step_kernel(double* __restrict__ A, l
   }
   // own rows: update of step j and the rows of y_{j+1}
   double dot = 0.0;
-  for (int rr = rr0; rr < mn; rr += G * 4) {
+  for (int rr = g * 4 + wave; rr < mn; rr += G * 4) {
     double* row = A + (long)(j + 2 + rr) * ld + (j + 2);
     const double vr = vj[rr + 1], wr = wj[rr + 1];
     double acc = 0.0;
-    if (pre && rr == rr0) {
-#pragma unroll
-      for (int u = 0; u < RV; ++u) {
-        const int t = lane + 64 * u;
-        if (t < mn) {
-          const double old = rv[u];
-          acc += old * vn[t];
-          if (tj != 0.0) row[t] = old - vr * wj[t + 1] - wr * vj[t + 1];
-        }
-      }
-    } else {
-      for (int t = lane; t < mn; t += 64) {
-        const double old = row[t];
-        acc += old * vn[t];
-        if (tj != 0.0) row[t] = old - vr * wj[t + 1] - wr * vj[t + 1];
-      }
+    for (int t = lane; t < mn; t += 64) {
+      const double old = row[t];
+      acc += old * vn[t];
+      if (tj != 0.0) row[t] = old - vr * wj[t + 1] - wr * vj[t + 1];
     }
     acc = wave_sum64(acc);
     if (lane == 0) {
@@ -352,6 +329,100 @@ __global__ __launch_bounds__(256) void trd_step_kernel(double* __restrict__ A, l
   }
   dot = block_sum(dot, red);
   if (tid == 0) partn[g] = dot;
+}
+
+// The fused step for rows of up to 64 U entries (mn = p - j - 2), a wavefront
+// per row: every wavefront holds v_j, w_j, row j + 1 and its own row in
+// registers (entry t = lane + 64 u) and forms the reflector itself, so nothing
+// but the final partial sum passes through LDS.  Bound by the launch and one
+// chain of load, four sums over the wavefront, square root and division: 4.1 us
+// a column up to 256 entries, 4.9 up to 512 (through LDS with a workgroup's
+// sums and two chained loads 7.0 us).
+template <int U>
+__global__ __launch_bounds__(256) void trd_step_reg_kernel(double* __restrict__ A, long ld, int p, int j,
+                                                           const double* __restrict__ vj_in,
+                                                           const double* __restrict__ yj,
+                                                           const double* __restrict__ partj, int npj,
+                                                           double* __restrict__ vn_out, double* __restrict__ yn,
+                                                           double* __restrict__ partn, double* __restrict__ dv,
+                                                           double* __restrict__ ev, double* __restrict__ tauv) {
+  __shared__ double red[4];
+  const int mn = p - j - 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rr = blockIdx.x * 4 + wave, rc = min(rr, mn - 1);
+  const double* orow = A + (long)(j + 1) * ld + (j + 2);
+  double* row = A + (long)(j + 2 + rc) * ld + (j + 2);
+  // all loads of the step, past the end from the last entry (zeroed below)
+  double o[U], rv[U], pv[U], w[U], ps[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ps[i] = partj[min(lane + 64 * i, npj - 1)];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int t = min(lane + 64 * u, mn - 1);
+    pv[u] = vj_in[t + 1];
+    w[u] = yj[t + 1];
+    o[u] = orow[t];
+    rv[u] = row[t];
+  }
+  const double tj = tauv[j], v0 = vj_in[0], y0 = yj[0], vr = vj_in[rc + 1], yr = yj[rc + 1], dj = orow[-1];
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s += lane + 64 * i < npj ? ps[i] : 0.0;
+  const double hs = tj != 0.0 ? 0.5 * tj * wave_sum64(s) : 0.0;
+  const double w0 = tj != 0.0 ? y0 - hs * v0 : 0.0, wr = tj != 0.0 ? yr - hs * vr : 0.0;
+  // new row j+1 and its reflector
+  double ss = 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int t = lane + 64 * u;
+    w[u] = t < mn && tj != 0.0 ? w[u] - hs * pv[u] : 0.0;
+    pv[u] = t < mn ? pv[u] : 0.0;
+    o[u] = t < mn ? o[u] - v0 * w[u] - w0 * pv[u] : 0.0;
+    ss += t > 0 ? o[u] * o[u] : 0.0;
+  }
+  double tau, alpha, scale;
+  trd_reflector(read_lane(o[0], 0), wave_sum64(ss), tau, alpha, scale);
+  double a = 0.0, b = 0.0, acc = 0.0, vown = 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const double v = lane + 64 * u == 0 ? 1.0 : o[u] * scale;
+    o[u] = v;
+    a += w[u] * v;
+    b += pv[u] * v;
+    acc += rv[u] * v;
+    vown = lane + 64 * u == rc ? v : vown;
+  }
+  a = wave_sum64(a);
+  b = wave_sum64(b);
+  acc = wave_sum64(acc);
+  vown = wave_sum64(vown);  // one lane holds it
+  if (tj != 0.0 && rr < mn) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (lane + 64 * u < mn) row[lane + 64 * u] = rv[u] - vr * w[u] - wr * pv[u];
+  }
+  const double yv = tau * (acc - vr * a - wr * b);
+  if (lane == 0) {
+    if (rr < mn) yn[rr] = yv;
+    red[wave] = rr < mn ? yv * vown : 0.0;
+  }
+  if (rr == 0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = lane + 64 * u;
+      if (t < mn) {
+        A[(long)(j + 2 + t) * ld + (j + 1)] = o[u];
+        vn_out[t] = o[u];
+      }
+    }
+    if (lane == 0) {
+      dv[j + 1] = dj - 2.0 * v0 * w0;
+      ev[j + 1] = alpha;
+      tauv[j + 1] = tau;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) partn[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // ---- blocked reduction for large p (LAPACK dlatrd panels of NBT columns).
@@ -1782,8 +1853,12 @@ static void trd_columns(tn_ctx* c, double* G, int P, long ldg, int j0, double* d
   for (int j = 0; j + 2 <= j0; ++j) {
     const int mj = P - j - 1, mn = mj - 1;
     const int nwg = std::min(256, (mn + 3) / 4);
-    hipLaunchKernelGGL(trd_step_kernel, dim3(nwg), dim3(256), 3 * (size_t)mj * sizeof(double), c->stream, G, ldg, P, j,
-                       cv, cy, cp, cnp, nv, ny, npart, dv, ev, tauv);
+    if (mn > 1020)
+      hipLaunchKernelGGL(trd_step_kernel, dim3(nwg), dim3(256), 3 * (size_t)mj * sizeof(double), c->stream, G, ldg, P,
+                         j, cv, cy, cp, cnp, nv, ny, npart, dv, ev, tauv);
+    else  // a row in the registers of a wavefront, at most 256 partial sums (trd_reflect_kernel's: (mn + 1) / 4)
+      hipLaunchKernelGGL(mn <= 256 ? trd_step_reg_kernel<4> : mn <= 512 ? trd_step_reg_kernel<8> : trd_step_reg_kernel<16>,
+                         dim3(nwg), dim3(256), 0, c->stream, G, ldg, P, j, cv, cy, cp, cnp, nv, ny, npart, dv, ev, tauv);
     std::swap(cv, nv);
     std::swap(cy, ny);
     std::swap(cp, npart);
