@@ -437,17 +437,17 @@ __global__ __launch_bounds__(256) void trd_step_reg_kernel(double* __restrict__ 
 // rank-2 update).  Vectors are stored by global row in the panel buffers
 // P = [V; W] and Q = [W; V] (2 NBT rows of length p; unused rows zero).
 constexpr int NBT = 32;
-constexpr int RCHUNK = 256;  // row entries per workgroup in trd_panel_row_kernel (one per thread)
-// dynamic LDS of trd_panel_row_kernel: four waves' products, (2 NBT + 1) rows of 65
-constexpr size_t TRD_ROW_LDS = (size_t)4 * (2 * NBT + 1) * 65 * sizeof(double);
+constexpr int RCHUNK = 64;  // row entries per workgroup in trd_panel_row_kernel (one per lane)
 
 // Column j: forms w_{k-1} (the previous column's, from y_{j-1} and the
 // partial sums of y_{j-1}^T v_{j-1}), then the current row x (stored in xbuf,
 // entries c = 0..m-1 for columns j+1+c) with partial sums of sum_{c>=1} x_c^2,
 // v_i . x and w_i . x over c >= 1 (i < k); d_j from workgroup 0.
-// One entry per thread: its panel entries are loaded first, and the values
-// every thread shares (y_{j-1}^T v_{j-1}, v_i[j], w_i[j]) are read by each
-// wave itself, so nothing waits on a barrier before the row is formed.
+// Bound by latency: 64 entries a workgroup, a quarter of the panel's columns a
+// wavefront (with 256 entries, a wavefront for all columns and a branch per
+// column, whose loads then waited for each other, p / 256 workgroups took
+// 10.4 us at p = 4096; now 4.4).  All loads come first; v_i[j] and w_i[j]
+// are one load, a column per lane.
 // Grid: ceil(m / RCHUNK) workgroups.
 __global__ __launch_bounds__(256) void trd_panel_row_kernel(const double* __restrict__ A, long ld, int p, int j, int k,
                                                             double* __restrict__ P, double* __restrict__ Q,
@@ -456,22 +456,27 @@ __global__ __launch_bounds__(256) void trd_panel_row_kernel(const double* __rest
                                                             const double* __restrict__ tauv,
                                                             double* __restrict__ xbuf, double* __restrict__ partA,
                                                             double* __restrict__ dv) {
-  __shared__ double accs[4][2 * NBT + 1];
-  extern __shared__ double tr[];  // per wave (2 NBT + 1) x 65: the products, transposed for the sums
-  const int m = p - j - 1, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int c = blockIdx.x * RCHUNK + tid;
+  constexpr int NI = NBT / 4;        // panel columns of a wavefront
+  __shared__ double xp[4][RCHUNK];
+  __shared__ double tr[4][2 * NI][RCHUNK + 1];  // products, transposed for the sums
+  const int m = p - j - 1, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = blockIdx.x * RCHUNK + lane, i0 = wave * NI;
   const bool act = c < m;
-  const long r = j + 1 + c;  // global row / column index
-  // this entry's loads
-  double V[NBT], W[NBT];
+  const long r = j + 1 + min(c, m - 1);  // global row / column index
+  // this entry's panel columns (rows of P not in use yet hold zeros), row j of the panel, one column a lane
+  double V[NI], W[NI];
 #pragma unroll
-  for (int i = 0; i < NBT; ++i) {
-    V[i] = (act && i < k) ? P[(long)i * p + r] : 0.0;
-    W[i] = (act && i < k - 1) ? P[(long)(NBT + i) * p + r] : 0.0;
+  for (int i = 0; i < NI; ++i) {
+    V[i] = P[(long)(i0 + i) * p + r];
+    W[i] = P[(long)(NBT + i0 + i) * p + r];
   }
-  const double a = act ? A[r * ld + j] : 0.0;  // column j below the diagonal (the lower triangle is current)
-  const double yp = (act && k >= 1) ? yprev[c + 1] : 0.0;
-  // hs = (tau_{j-1} / 2) y_{j-1}^T v_{j-1}, reduced by every wave alike
+  const int il = lane & (NBT - 1);
+  const double sv = P[(long)il * p + j];
+  double sw = P[(long)(NBT + il) * p + j];
+  const double a = A[r * ld + j];  // column j below the diagonal (the lower triangle is current)
+  const double yp = k >= 1 ? yprev[r - j] : 0.0, y0 = k >= 1 ? yprev[0] : 0.0;
+  const double aj = A[(long)j * ld + j];
+  // hs = (tau_{j-1} / 2) y_{j-1}^T v_{j-1}, reduced by every wavefront alike
   double hs = 0.0;
   if (k >= 1) {
     double s = 0.0;
@@ -479,76 +484,63 @@ __global__ __launch_bounds__(256) void trd_panel_row_kernel(const double* __rest
     hs = 0.5 * tauv[j - 1] * wave_sum64(s);
   }
   // w_{k-1} = y_{j-1} - hs v_{k-1} over rows >= j
-  double wj = 0.0;
   if (k >= 1) {
-    wj = yprev[0] - hs * P[(long)(k - 1) * p + j];
-    double vk1 = 0.0;  // V[k - 1], selected without a runtime index (keeps V in registers)
+    sw = il == k - 1 ? y0 - hs * sv : sw;
 #pragma unroll
-    for (int i = 0; i < NBT; ++i)
-      if (i == k - 1) vk1 = V[i];
-    const double wn = yp - hs * vk1;
-#pragma unroll
-    for (int i = 0; i < NBT; ++i)
-      if (i == k - 1) W[i] = wn;
-    if (act) {
-      P[(long)(NBT + k - 1) * p + r] = wn;
-      Q[(long)(k - 1) * p + r] = wn;
-    }
-    if (blockIdx.x == 0 && tid == 0) {
-      P[(long)(NBT + k - 1) * p + j] = wj;
-      Q[(long)(k - 1) * p + j] = wj;
-    }
-  }
-  // x = A[j, r] - sum_i (v_i[j] w_i[r] + w_i[j] v_i[r])
-  double x = a;
-#pragma unroll
-  for (int i = 0; i < NBT; ++i) {
-    if (i < k) {
-      const double svi = P[(long)i * p + j];
-      const double swi = (i == k - 1) ? wj : P[(long)(NBT + i) * p + j];
-      x -= svi * W[i] + swi * V[i];
-    }
-  }
-  if (act) xbuf[c] = x;
-  const double xs = (act && c >= 1) ? x : 0.0;
-  const int nq = 1 + 2 * NBT;
-  // the wave's 64 x nq products go to LDS as rows q of 65 (padded), and lane
-  // q sums row q (lane 0 also row 64): one LDS pass instead of nq cross-lane
-  // reductions
-  double* T = tr + (long)wave * nq * 65;
-#pragma unroll
-  for (int q = 0; q < nq; ++q) {
-    if (q == 0 || (q - 1) % NBT < k) {
-      const double f = q == 0 ? xs * xs : (q <= NBT ? V[q - 1] * xs : W[q - 1 - NBT] * xs);
-      T[q * 65 + lane] = f;
-    }
-  }
-  __syncthreads();
-  for (int q = lane; q < nq; q += 64) {
-    if (q == 0 || (q - 1) % NBT < k) {
-      const double* row = T + q * 65;
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll
-      for (int t = 0; t < 64; t += 4) {
-        s0 += row[t];
-        s1 += row[t + 1];
-        s2 += row[t + 2];
-        s3 += row[t + 3];
+    for (int i = 0; i < NI; ++i)
+      if (i0 + i == k - 1) {  // uniform over the wavefront
+        const double wn = yp - hs * V[i];
+        W[i] = wn;
+        if (act) {
+          P[(long)(NBT + k - 1) * p + r] = wn;
+          Q[(long)(k - 1) * p + r] = wn;
+        }
+        if (blockIdx.x == 0 && lane == k - 1) {
+          P[(long)(NBT + k - 1) * p + j] = sw;
+          Q[(long)(k - 1) * p + j] = sw;
+        }
       }
-      accs[wave][q] = (s0 + s1) + (s2 + s3);
-    }
   }
+  // x = A[j, r] - sum_i (v_i[j] w_i[r] + w_i[j] v_i[r]), a quarter of the columns each wavefront
+  double px = 0.0;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const double svi = read_lane(sv, i0 + i), swi = read_lane(sw, i0 + i);
+    px += svi * W[i] + swi * V[i];
+  }
+  xp[wave][lane] = px;
   __syncthreads();
-  for (int q = tid; q < nq; q += 256)
-    if (q == 0 || (q - 1) % NBT < k)
-      partA[(long)blockIdx.x * nq + q] = (accs[0][q] + accs[1][q]) + (accs[2][q] + accs[3][q]);
-  if (blockIdx.x == 0 && tid == 0) {
-    double dj = A[(long)j * ld + j];
-    for (int i = 0; i < k; ++i) {
-      const double swi = (i == k - 1) ? wj : P[(long)(NBT + i) * p + j];
-      dj -= 2.0 * P[(long)i * p + j] * swi;
-    }
-    dv[j] = dj;
+  const double x = a - ((xp[0][lane] + xp[1][lane]) + (xp[2][lane] + xp[3][lane]));
+  if (act && wave == 0) xbuf[c] = x;
+  const double xs = act && c >= 1 ? x : 0.0;
+  // this wavefront's 2 NI sums over the 64 entries: transposed in LDS, four lanes a sum
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    tr[wave][i][lane] = V[i] * xs;
+    tr[wave][NI + i][lane] = W[i] * xs;
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int q = lane & (2 * NI - 1), part = lane / (2 * NI);
+  constexpr int NP = RCHUNK * 2 * NI / 64;
+  double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+  for (int t = 0; t < NP; t += 2) {
+    s0 += tr[wave][q][part * NP + t];
+    s1 += tr[wave][q][part * NP + t + 1];
+  }
+  s0 += s1;
+  s0 += __shfl_xor(s0, 32);
+  s0 += __shfl_xor(s0, 16);
+  double* pa = partA + (long)blockIdx.x * (1 + 2 * NBT);
+  const int i = i0 + (q & (NI - 1));
+  if (part == 0 && i < k) pa[1 + (q < NI ? 0 : NBT) + i] = s0;
+  if (wave == 0) {
+    const double ss = wave_sum64(xs * xs);
+    if (lane == 0) pa[0] = ss;
+  }
+  if (wave == 3 && blockIdx.x == 0) {
+    const double dj = wave_sum64(lane < k ? 2.0 * sv * sw : 0.0);
+    if (lane == 0) dv[j] = aj - dj;
   }
 }
 
@@ -572,7 +564,13 @@ __global__ __launch_bounds__(256) void trd_panel_symv_kernel(double* __restrict_
   for (int q = tid; q < nq; q += 256) {
     double s = 0.0;
     if (q == 0 || (q - 1) % NBT < k)
-      for (int b = 0; b < nA; ++b) s += partA[(long)b * nq + q];
+      for (int b0 = 0; b0 < nA; b0 += 16) {
+        double u[16];
+#pragma unroll
+        for (int b = 0; b < 16; ++b) u[b] = partA[(long)min(b0 + b, nA - 1) * nq + q];
+#pragma unroll
+        for (int b = 0; b < 16; ++b) s += b0 + b < nA ? u[b] : 0.0;
+      }
     sums[q] = s;
   }
   __syncthreads();
@@ -810,7 +808,7 @@ __global__ __launch_bounds__(256) void trd_symv_tile_kernel(const double* __rest
 // stores v_j for its rows (below the diagonal of column j and in P, Q),
 // workgroup 0 e_j and tau_j.  Eight lanes per row, each summing every eighth
 // slot and correction term, then combined in a fixed order.
-// Grid: ceil(m / 32) workgroups; nA <= 64.
+// Grid: ceil(m / 32) workgroups; nA <= 256.
 __global__ __launch_bounds__(256) void trd_symv_reduce_kernel(double* __restrict__ A, long ld, int p, int j, int k,
                                                               double* __restrict__ P, double* __restrict__ Q,
                                                               const double* __restrict__ xbuf,
@@ -851,6 +849,13 @@ __global__ __launch_bounds__(256) void trd_symv_reduce_kernel(double* __restrict
     for (int uu = 0; uu < (2 * NBT + 3) / 4; ++uu) {
       const int q = 1 + wave + 4 * uu;
       vals[uu] = (lane < nA && q < nq && (q - 1) % NBT < k) ? partA[(long)lane * nq + q] : 0.0;
+    }
+    for (int b = 64; b < nA; b += 64) {
+#pragma unroll
+      for (int uu = 0; uu < (2 * NBT + 3) / 4; ++uu) {
+        const int q = 1 + wave + 4 * uu;
+        vals[uu] += (lane + b < nA && q < nq && (q - 1) % NBT < k) ? partA[(long)(lane + b) * nq + q] : 0.0;
+      }
     }
 #pragma unroll
     for (int uu = 0; uu < (2 * NBT + 3) / 4; ++uu) {
@@ -1974,7 +1979,6 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
     double* partB = partA + (size_t)nAmax * (2 * NBT + 1);
     double* Sy = partB + nBmax + 64;  // tile slots of the lower-triangle product
     raise_lds_limit((const void*)trd_panel_symv_kernel, (size_t)p * sizeof(double));
-    raise_lds_limit((const void*)trd_panel_row_kernel, TRD_ROW_LDS);
     // panel updates touch only the lower triangle while the next panel's
     // columns all take the lower-triangle product
     bool lower_only = P - NBT >= TRD_TILE_MIN;
@@ -1985,7 +1989,7 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
       for (int j = j0; j < j1; ++j) {
         const int k = j - j0, m = P - j - 1;
         const int nA = (m + RCHUNK - 1) / RCHUNK;
-        hipLaunchKernelGGL(trd_panel_row_kernel, dim3(nA), dim3(256), TRD_ROW_LDS, c->stream, (const double*)G, ldg, P, j, k,
+        hipLaunchKernelGGL(trd_panel_row_kernel, dim3(nA), dim3(256), 0, c->stream, (const double*)G, ldg, P, j, k,
                            Pp, Qp, (const double*)y, (const double*)partB, nBprev, (const double*)tauv, xb, partA,
                            dv);
         if (m >= TRD_TILE_MIN) {
@@ -1993,7 +1997,7 @@ void sym_eig_dc(tn_ctx* c, double* G, long p, long ldg, double* Vt, long ldv, st
           const int a0 = (j + 1) / SYT;
           const int nt = (P + SYT - 1) / SYT - a0;
           const int nB = (m + 31) / 32;  // eight lanes per row
-          TN_REQUIRE(nA <= 64 && nB <= nBmax && nt <= ntmax, TN_E_INVALID, "tridiagonalisation: tile plan");
+          TN_REQUIRE(nA <= 256 && nB <= nBmax && nt <= ntmax, TN_E_INVALID, "tridiagonalisation: tile plan");
           PhaseTimer pt(c, PH_TRD_SYMV);
           if (c->timing) c->phase_bytes[PH_TRD_SYMV] += 4.0 * (double)m * (double)(m + SYT);  // lower half of G22
           hipLaunchKernelGGL(trd_symv_tile_kernel, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(256), 0, c->stream,
