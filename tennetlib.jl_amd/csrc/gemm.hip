@@ -431,14 +431,6 @@ static long split_chunk(Prec p, const GemmDesc& g) {
   return ((g.K + P0 - 1) / P0 + 15) / 16 * 16;
 }
 
-size_t gemm_split_bytes(Prec p, const GemmDesc& g) {
-  if (g.M <= 0 || g.N <= 0) return 0;
-  const long Kc = split_chunk(p, g);
-  if (Kc == 0) return 0;
-  const long P = (g.K + Kc - 1) / Kc;
-  return (size_t)P * g.M * g.N * ((p == Prec::F64) ? 8 : 4);
-}
-
 static bool gemm_split_k(tn_ctx* c, Prec p, const GemmDesc& g) {
   const long Kc = split_chunk(p, g);
   if (Kc == 0) return false;
@@ -448,7 +440,7 @@ static bool gemm_split_k(tn_ctx* c, Prec p, const GemmDesc& g) {
   const size_t need = (size_t)P * g.M * g.N * es;
   char* part;
   if (g.split_ws) {
-    TN_REQUIRE(need <= g.split_cap, TN_E_INVALID, "gemm: split-K buffer too small");
+    if (need > g.split_cap) return false;
     part = (char*)g.split_ws;
   } else {
     part = (char*)c->workspace(WS_GEMM_SPLIT, need);

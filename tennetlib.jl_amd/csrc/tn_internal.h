@@ -238,7 +238,7 @@ struct GemmDesc {
   int batch = 1;
   double alpha = 1.0, beta = 0.0;
   // split-K partial products: a caller-owned device buffer of split_cap bytes
-  // (see gemm_split_bytes) used instead of the context workspace when set
+  // used instead of the context workspace when set (no split if it is too small)
   void* split_ws = nullptr;
   size_t split_cap = 0;
   // zpA / zpB: the rows of A (not transposed) / B (not transposed) hold finite
@@ -249,8 +249,6 @@ struct GemmDesc {
   int zpA = 0, zpB = 0;
 };
 void gemm(tn_ctx* c, Prec p, const GemmDesc& g);
-// bytes of split-K partial products gemm() needs for g (0: no split)
-size_t gemm_split_bytes(Prec p, const GemmDesc& g);
 // FP64 grouped GEMM: for every output group g < ngroups and batch z < batch,
 // C_g[z] (M x N, row stride ldc) = sum over terms t in [off[g], off[g+1]) of
 // w[t] * A_{ia[t]}[z] (M x K, lda) * B_{ib[t]}[z] (K x N, ldb), with

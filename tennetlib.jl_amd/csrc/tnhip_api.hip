@@ -1361,6 +1361,21 @@ void* scratch_address(int device) {
 
 inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
+// bytes that the scratch limit counts for the partial sums of one product: the
+// entry's contract, whatever the products use of it
+size_t noalloc_partials(Prec p, const GemmDesc& g) {
+  if (p != Prec::F64) return 0;
+  auto tiles = [&](long b) { return ((g.M + b - 1) / b) * ((g.N + b - 1) / b); };
+  const long t128 = tiles(128), t64 = tiles(64);
+  long parts;
+  if (t128 < 64 && g.K >= 4096) parts = std::min<long>(g.K / 512, 256 / t128);
+  else if (t64 < 64 && g.K >= 256) parts = std::min<long>(g.K / 64, 128 / t64);
+  else return 0;
+  if (parts < 2) return 0;
+  const long chunk = ((g.K + parts - 1) / parts + 15) / 16 * 16;
+  return (size_t)((g.K + chunk - 1) / chunk) * g.M * g.N * 8;
+}
+
 // product(sysenv, v) in FP64 with every intermediate in the fixed scratch:
 // the same GEMM / W-step / GEMM chain as matvec_mpo, no device allocation,
 // no host-device copy.  Needs position! at the current position (which builds
@@ -1402,14 +1417,14 @@ void matvec_noalloc(tn_env* e, const void* v, void* out) {
   g3.A = base + align256(t1); g3.lda = (long)w2 * chir;
   g3.B = R.buf.p; g3.ldb = chir;
   g3.C = out; g3.ldc = chir;
-  const size_t split = std::max(gemm_split_bytes(P, g1), gemm_split_bytes(P, g3));
+  const size_t split = std::max(noalloc_partials(P, g1), noalloc_partials(P, g3));
   const size_t need = align256(t1) + align256(t2) + align256(split);
   TN_REQUIRE(need <= NOALLOC_SCRATCH_BYTES, TN_E_INVALID,
              "allocation-free product needs " + std::to_string(need) + " bytes of scratch, more than the fixed " +
                  std::to_string(NOALLOC_SCRATCH_BYTES));
   if (mv_small(c, cx, op, L.buf.p, v, R.buf.p, out, w0, w2, DD, chil, chir, false)) return;
   g1.split_ws = g3.split_ws = base + align256(t1) + align256(t2);
-  g1.split_cap = g3.split_cap = split;
+  g1.split_cap = g3.split_cap = NOALLOC_SCRATCH_BYTES - align256(t1) - align256(t2);  // no split where it is too small
   gemm(c, P, g1);
   WStepDesc ws;
   ws.G = w0; ws.Gp = w2; ws.D = DD; ws.Dp = DD;
