@@ -196,7 +196,8 @@ int tn_env_get_link_qn(tn_env* env, int k, int* out, long cap, long* n);
 /* shape of the projected-operator domain at the current position:
  * dims[0..3] = (chil, d_p, d_{p+1} or 1, chir); *n = element count */
 int tn_env_phi_dims(tn_env* env, long* dims4, long* n);
-/* product(sysenv, v) at the current position and nsite; v, out on device */
+/* product(sysenv, v) at the current position and nsite; v, out on device.
+ * out may be v, except with QN conservation or penalty projectors. */
 int tn_env_matvec(tn_env* env, const void* v_dev, void* out_dev, int precision);
 /* Allocation-free FP64 product (no counterpart in the reference): the
  * product of tn_env_matvec with TN_PREC_FP64 for callers that cannot
@@ -205,7 +206,8 @@ int tn_env_matvec(tn_env* env, const void* v_dev, void* out_dev, int precision);
  * device array per GPU, so (w_l + w_r) * chil * d_p * d_{p+1} * chir elements
  * plus split-K partial sums must fit (else TN_E_INVALID).  Needs position! at
  * the current position (nsite 1 or 2) and no penalty projectors (else
- * TN_E_UNSUPPORTED).  Calls that overlap on one GPU race on that array. */
+ * TN_E_UNSUPPORTED).  out may be v.  Calls that overlap on one GPU race on
+ * that array. */
 int tn_env_matvec_noalloc(tn_env* env, const void* v_dev, void* out_dev);
 /* phi = A_pos * A_{pos+1} (update_site.jl:46) into phi_dev */
 int tn_env_contract_phi(tn_env* env, int pos, void* phi_dev);

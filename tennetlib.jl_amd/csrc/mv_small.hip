@@ -288,6 +288,11 @@ bool mv_small(tn_ctx* c, bool cplx, const SparseOp& op, const void* L, const voi
               int w2, int DD, long chil, long chir, bool timed) {
   if (!op.mat || chil > 512 || chir > 512) return false;
   const int C = cplx ? 2 : 1, cl = (int)chil, cr = (int)chir;
+  // every workgroup reads all of v while others already write out; the three
+  // launches have read v before the last one writes
+  const size_t bytes = (size_t)cl * DD * cr * C * sizeof(double);
+  const uintptr_t v0 = (uintptr_t)v, o0 = (uintptr_t)out;
+  if (v0 < o0 + bytes && o0 < v0 + bytes) return false;
   MvArgs a;
   a.L = (const double*)L;
   a.v = (const double*)v;

@@ -336,7 +336,8 @@ struct WStepDesc {
 };
 // H psi in FP64 (complex128 when cplx) in one launch (mv_small.hip): L[(w0
 // a'), a], psi[a, S, b], op, R[(w2 b), b'] to out[a', S', b'].  false (nothing
-// queued) for sizes that its workgroups do not take; timed: as PH_MV_GEMM.
+// queued) for sizes that its workgroups do not take and for v and out that
+// overlap; timed: as PH_MV_GEMM.
 bool mv_small(tn_ctx* c, bool cplx, const SparseOp& op, const void* L, const void* v, const void* R, void* out, int w0,
               int w2, int DD, long chil, long chir, bool timed);
 void wstep(tn_ctx* c, bool fp32, const WStepDesc& w);

@@ -69,3 +69,39 @@ def test_one_launch_product(T, size, cplx, fill):
     assert np.array_equal(T.product(env, psi).reshape(-1), got.reshape(-1))
     dv.free()
     out.free()
+
+
+@pytest.mark.parametrize("chi", [16, 64])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_product_in_place(T, chi, cplx, noalloc):
+    """out == v, and out overlapping the end of v: the separate product's
+    result.  chi = 16 takes one launch with separate vectors, 64 three.  Other
+    kernels sum in another order: eps per term of the sums as above, on
+    vectors of norm |psi| |H|."""
+    rng = np.random.default_rng(chi + cplx)
+
+    def draw(*shape):
+        x = rng.standard_normal(shape)
+        return x + 1j * rng.standard_normal(shape) if cplx else x
+
+    cd = [1, 2, chi, 4, chi, 2, 1]
+    A = [draw(cd[k], 2, cd[k + 1]) / np.sqrt(cd[k] * cd[k + 1]) for k in range(6)]
+    env = T.StateEnvs(A, O.heisenberg_mpo(6))
+    T.position_(env, 3)
+    dims, n = env.phi_dims()
+    psi = draw(*dims).reshape(-1)
+    want = T.product(env, psi.reshape(dims)).reshape(-1)
+    tol = 3 * 5 * chi * 2.0 ** -53 * np.linalg.norm(np.abs(want)) * (2 if cplx else 1)
+    item = np.dtype(env.dtype).itemsize
+    for shift in (0, n - 3):
+        buf = T.DeviceArray.from_numpy(env.ctx, np.concatenate([psi, np.zeros_like(psi)]).astype(env.dtype))
+        v, out = buf.ptr.value, buf.ptr.value + shift * item
+        print("in place", chi, cplx, noalloc, shift, flush=True)
+        if noalloc:
+            env.ctx.check(env.ctx.lib.tn_env_matvec_noalloc(env.h, v, out))
+        else:
+            env.ctx.check(env.ctx.lib.tn_env_matvec(env.h, v, out, 0))
+        got = buf.numpy()[shift:shift + n]
+        buf.free()
+        assert np.linalg.norm(got - want) <= tol
