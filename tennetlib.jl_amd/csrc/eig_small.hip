@@ -283,6 +283,13 @@ __global__ __launch_bounds__(GR* GC) void trd_reg_kernel(SmallEig one, const Sma
 // ---------------------------------------------------------------------------
 typedef double d4 __attribute__((ext_vector_type(4)));
 
+// Least deflation tolerance of a matrix scaled to entries of one: far below its
+// rounding.  Kept columns then have rho |z| and pole distances above 2^-400 and
+// (|z| being above rounding) rho z^2 above 2^-510, all with a normal square.
+// Without it a block of entries near 2^-1030 has the tolerance zero and rcp2
+// gets a denormal: NaN.
+constexpr double TINY = 0x1p-400;
+
 template <int NM>
 constexpr size_t dc_small_lds() {
   return ((size_t)NM * (NM + 1) + 12 * NM) * sizeof(double) + (size_t)9 * NM * sizeof(int);
@@ -497,7 +504,8 @@ __global__ __launch_bounds__(4 * NM) void dc_small_kernel(SmallEig one, const Sm
   auto bnd = [&](int i) { return (i * n) >> L; };
   auto leaf_of = [&](int t) { return (((t + 1) << L) - 1) / n; };
   for (int i = tid; i < n * LD; i += NT) Q[i] = 0.0;
-  // scaled by a power of two to entries of at most one: nothing below leaves the normal range
+  // scaled by a power of two to entries of at most one; couplings below TINY
+  // are deflated, so the products and reciprocals of what is left stay normal
   double big = 0.0;
   const double tl = (S.flags & SE_TEAR_L) ? e[-1] : 0.0, tr = (S.flags & SE_TEAR_R) ? e[n - 1] : 0.0;
   auto diag = [&](int t) { return d[t] - (t == 0 ? tl : 0.0) - (t == n - 1 ? tr : 0.0); };
@@ -581,7 +589,7 @@ __global__ __launch_bounds__(4 * NM) void dc_small_kernel(SmallEig one, const Sm
         dm = fmax(dm, __shfl_xor(dm, o, 64));
         zm = fmax(zm, __shfl_xor(zm, o, 64));
       }
-      tol = 8.0 * EPS * fmax(dm, rho * zm);
+      tol = fmax(8.0 * EPS * fmax(dm, rho * zm), TINY);
       if (sub == 0) {
         perm[a + cnt] = t;
         tau[a + cnt] = mine;

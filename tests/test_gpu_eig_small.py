@@ -91,3 +91,31 @@ def test_factorisation_extreme_scales(T):
         a, b, w = factorise(T, np.ldexp(phi, e), True)
         assert np.abs(np.ldexp(w, -2 * e) - ref[2]).max() <= 40 * EPS
         assert np.abs(a.reshape(40, -1) @ b.reshape(-1, 40) - phi.reshape(40, 40)).max() <= 40 * EPS
+
+
+@pytest.mark.parametrize("chi", [2, 3, 10, 50])
+@pytest.mark.parametrize("cplx", [False])
+@pytest.mark.parametrize("e", [-515, -400])
+@pytest.mark.parametrize("tiny_first", [False, True])
+def test_factorisation_of_blocks_of_unlike_scale(T, chi, cplx, e, tiny_first):
+    """A dense block of the density matrix at 2^(2e) beside one at one (its
+    entries or their products below the normal range): the factors of the block
+    at one to its rounding, and all vectors orthonormal."""
+    rng = np.random.default_rng(chi)
+    p = 2 * chi
+    M = np.zeros((p, p), np.complex128 if cplx else np.float64)
+    for rows, scale in ((slice(0, chi), 0 if not tiny_first else e), (slice(chi, p), e if not tiny_first else 0)):
+        b = rng.standard_normal((chi, chi))
+        if cplx:
+            b = b + 1j * rng.standard_normal((chi, chi))
+        M[rows, rows] = b / np.linalg.norm(b) * 2.0 ** scale
+    print("unlike", chi, cplx, e, tiny_first, flush=True)
+    for left in (True, False):
+        a, b, w = factorise(T, np.ascontiguousarray(M.reshape(chi, 2, 2, chi)), left)
+        k = len(w)
+        want = np.sort(np.linalg.svd(M, compute_uv=False) ** 2)[::-1][:k]
+        assert np.abs(np.sort(w)[::-1] - want).max() <= 40 * EPS
+        A, B = a.reshape(p, k), b.reshape(k, p)
+        assert np.abs(A @ B - M).max() <= 40 * EPS
+        Q = A if left else B.conj().T
+        assert np.abs(Q.conj().T @ Q - np.eye(k)).max() <= 60 * EPS
