@@ -14,6 +14,11 @@ namespace tn {
 namespace {
 
 constexpr double EPS = 2.220446049250313e-16;
+// A column whose entries below the subdiagonal are under 2^-450 of the block's
+// largest entry (one, after scaling) is left as it is: dropping them is far
+// below its rounding, and a reflector from squares that lost bits would not be
+// orthogonal.
+constexpr double TINY_SS = 0x1p-900;
 
 __device__ __forceinline__ const SmallEig& pick(const SmallEig& one, const SmallEig* list, unsigned b) {
   return list ? list[b] : one;
@@ -34,12 +39,13 @@ template <> struct El<false> {
   static __device__ __forceinline__ T scale(T a, double s) { return a * s; }
   static __device__ __forceinline__ double norm2(T a) { return a * a; }
   static __device__ __forceinline__ double re(T a) { return a; }
+  static __device__ __forceinline__ int high_word(T a) { return __double2hiint(a) & 0x7fffffff; }
   static __device__ __forceinline__ bool is_zero(T a) { return a == 0.0; }
   static __device__ __forceinline__ T sel(bool f, T a, T b) { return f ? a : b; }
   template <class F> static __device__ __forceinline__ T each(T a, F f) { return f(a); }
   // reflector H = I - tau v v^T of x (x_0, sum of squares ss of the rest): H x = beta e_1
   static __device__ __forceinline__ void reflector(T x0, double ss, T& tau, double& beta, T& sc) {
-    trd_reflector(x0, ss, tau, beta, sc);
+    trd_reflector(x0, ss < TINY_SS ? 0.0 : ss, tau, beta, sc);
   }
 };
 template <> struct El<true> {
@@ -61,12 +67,15 @@ template <> struct El<true> {
   static __device__ __forceinline__ T scale(T a, double s) { return make_double2(a.x * s, a.y * s); }
   static __device__ __forceinline__ double norm2(T a) { return a.x * a.x + a.y * a.y; }
   static __device__ __forceinline__ double re(T a) { return a.x; }
+  static __device__ __forceinline__ int high_word(T a) {
+    return max(__double2hiint(a.x) & 0x7fffffff, __double2hiint(a.y) & 0x7fffffff);
+  }
   static __device__ __forceinline__ bool is_zero(T a) { return a.x == 0.0 && a.y == 0.0; }
   static __device__ __forceinline__ T sel(bool f, T a, T b) { return make_double2(f ? a.x : b.x, f ? a.y : b.y); }
   template <class F> static __device__ __forceinline__ T each(T a, F f) { return make_double2(f(a.x), f(a.y)); }
   // the zlarfg convention: beta real
   static __device__ __forceinline__ void reflector(T x0, double ss, T& tau, double& beta, T& sc) {
-    if (ss == 0.0 && x0.y == 0.0) {
+    if (ss + x0.y * x0.y < TINY_SS) {
       tau = sc = zero();
       beta = x0.x;
       return;
@@ -131,6 +140,25 @@ __global__ __launch_bounds__(GR* GC) void trd_reg_kernel(SmallEig one, const Sma
       const int r = tr + GR * i, c = tc + GC * j;
       a[i][j] = (r < n && c < n) ? A[(long)r * S.lda + c] : E::zero();
     }
+  // scaled by a power of two to a largest entry in [1/2, 1), so that no sum of
+  // squares leaves the range (exponents: the high words of the absolute values)
+  int hw = 0;
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) hw = max(hw, E::high_word(a[i][j]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) hw = max(hw, __shfl_xor(hw, o, 64));
+  int* hws = reinterpret_cast<int*>(part);
+  if (lane == 0) hws[tid >> 6] = hw;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NT / 64; ++k) hw = max(hw, hws[k]);
+  const int ex = __builtin_amdgcn_readfirstlane((hw >> 20) < 2047 ? (hw >> 20) - 1022 : 0);
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) a[i][j] = E::each(a[i][j], [ex](double x) { return ldexp(x, -ex); });
   // column j, held in column chunk J0 or (J2 > J0 + 1) J0 + 1, to LDS; its diagonal element to ds
   auto publish = [&](int j, auto J0, auto J2) {
     constexpr int C0 = decltype(J0)::value, C1 = decltype(J2)::value - 1;
@@ -259,9 +287,9 @@ __global__ __launch_bounds__(GR* GC) void trd_reg_kernel(SmallEig one, const Sma
     }
   T* tauv = reinterpret_cast<T*>(taubase) + S.de;
   for (int t = tid; t < n; t += NT) {
-    dbase[S.de + t] = ds[t];
+    dbase[S.de + t] = ldexp(ds[t], ex);
     tauv[t] = t < n - 1 ? ts[t] : E::zero();
-    if (t < n - 1) ebase[S.de + t] = es[t];
+    if (t < n - 1) ebase[S.de + t] = ldexp(es[t], ex);
   }
 }
 

@@ -80,9 +80,10 @@ def test_factorisation_at_eigensolver_size_classes(T, kind, cplx, chi):
 
 def test_factorisation_extreme_scales(T):
     """A tensor scaled by a large power of two has the same factors and weights
-    scaled exactly: the divide and conquer works on scaled entries.  The
-    density matrix's entries scale by 2^(2e) and the reflectors sum their
-    squares, so 4 |e| has to stay below 1022 less the 2^-40 of the entries."""
+    scaled exactly: the reduction and the divide and conquer of up to 128 rows
+    work on scaled entries (the exponents of larger ones, whose column kernels
+    sum squares of the density matrix: 4 |e| below 1022 less the 40 bits of its
+    entries; those of small ones are below)."""
     rng = np.random.default_rng(3)
     phi = rng.standard_normal((20, 2, 2, 20))
     phi /= np.linalg.norm(phi)
@@ -94,8 +95,8 @@ def test_factorisation_extreme_scales(T):
 
 
 @pytest.mark.parametrize("chi", [2, 3, 10, 50])
-@pytest.mark.parametrize("cplx", [False])
-@pytest.mark.parametrize("e", [-515, -400])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("e", [-515, -400, -270, -267, -262])
 @pytest.mark.parametrize("tiny_first", [False, True])
 def test_factorisation_of_blocks_of_unlike_scale(T, chi, cplx, e, tiny_first):
     """A dense block of the density matrix at 2^(2e) beside one at one (its
@@ -119,3 +120,26 @@ def test_factorisation_of_blocks_of_unlike_scale(T, chi, cplx, e, tiny_first):
         assert np.abs(A @ B - M).max() <= 40 * EPS
         Q = A if left else B.conj().T
         assert np.abs(Q.conj().T @ Q - np.eye(k)).max() <= 60 * EPS
+
+
+@pytest.mark.parametrize("chi,cplx", [(1, False), (2, False), (4, False), (7, True), (20, False), (50, True),
+                                      (64, True), (64, False)])
+@pytest.mark.parametrize("e", [-480, -400, 400, 500])
+def test_small_factorisation_scales_exactly(T, chi, cplx, e):
+    """Factorisations of up to 128 rows (one workgroup a stage) of a
+    unit tensor times 2^e: the same factors (the new sites are normalised), the
+    weights times 2^(2e), which stay normal numbers while their squares do not."""
+    rng = np.random.default_rng(chi)
+    phi = rng.standard_normal((chi, 2, 2, chi))
+    if cplx:
+        phi = phi + 1j * rng.standard_normal((chi, 2, 2, chi))
+    phi /= np.linalg.norm(phi)
+    ref = factorise(T, phi, True)
+    print("scaled", chi, cplx, e, flush=True)
+    a, b, w = factorise(T, phi * 2.0 ** e, True)
+    p = 2 * chi
+    # entries of the density matrix under 2^-1022 keep an absolute error of 2^-1075
+    assert np.abs(np.ldexp(w, -2 * e) - ref[2]).max() <= 40 * EPS
+    A, B = a.reshape(p, -1), b.reshape(-1, p)
+    assert np.abs(A @ B - phi.reshape(p, p)).max() <= 40 * EPS
+    assert np.abs(A.conj().T @ A - np.eye(A.shape[1])).max() <= 60 * EPS

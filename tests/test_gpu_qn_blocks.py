@@ -48,6 +48,18 @@ CASES = {
 @pytest.mark.parametrize("case", CASES)
 @pytest.mark.parametrize("ortho", ["left", "right"])
 def test_sector_sizes(T, case, ortho):
+    run_case(T, case, ortho)
+
+
+@pytest.mark.parametrize("ortho", ["left", "right"])
+@pytest.mark.parametrize("e", [-400, 400])
+def test_sector_scales(T, ortho, e):
+    """The unit tensor times 2^e: the same vectors (the new sites are
+    normalised), the weights times 2^(2e)."""
+    run_case(T, "small", ortho, e)
+
+
+def run_case(T, case, ortho, e=0):
     sectors, chir = CASES[case]
     sizes = left_sizes(sectors)
     qs = Q.spin_half_qns()
@@ -74,14 +86,14 @@ def test_sector_sizes(T, case, ortho):
     ctx.check(ctx.lib.tn_env_set_qn(env.h, 1, sq.ctypes.data_as(pi), lq.ctypes.data_as(pi)))
     env.nq = 1
     Ab, Ab1, newq, spec = Q.block_factorize(phi, ql, qs, qs, qr, 10 ** 6, 1, 1e-13, ortho)
-    dphi = T.DeviceArray.from_numpy(ctx, phi)
+    dphi = T.DeviceArray.from_numpy(ctx, phi * 2.0 ** e)
     terr, nk = C.c_double(), C.c_long()
     eigs = (C.c_double * 8192)()
-    print("qn blocks", case, ortho, flush=True)
+    print("qn blocks", case, ortho, e, flush=True)
     ctx.check(ctx.lib.tn_replacebond(env.h, b, dphi.ptr, 1 if ortho == "left" else 0, 10 ** 6, 1, 1e-13, 0.0, 1,
                                      C.byref(terr), eigs, 8192, C.byref(nk)))
     assert nk.value == len(newq)
-    assert np.abs(np.array(eigs[:nk.value]) - spec.eigs).max() < 1e-13
+    assert np.abs(np.ldexp(np.array(eigs[:nk.value]), -2 * e) - spec.eigs).max() < 1e-13
     assert env.sectors(b) == spec.sectors
     got = [env.get_site(b), env.get_site(b + 1)]
     U = got[0].reshape(-1, nk.value) if ortho == "left" else got[1].reshape(nk.value, -1).T
