@@ -248,7 +248,17 @@ __global__ __launch_bounds__(MV_THREADS) void mv_small_kernel(MvArgs g) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = t.m0 + kg + 4 * r;
-      if (row < M2 && t.c0 + ln < N2) T2[t.x + roff[row]] = acc[0][r];
+      if (row < M2 && t.c0 + ln < N2) {
+        double x = acc[0][r];
+        if (x - x != 0.0) {  // Inf or NaN: only the operator's entries may meet it, not its zeros
+          x = 0.0;
+          for (int k = 0; k < K2; ++k) {
+            const double o = mv_ld<double>(op, (unsigned)(row * K2 + k) * 8u);
+            if (o != 0.0) x = fma(o, T1[t.ob + koff[k]], x);
+          }
+        }
+        T2[t.x + roff[row]] = x;
+      }
     }
   }, ga2, gb2);
   __syncthreads();

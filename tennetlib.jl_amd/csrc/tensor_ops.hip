@@ -119,7 +119,9 @@ __global__ __launch_bounds__(256) void wstep_vec_kernel(int G, int Gp, int D, in
 // K steps on their way while five are multiplied) and the results straight
 // out.  All output rows of a strip are accumulated at once (NMB blocks of 32
 // rows, v_mfma_f32_32x32x2f32, or 16, v_mfma_f64_16x16x4f64).  A sparse
-// operator costs its full M x K here and still stays under the HBM time.
+// operator costs its full M x K here and still stays under the HBM time; strips
+// with a result that is not finite are done again entry by entry, so that its
+// zeros do not spread an Inf or NaN (the check costs nothing measurable).
 // K runs from the operator's last column to its first.  In place of a
 // workgroup per 128 columns that staged operator and input in LDS, with the
 // w = 20 pair operator: FP32 to bf16 pairs at chi = 2048 2.46 -> 0.85 ms
@@ -214,35 +216,57 @@ __global__ __launch_bounds__(256, 2) void wstep_mfma_kernel(WmArgs<T> w) {
 #pragma unroll
       for (int p = 0; p < WM_PF; ++p) cur[p] = nxt[p];
     }
-    // register r of a lane: f64 row lane / 16 + 4 r; f32 row 8 (r / 4) + 4 (lane / 32) + r % 4
     const long obase = Ai * w.out_sA;
+    auto put = [&](int row, T x0, T x1) {
+      if (row >= w.M) return;
+      const long off = ooff[row] + obase;
+      if constexpr (SPLIT) {
+        const unsigned short h0 = f2bf_rne(x0), h1 = f2bf_rne(x1);
+        const unsigned short l0 = f2bf_rne(x0 - __uint_as_float(((unsigned int)h0) << 16));
+        const unsigned short l1 = f2bf_rne(x1 - __uint_as_float(((unsigned int)h1) << 16));
+        if constexpr (VEC) {
+          if (c0 < w.nB) {
+            *reinterpret_cast<unsigned int*>(w.ohi + off + c0) = (unsigned int)h0 | ((unsigned int)h1 << 16);
+            *reinterpret_cast<unsigned int*>(w.olo + off + c0) = (unsigned int)l0 | ((unsigned int)l1 << 16);
+          }
+        } else {
+          if (c0 < w.nB) { w.ohi[off + c0] = h0; w.olo[off + c0] = l0; }
+          if (c1 < w.nB) { w.ohi[off + c1] = h1; w.olo[off + c1] = l1; }
+        }
+      } else if constexpr (VEC) {
+        if (c0 < w.nB) *reinterpret_cast<vec2*>(w.out + off + c0) = vec2{x0, x1};
+      } else {
+        if (c0 < w.nB) w.out[off + c0] = x0;
+        if (c1 < w.nB) w.out[off + c1] = x1;
+      }
+    };
+    T fin = T(0);  // NaN if any result is not finite
 #pragma unroll
     for (int i = 0; i < NMB; ++i)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const int row = i * MB + (F64 ? kg + 4 * r : 8 * (r >> 2) + 4 * kg + (r & 3));
-        const long off = ooff[row] + obase;
-        const T x0 = acc[i][0][r], x1 = acc[i][1][r];
-        if constexpr (SPLIT) {
-          const unsigned short h0 = f2bf_rne(x0), h1 = f2bf_rne(x1);
-          const unsigned short l0 = f2bf_rne(x0 - __uint_as_float(((unsigned int)h0) << 16));
-          const unsigned short l1 = f2bf_rne(x1 - __uint_as_float(((unsigned int)h1) << 16));
-          if constexpr (VEC) {
-            if (row < w.M && c0 < w.nB) {
-              *reinterpret_cast<unsigned int*>(w.ohi + off + c0) = (unsigned int)h0 | ((unsigned int)h1 << 16);
-              *reinterpret_cast<unsigned int*>(w.olo + off + c0) = (unsigned int)l0 | ((unsigned int)l1 << 16);
-            }
-          } else {
-            if (row < w.M && c0 < w.nB) { w.ohi[off + c0] = h0; w.olo[off + c0] = l0; }
-            if (row < w.M && c1 < w.nB) { w.ohi[off + c1] = h1; w.olo[off + c1] = l1; }
+      for (int r = 0; r < NR; ++r) fin += (acc[i][0][r] - acc[i][0][r]) + (acc[i][1][r] - acc[i][1][r]);
+    if (__any(fin != T(0))) {
+      // only the operator's entries may meet an Inf or NaN, not its zeros: the strip again, entry by entry
+      for (int m = kg; m < w.M; m += 64 / MB) {
+        T x0 = T(0), x1 = T(0);
+        for (int i = w.Kp - w.K; i < w.Kp; ++i) {
+          const T o = Aop[m * lda + i];
+          if (o != T(0)) {
+            const vec2 v = load(s, ioff[i]);
+            x0 = fma(o, v[0], x0);
+            x1 = fma(o, v[1], x1);
           }
-        } else if constexpr (VEC) {
-          if (row < w.M && c0 < w.nB) *reinterpret_cast<vec2*>(w.out + off + c0) = vec2{x0, x1};
-        } else {
-          if (row < w.M && c0 < w.nB) w.out[off + c0] = x0;
-          if (row < w.M && c1 < w.nB) w.out[off + c1] = x1;
         }
+        put(m, x0, x1);
       }
+      continue;
+    }
+    // register r of a lane: f64 row lane / 16 + 4 r; f32 row 8 (r / 4) + 4 (lane / 32) + r % 4
+#pragma unroll
+    for (int i = 0; i < NMB; ++i)
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        put(i * MB + (F64 ? kg + 4 * r : 8 * (r >> 2) + 4 * kg + (r & 3)), acc[i][0][r], acc[i][1][r]);
   }
 }
 

@@ -65,3 +65,35 @@ def test_operator_step(T, size, fill):
         got = T.product(env, psi, precision=prec).reshape(want.shape)
         err = np.linalg.norm(got - want)
         assert err <= tol * scale, (prec, err / max(scale, 1e-300))
+
+
+@pytest.mark.parametrize("chi", [8, 15, 64, 65])
+@pytest.mark.parametrize("cplx,prec", [(False, "fp64"), (False, "fp32"), (False, "bf16x3"), (True, "fp64"),
+                                       (True, "fp32")])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_operator_zeros_leave_non_finite_values_out(T, chi, cplx, prec, value):
+    """An Inf or NaN in psi at the spins (up, up) reaches only the rows that the
+    operator couples to them: a Heisenberg bond does not flip both spins, so
+    the rows (down, down) are those of psi with a zero in its place.  One launch
+    (chi = 8, 15 in FP64) and three, even and odd column counts.  Tolerance as
+    for the products above: other sums, of at most 5 chi terms."""
+    rng = np.random.default_rng(chi + cplx)
+
+    def draw(*shape):
+        x = rng.standard_normal(shape)
+        return x + 1j * rng.standard_normal(shape) if cplx else x
+
+    cd = [1, 2, chi, 4, chi, 2, 1]
+    A = [draw(cd[k], 2, cd[k + 1]) / np.sqrt(cd[k] * cd[k + 1]) for k in range(6)]
+    env = T.StateEnvs(A, O.heisenberg_mpo(6))
+    T.position_(env, 3)
+    dims, _ = env.phi_dims()
+    psi = draw(*dims)
+    psi[chi // 2, 0, 0, chi // 3] = 0.0
+    want = T.product(env, psi, precision=prec).reshape(dims)[:, 1, 1]
+    psi[chi // 2, 0, 0, chi // 3] = value
+    print("zeros", chi, cplx, prec, value, flush=True)
+    got = T.product(env, psi, precision=prec).reshape(dims)
+    assert not np.isfinite(got[:, 0, 0]).any()
+    eps = 2.0 ** -53 if prec == "fp64" else 2.0 ** -24
+    assert np.linalg.norm(got[:, 1, 1] - want) <= 15 * chi * eps * np.linalg.norm(want)
