@@ -15,8 +15,8 @@
 //    hi/lo pairs (k contiguous, pre-split by split_bf16_*).  Each 32x32x16
 //    step issues lo*hi + hi*lo + hi*hi with FP32 accumulation.
 // Operands whose rows are 16-byte aligned with whole vectors take vector
-// loads, others element loads; any size and stride whose tile extents fit a
-// 32-bit byte offset runs here, the rest in gemm.hip.
+// loads, others element loads, both with 32-bit offsets into the tile; row
+// strides past those take element loads from 64-bit addresses.
 #include <map>
 #include <mutex>
 
@@ -115,6 +115,34 @@ __device__ __forceinline__ uint4 ldvec(Rsrc r, int rr, long c, long ld, long col
   }
 }
 
+// the same VN elements through 64-bit addresses: rows [0, rows) of the tile,
+// columns [0, cols), both at least one; loads without branches, from the last
+// valid element past the ends
+template <typename T>
+__device__ __forceinline__ uint4 ldvec_far(const T* base, int rr, long rows, long c, long ld, long cols) {
+  constexpr int VN = 16 / (int)sizeof(T);
+  struct alignas(16) V { T e[VN]; } v;
+  const T* p = base + min((long)rr, rows - 1) * ld;
+#pragma unroll
+  for (int q = 0; q < VN; ++q) v.e[q] = p[min(c + q, cols - 1)];
+  uint4 u = __builtin_bit_cast(uint4, v);
+  constexpr int D = (int)sizeof(T) / 4;  // words an element
+#pragma unroll
+  for (int q = 0; q < VN; ++q) {
+    const bool in = rr < rows && c + q < cols;
+    unsigned* w = &u.x + q * D;
+#pragma unroll
+    for (int i = 0; i < D; ++i) w[i] = in ? w[i] : 0u;
+  }
+  return u;
+}
+
+// how a kernel loads its operands: LOAD_ELEM and LOAD_VEC as in ldvec, LOAD_FAR
+// as in ldvec_far.  Factorisation of 200 rows of 2.1 10^6 numbers with LOAD_FAR
+// 15.5 ms, of 1.05 10^6 complex ones 93 ms (kernels of their own for such rows:
+// 16.2 to 17.2 and 207 ms); with branches around each load 13.3 and 165 ms.
+constexpr int LOAD_ELEM = 0, LOAD_VEC = 1, LOAD_FAR = 2;
+
 // ---------------------------------------------------------------------------
 // bf16 hi/lo split: hi = rne(x), lo = rne(x - hi); from FP64 or FP32 sources
 // ---------------------------------------------------------------------------
@@ -195,19 +223,26 @@ __device__ __forceinline__ void tile_product(Seg& seg, long M, long N, long m0, 
     constexpr int Q = decltype(slot)::value;
     const T* A = reinterpret_cast<const T*>(seg.A);
     const T* B = reinterpret_cast<const T*>(seg.B);
-    const Rsrc ar = TA ? tile_rsrc(A, k0, seg.K, BK, lda, seg.wA, ES) : tile_rsrc(A, m0, M, BM, lda, seg.wA, ES);
-    const Rsrc br = TB ? tile_rsrc(B, n0, N, BN, ldb, seg.wB, ES) : tile_rsrc(B, k0, seg.K, BK, ldb, seg.wB, ES);
+    const long ra0 = TA ? k0 : m0, na = TA ? seg.K : M, rb0 = TB ? n0 : k0, nb = TB ? N : seg.K;  // first row, rows
+    const Rsrc ar = tile_rsrc(A, ra0, na, TA ? BK : BM, lda, seg.wA, ES);
+    const Rsrc br = tile_rsrc(B, rb0, nb, TB ? BN : BK, ldb, seg.wB, ES);
 #pragma unroll
     for (int i = 0; i < CF::A_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::A_COLS / VN), cc = (idx % (CF::A_COLS / VN)) * VN;
-      ra[Q][i] = ldvec<T, AL>(ar, rr, (TA ? m0 : k0) + cc, lda, seg.wA);
+      if constexpr (AL == LOAD_FAR)
+        ra[Q][i] = ldvec_far<T>(A + ra0 * lda, rr, na - ra0, (TA ? m0 : k0) + cc, lda, seg.wA);
+      else
+        ra[Q][i] = ldvec<T, AL>(ar, rr, (TA ? m0 : k0) + cc, lda, seg.wA);
     }
 #pragma unroll
     for (int i = 0; i < CF::B_VECS; ++i) {
       const int idx = tid + i * 256;
       const int rr = idx / (CF::B_COLS / VN), cc = (idx % (CF::B_COLS / VN)) * VN;
-      rb[Q][i] = ldvec<T, AL>(br, rr, (TB ? k0 : n0) + cc, ldb, seg.wB);
+      if constexpr (AL == LOAD_FAR)
+        rb[Q][i] = ldvec_far<T>(B + rb0 * ldb, rr, nb - rb0, (TB ? k0 : n0) + cc, ldb, seg.wB);
+      else
+        rb[Q][i] = ldvec<T, AL>(br, rr, (TB ? k0 : n0) + cc, ldb, seg.wB);
     }
     if constexpr (SCALE) w[Q] = seg.w;
     k0 += BK;
@@ -563,7 +598,7 @@ struct BlockSeg {
   }
 };
 
-template <typename T, int TB, bool SPLIT>
+template <typename T, int TB, bool SPLIT, int AL>
 __global__ __launch_bounds__(256, 2) void gemm_bs_kernel(BsDesc d) {
   using CF = TileCfg<T, 0, TB, BS_TILE, SPLIT ? 16 : tile_bk<T>(BS_TILE)>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -575,7 +610,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bs_kernel(BsDesc d) {
   seg.set();
   typename Acc<T>::type acc[CF::F][CF::F];
   tile_zero<CF, T>(acc);
-  tile_product<CF, T, 0, TB, 0, false, SPLIT>(seg, tk.M, tk.N, tl.y, tl.z, d.lda, d.ldb, 0, 0,
+  tile_product<CF, T, 0, TB, AL, false, SPLIT>(seg, tk.M, tk.N, tl.y, tl.z, d.lda, d.ldb, 0, 0,
                                               reinterpret_cast<T*>(smem), acc);
   tile_store<CF, T>(reinterpret_cast<T*>(d.C) + tk.c_off, d.ldc, tk.M, tk.N, tl.y, tl.z, d.alpha, 0.0, acc);
 }
@@ -797,16 +832,14 @@ static bool fast_aligned(Prec p, const GemmDesc& g) {
   return al(g.A, g.lda, g.sA, width_a(p, g)) && al(g.B, g.ldb, g.sB, width_b(p, g));
 }
 
-// a tile of up to 128 rows must span less than 2^31 bytes (32-bit buffer offsets)
-static bool extent_ok(long ld, long rows, size_t es) {
-  return (size_t)ld * es * (size_t)(std::min(rows, 130L) + 1) < ((size_t)1 << 31);
-}
-
-bool gemm_fast_ok(Prec p, const GemmDesc& g) {
-  if (p != Prec::F64 && p != Prec::F32 && p != Prec::Z64) return false;
-  if (p == Prec::Z64 && ((uintptr_t)g.A % 16 != 0 || (uintptr_t)g.B % 16 != 0)) return false;
-  const size_t es = elem_bytes(p);
-  return extent_ok(g.lda, g.tA ? g.K : g.M, es) && extent_ok(g.ldb, g.tB ? g.N : g.K, es);
+// Operands whose tiles have 32-bit offsets: the rows that a tile holds span less
+// than 2^31 bytes, and the offsets that the kernel forms for all rows of the
+// tile stay below 2^32, so that those past the operand's end are past its
+// extent and do not wrap into it.
+static bool extent_ok(long ld, long rows, long tile_rows, size_t es) {
+  const size_t row = (size_t)ld * es;
+  return row * (size_t)(std::min(rows, tile_rows) + 1) < ((size_t)1 << 31) &&
+         row * (size_t)(tile_rows + 1) < ((size_t)1 << 32);
 }
 
 // Tile of an M x N product over a batch: the one with the least work on the
@@ -842,7 +875,7 @@ void launch_tile(tn_ctx* c, const FArgs& a, int batch) {
 }
 template <typename T, int TA, int TB, int AL>
 void launch_bm(tn_ctx* c, const FArgs& a, int batch, int bm) {
-  if constexpr (sizeof(T) != 16)
+  if constexpr (sizeof(T) != 16 && AL != LOAD_FAR)
     if (bm == 128) return launch_tile<T, TA, TB, AL, 128>(c, a, batch);
   if constexpr (sizeof(T) != 4)
     if (bm == 32) return launch_tile<T, TA, TB, AL, 32>(c, a, batch);
@@ -857,31 +890,42 @@ void launch_ops(tn_ctx* c, const FArgs& a, const GemmDesc& g, int bm) {
 }
 }  // namespace
 
-void gemm_fast(tn_ctx* c, Prec p, const GemmDesc& g) {
+void gemm_tiles(tn_ctx* c, Prec p, const GemmDesc& g) {
+  TN_REQUIRE(p != Prec::BF16X3, TN_E_INVALID, "gemm: BF16x3 operands come pre-split (gemm_bf16x3_nt)");
+  const size_t es = elem_bytes(p);
+  const bool far = !extent_ok(g.lda, g.tA ? g.K : g.M, 128, es) || !extent_ok(g.ldb, g.tB ? g.N : g.K, 128, es) ||
+                   (p == Prec::Z64 && ((uintptr_t)g.A % 16 != 0 || (uintptr_t)g.B % 16 != 0));
+  const bool aligned = !far && fast_aligned(p, g);
   FArgs a;
   a.M = g.M; a.N = g.N; a.K = g.K;
-  const bool aligned = fast_aligned(p, g);
   a.A = g.A; a.lda = g.lda; a.sA = g.sA; a.cA = g.cA;
   a.B = g.B; a.ldb = g.ldb; a.sB = g.sB; a.cB = g.cB;
-  // the vector kernel reads the padded widths; the element kernel the valid ones
+  // the vector kernel reads the padded widths; the element kernels the valid ones
   a.wA = aligned ? width_a(p, g) : (g.tA ? g.M : g.K);
   a.wB = aligned ? width_b(p, g) : (g.tB ? g.K : g.N);
   a.C = g.C; a.ldc = g.ldc; a.sC = g.sC;
   a.alpha = g.alpha; a.beta = g.beta;
   const int bm = pick_tile(p, g.M, g.N, g.batch);
-  if (p == Prec::Z64) launch_ops<double2, 1>(c, a, g, bm);
-  else if (p == Prec::F64 && aligned) launch_ops<double, 1>(c, a, g, bm);
-  else if (p == Prec::F64) launch_ops<double, 0>(c, a, g, bm);
-  else if (aligned) launch_ops<float, 1>(c, a, g, bm);
-  else launch_ops<float, 0>(c, a, g, bm);
+  if (p == Prec::Z64) {
+    if (far) launch_ops<double2, LOAD_FAR>(c, a, g, bm);
+    else launch_ops<double2, LOAD_VEC>(c, a, g, bm);
+  } else if (p == Prec::F64) {
+    if (far) launch_ops<double, LOAD_FAR>(c, a, g, bm);
+    else if (aligned) launch_ops<double, LOAD_VEC>(c, a, g, bm);
+    else launch_ops<double, LOAD_ELEM>(c, a, g, bm);
+  } else {
+    if (far) launch_ops<float, LOAD_FAR>(c, a, g, bm);
+    else if (aligned) launch_ops<float, LOAD_VEC>(c, a, g, bm);
+    else launch_ops<float, LOAD_ELEM>(c, a, g, bm);
+  }
   TN_HIP(hipGetLastError());
 }
 
 void gemm_grouped_f64(tn_ctx* c, const GroupedDesc& d) {
   if (d.M <= 0 || d.N <= 0 || d.ngroups <= 0 || d.batch <= 0) return;
   TN_REQUIRE(d.ngroups <= 65535 && d.batch <= 65535, TN_E_INVALID, "grouped gemm: grid too large");
-  TN_REQUIRE(extent_ok(d.lda, d.M, 8) && extent_ok(d.ldb, d.K, 8), TN_E_INVALID, "grouped gemm: row stride too large");
-  const int bm = std::min(64, pick_tile(Prec::F64, d.M, d.N, (long)d.ngroups * d.batch));
+  const bool far = !extent_ok(d.lda, d.M, 64, 8) || !extent_ok(d.ldb, d.K, 64, 8);
+  const int bm = far ? 64 : std::min(64, pick_tile(Prec::F64, d.M, d.N, (long)d.ngroups * d.batch));
   const long tiles = ((d.M + bm - 1) / bm) * ((d.N + bm - 1) / bm);
   TN_REQUIRE(tiles < (1L << 31), TN_E_INVALID, "grouped gemm: too many tiles");
   const bool al = (uintptr_t)d.A % 16 == 0 && (uintptr_t)d.B % 16 == 0 &&
@@ -893,10 +937,11 @@ void gemm_grouped_f64(tn_ctx* c, const GroupedDesc& d) {
   };
   constexpr size_t s64 = TileCfg<double, 0, 0, 64, tile_bk<double>(64)>::LDS;
   constexpr size_t s32 = TileCfg<double, 0, 0, 32, tile_bk<double>(32)>::LDS;
-  if (bm == 64 && al) launch(gemm_grouped_kernel<1, 64>, s64);
-  else if (bm == 64) launch(gemm_grouped_kernel<0, 64>, s64);
-  else if (al) launch(gemm_grouped_kernel<1, 32>, s32);
-  else launch(gemm_grouped_kernel<0, 32>, s32);
+  if (far) launch(gemm_grouped_kernel<LOAD_FAR, 64>, s64);
+  else if (bm == 64 && al) launch(gemm_grouped_kernel<LOAD_VEC, 64>, s64);
+  else if (bm == 64) launch(gemm_grouped_kernel<LOAD_ELEM, 64>, s64);
+  else if (al) launch(gemm_grouped_kernel<LOAD_VEC, 32>, s32);
+  else launch(gemm_grouped_kernel<LOAD_ELEM, 32>, s32);
   TN_HIP(hipGetLastError());
 }
 
@@ -906,14 +951,17 @@ void gemm_blocksparse(tn_ctx* c, Prec p, const BsDesc& d) {
              "block-sparse gemm: FP64, FP32 or BF16x3 (FP32 operands) only");
   TN_REQUIRE(d.ntiles % 8 == 0 && d.ntiles < (1L << 31), TN_E_INVALID, "block-sparse gemm: bad tile list");
   const size_t es = p == Prec::F64 ? 8 : 4;
-  TN_REQUIRE(extent_ok(d.lda, BS_TILE, es) && extent_ok(d.ldb, BS_TILE, es), TN_E_INVALID,
-             "block-sparse gemm: row stride too large");
+  const bool far = !extent_ok(d.lda, BS_TILE, BS_TILE, es) || !extent_ok(d.ldb, BS_TILE, BS_TILE, es);
   auto launch = [&](auto kern, size_t shm) {
     allow_lds((const void*)kern, shm);
     hipLaunchKernelGGL(kern, dim3((unsigned)d.ntiles), dim3(256), shm, c->stream, d);
   };
-#define TN_BS(T, TB, SPLIT) \
-  launch(gemm_bs_kernel<T, TB, SPLIT>, TileCfg<T, 0, TB, BS_TILE, SPLIT ? 16 : tile_bk<T>(BS_TILE)>::LDS)
+#define TN_BS(T, TB, SPLIT)                                                                                   \
+  do {                                                                                                        \
+    constexpr size_t shm = TileCfg<T, 0, TB, BS_TILE, SPLIT ? 16 : tile_bk<T>(BS_TILE)>::LDS;                 \
+    if (far) launch(gemm_bs_kernel<T, TB, SPLIT, LOAD_FAR>, shm);                                             \
+    else launch(gemm_bs_kernel<T, TB, SPLIT, LOAD_ELEM>, shm);                                                \
+  } while (0)
   if (p == Prec::F64) {
     if (d.tB) TN_BS(double, 1, false);
     else TN_BS(double, 0, false);

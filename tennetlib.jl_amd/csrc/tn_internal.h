@@ -290,10 +290,8 @@ struct BsDesc {
   double alpha = 1.0;
 };
 void gemm_blocksparse(tn_ctx* c, Prec p, const BsDesc& d);
-// double-buffered kernels (gemm_fast.hip); gemm() uses them when
-// gemm_fast_ok() holds (tile extents below 2^31 bytes)
-bool gemm_fast_ok(Prec p, const GemmDesc& g);
-void gemm_fast(tn_ctx* c, Prec p, const GemmDesc& g);
+// gemm() without the checks and split-K (gemm_fast.hip)
+void gemm_tiles(tn_ctx* c, Prec p, const GemmDesc& g);
 // C (M x N, float) = A * B^T with A (M x K) and B (N x K) as bf16 hi/lo
 // pairs, rows padded to multiples of 8 elements
 void gemm_bf16x3_nt(tn_ctx* c, long M, long N, long K, const unsigned short* Ah, const unsigned short* Al,

@@ -3,6 +3,8 @@ several K tiles (16, 32 rows) ahead in registers, whole and ragged, for output
 sizes at the edges of 32, 64 and 128 tiles; real, complex and FP32, aligned
 and unaligned rows, against the oracle's contraction."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,76 @@ def test_products_over_k_lengths(T, chil, chir, cplx):
         got = T.product(env, psi, precision=prec).reshape(want.shape)
         err = np.linalg.norm(got - want)
         assert err <= n * eps * scale, (prec, err / scale)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("p,n", [(2, 2 ** 21 + 74), (126, 2 ** 21 + 74), (2, 2 ** 22 + 74), (2, 2 ** 25 + 2)])
+def test_rows_beyond_32_bit_offsets(T, p, n, cplx):
+    """Products whose operands' rows are so long (n doubles) that the rows of a
+    tile reach 2^31 or 2^32 bytes, those that are there or with those past the
+    end: the density matrix M M^H and the other factor U^H M of a wide tensor.
+    Sums of n products of a unit tensor: sqrt(n) eps in practice."""
+    ctx = T.default_context()
+    n = n // 4 * 2 if cplx else n
+    rng = np.random.default_rng(n)
+    M = rng.standard_normal((p, n))
+    if cplx:
+        M = M + 1j * rng.standard_normal(M.shape)
+    M /= np.linalg.norm(M)
+    chir = M.shape[1] // 2
+    dt = M.dtype
+    A = [np.ones((1, 2, p // 2), dt), np.ones((p // 2, 2, 1), dt), np.ones((1, 2, chir), dt), np.ones((chir, 2, 1), dt)]
+    env = T.StateEnvs(A, T.heisenberg_mpo(4))
+    dphi = T.DeviceArray.from_numpy(ctx, M.reshape(p // 2, 2, 2, chir))
+    w, err, k = (C.c_double * p)(), C.c_double(), C.c_long()
+    print("long rows", p, n, cplx, flush=True)
+    ctx.check(ctx.lib.tn_replacebond(env.h, 2, dphi.ptr, 1, p, 1, -1.0, 0.0, 1, C.byref(err), w, p, C.byref(k)))
+    a, b = env.get_site(2).reshape(p, -1), env.get_site(3).reshape(-1, M.shape[1])
+    env.close()
+    dphi.free()
+    tol = np.sqrt(n) * 2.0 ** -52
+    assert np.abs(np.array(w[:k.value]) - np.linalg.eigvalsh(M @ M.conj().T)[::-1]).max() <= tol
+    assert np.linalg.norm(a @ b - M) <= tol
+    assert np.abs(a.conj().T @ a - np.eye(p)).max() <= p * 1e-15
+
+
+def test_block_sparse_rows_beyond_32_bit_offsets(T):
+    """The QN product with an operator of 16300 channels on the right: its second
+    block-sparse product reads rows of 4 * 16300 * 64 numbers.  All channels are
+    diagonal, so the environment and the result are short contractions.  Sums of
+    16300 * 64 products, sqrt of that in eps in practice: 1e-12 of the sums of
+    absolute values."""
+    rng = np.random.default_rng(5)
+    w, chil, chir = 16300, 3, 64
+    ql, qr = np.array([-1, -1, 1]), np.repeat([-1, 1], chir // 2)
+    spin = np.array([1, -1])
+    f1, f2 = rng.standard_normal(2), rng.standard_normal(2)
+    f3, f4 = rng.standard_normal((2, w)), rng.standard_normal((w, 2))
+    eye = np.eye(2)
+    Ws = [np.einsum("ij,j->ij", eye, f)[None, :, :, None] for f in (f1, f2)]
+    Ws += [np.einsum("ij,jc->ijc", eye, f3)[None], np.einsum("ij,cj->cij", eye, f4)[..., None]]
+    A1 = rng.standard_normal((1, 2, chil)) * (spin[None, :, None] == ql)
+    A4 = rng.standard_normal((chir, 2, 1)) * (qr[:, None, None] + spin[None, :, None] == 0)
+    A2, A3 = rng.standard_normal((chil, 2, 2)), rng.standard_normal((2, 2, chir))
+    env = T.StateEnvs([A1, A2, A3, A4], Ws)
+    ctx, pi = env.ctx, C.POINTER(C.c_int)
+    sq = np.tile(spin, 4).astype(np.int32)
+    lq = np.concatenate([[0], ql, [0, 0], qr, [0]]).astype(np.int32)
+    ctx.check(ctx.lib.tn_env_set_qn(env.h, 1, sq.ctypes.data_as(pi), lq.ctypes.data_as(pi)))
+    T.position_(env, 2)
+    mask = (ql[:, None, None, None] + spin[:, None, None] + spin[:, None] == qr)
+    psi = rng.standard_normal(mask.shape) * mask
+
+    def product(a1, a4, g1, g2, g3, g4, v):
+        L = np.einsum("sa,sc,s->ac", a1[0], a1[0], g1)
+        v = np.einsum("ac,cstb,s->astb", L, v, g2)
+        O = g3 @ g4                                    # [spin 3, spin 4], summed over the channels
+        R = np.einsum("bs,cs,ts->tbc", a4[..., 0], a4[..., 0], O)
+        return np.einsum("astb,tbc->astc", v, R)
+
+    print("long block rows", flush=True)
+    got = T.product(env, psi).reshape(psi.shape)
+    want = product(A1, A4, f1, f2, f3, f4, psi) * mask
+    cap = product(*(np.abs(x) for x in (A1, A4, f1, f2, f3, f4, psi)))
+    assert np.linalg.norm(got - want) <= 1e-12 * np.linalg.norm(cap)
+    env.close()
