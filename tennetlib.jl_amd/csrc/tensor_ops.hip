@@ -438,13 +438,13 @@ __global__ __launch_bounds__(256) void multidot_stage2(const double* __restrict_
 // next basis vector w / |w|.  Short vectors: one workgroup with w in
 // registers.  Others: a launch per pass over V -- dots; update and the second
 // pass's dots, from one read of V; update and norm; scaling -- where every
-// workgroup sums the previous launch's partial sums for itself, in a fixed
-// order.  Bound by launches and load latency up to about 10^6 elements (n = 1.4
+// workgroup sums the previous launch's partial sums for itself, or a launch in
+// between sums them (KP_SELF_SUM), in a fixed order.  Bound by launches and load latency up to about 10^6 elements (n = 1.4
 // 10^5, 10 vectors: V is 11 MB, 3 us), so all loads of a tile are issued before
 // the first is used.  A solve of 7 steps at n = 137k took 750 us with nine
 // launches a step (dots and their sums, update, twice; norm and its sum;
-// scaling) and the start's norm read by the host, with four 580 us; two-site
-// sweeps of 20 spins, mostly short vectors, 58 -> 49 ms.
+// scaling) and the start's norm read by the host, with four 590 us, with six 550;
+// two-site sweeps of 20 spins, mostly short vectors, 58 -> 49 ms.
 // ---------------------------------------------------------------------------
 constexpr int KS_THREADS = 1024;  // one-workgroup step
 constexpr int KP_TILE = 512;      // elements per tile of the others, two a thread
@@ -583,15 +583,28 @@ __device__ __forceinline__ double sum_parts16(const double* __restrict__ pin, in
   return s;
 }
 
+// sums of np partial results each, one workgroup per value
+__global__ __launch_bounds__(256) void krylov_sum_kernel(const double* __restrict__ pin, int np,
+                                                         double* __restrict__ out) {
+  __shared__ double red[4];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < np; i += 256) s += pin[(long)blockIdx.x * np + i];
+  s = wave_sum64(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 // PHASE 0: dots of w with the basis vectors.  PHASE 1: their sums, w updated,
 // dots of the new w.  PHASE 2: sums, update, |w|^2.  NV >= K, or 16 (then the
 // dots of PHASE 1 read V once more).  Partial results of workgroup g at
-// pout[value * gridDim.x + g]; hout: the coefficients of this phase.
+// pout[value * gridDim.x + g], np of the previous launch per value at pin;
+// hout: the coefficients of this phase.
 template <bool CX, int PHASE, int NV>
 __global__ __launch_bounds__(256) void krylov_pass_kernel(const double* __restrict__ basis, long ld, int K,
                                                           double* __restrict__ w, long n,
-                                                          const double* __restrict__ pin, double* __restrict__ pout,
-                                                          double* __restrict__ hout) {
+                                                          const double* __restrict__ pin, int np,
+                                                          double* __restrict__ pout, double* __restrict__ hout) {
   constexpr int C = CX ? 2 : 1;
   __shared__ double cf[128];
   __shared__ double red[4][C * NV];
@@ -601,7 +614,7 @@ __global__ __launch_bounds__(256) void krylov_pass_kernel(const double* __restri
     if (tid < 128) cf[tid] = 0.0;
     __syncthreads();
     for (int v = tid >> 4; v < nacc; v += 16) {
-      const double s = sum_parts16(pin + (long)v * nblk, nblk);
+      const double s = sum_parts16(pin + (long)v * np, np);
       if ((tid & 15) == 0) {
         cf[v] = s;
         if (blockIdx.x == 0) hout[v] = s;
@@ -1194,13 +1207,31 @@ static bool krylov_small(tn_ctx* c, const double* basis, long ld, int K, double*
   return true;
 }
 
+// Partial results a value up to which the next launch's workgroups sum them
+// each for itself; more take a launch of their own, since all workgroups
+// together read values * np^2 of them.  Kernel times of a solve, us, summed by
+// the passes and by launches of their own: real 14 400 elements and 10 vectors
+// (np 29) 173 and 222, complex 40 000 and 30 (79) 1068 and 1189; real 137 000
+// and 10 (268) 295 and 255, complex 160 000 and 30 (313) 2670 and 1810, complex
+// 600 000 and 10 (1024) 1180 and 647, and 30 9810 and 4050.
+constexpr int KP_SELF_SUM = 128;
+
 template <bool CX, int NV>
-static void krylov_passes(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, double* p1, double* p2,
-                          double* p3, double* hout) {
-  const dim3 g(krylov_blocks(n)), b(256);
-  hipLaunchKernelGGL((krylov_pass_kernel<CX, 0, NV>), g, b, 0, c->stream, basis, ld, K, w, n, nullptr, p1, nullptr);
-  hipLaunchKernelGGL((krylov_pass_kernel<CX, 1, NV>), g, b, 0, c->stream, basis, ld, K, w, n, p1, p2, hout);
-  hipLaunchKernelGGL((krylov_pass_kernel<CX, 2, NV>), g, b, 0, c->stream, basis, ld, K, w, n, p2, p3, hout + 128);
+static void krylov_passes(tn_ctx* c, const double* basis, long ld, int K, double* w, long n, int nb, double* p1,
+                          double* p2, double* p3, double* sums, double* hout) {
+  const dim3 g(nb), b(256);
+  const bool self = nb <= KP_SELF_SUM;
+  auto summed = [&](double* p) {
+    if (self) return p;
+    hipLaunchKernelGGL(krylov_sum_kernel, dim3(CX ? 2 * K : K), b, 0, c->stream, (const double*)p, nb, sums);
+    return sums;
+  };
+  const int np = self ? nb : 1;
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 0, NV>), g, b, 0, c->stream, basis, ld, K, w, n, nullptr, 0, p1, nullptr);
+  const double* s1 = summed(p1);
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 1, NV>), g, b, 0, c->stream, basis, ld, K, w, n, s1, np, p2, hout);
+  const double* s2 = summed(p2);
+  hipLaunchKernelGGL((krylov_pass_kernel<CX, 2, NV>), g, b, 0, c->stream, basis, ld, K, w, n, s2, np, p3, hout + 128);
   TN_HIP(hipGetLastError());
 }
 
@@ -1210,12 +1241,13 @@ static void krylov_step_t(tn_ctx* c, const double* basis, long ld, int K, double
   if (krylov_small<CX>(c, basis, ld, K, w, n, vnext, hout)) return;
   const int nb = krylov_blocks(n), nacc = CX ? 2 * K : K;
   const long nd = CX ? 2 * n : n;
-  double* p1 = (double*)c->workspace(WS_KRY_PART, (size_t)(2 * nacc + 1) * nb * sizeof(double));
+  double* p1 = (double*)c->workspace(WS_KRY_PART, ((size_t)(2 * nacc + 1) * nb + nacc) * sizeof(double));
   double* p2 = p1 + (size_t)nacc * nb;
   double* p3 = p2 + (size_t)nacc * nb;
-  if (K <= 4) krylov_passes<CX, 4>(c, basis, ld, K, w, n, p1, p2, p3, hout);
-  else if (K <= 8) krylov_passes<CX, 8>(c, basis, ld, K, w, n, p1, p2, p3, hout);
-  else krylov_passes<CX, 16>(c, basis, ld, K, w, n, p1, p2, p3, hout);
+  double* sums = p3 + nb;
+  if (K <= 4) krylov_passes<CX, 4>(c, basis, ld, K, w, n, nb, p1, p2, p3, sums, hout);
+  else if (K <= 8) krylov_passes<CX, 8>(c, basis, ld, K, w, n, nb, p1, p2, p3, sums, hout);
+  else krylov_passes<CX, 16>(c, basis, ld, K, w, n, nb, p1, p2, p3, sums, hout);
   hipLaunchKernelGGL(krylov_scale_kernel, dim3(grid1d(nd)), dim3(256), 0, c->stream, vnext, (const double*)w, nd,
                      (const double*)p3, nb, hout + 256);
   TN_HIP(hipGetLastError());

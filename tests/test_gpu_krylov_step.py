@@ -87,6 +87,30 @@ def test_expm(T, chil, chir, cplx):
     assert np.linalg.norm(y - want) <= 2.5e-12 * max(1.0, np.linalg.norm(want))
 
 
+@pytest.mark.parametrize("chil,chir", [(128, 128), (128, 129), (300, 437)])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("kd", [3, 7, 18])
+def test_eig_of_long_vectors(T, chil, chir, cplx, kd):
+    """The last size whose passes sum the previous launch's 128 partial results
+    themselves and the first that has them summed by a launch, and 1025 tiles of
+    512 elements for the 1024 workgroups: the value and vector against the
+    oracle's, and the value against the vector's own."""
+    env, ref, x = setup(T, chil, chir, cplx)
+    ctx = env.ctx
+    print("long eig", chil, chir, cplx, kd, flush=True)
+    th_ref, y_ref, _ = O.eigsolve_lanczos(ref.product, x, krylovdim=kd, maxiter=1, tol=1e-14)
+    dx = T.DeviceArray.from_numpy(ctx, x)
+    th, info = C.c_double(), T._lib.KrylovInfo()
+    ctx.check(ctx.lib.tn_krylov_eig(env.h, dx.ptr, kd, 1, 1e-14, 0, C.byref(th), C.byref(info)))
+    y = dx.numpy()
+    dx.free()
+    scale = max(np.linalg.norm(ref.product(x)) / np.linalg.norm(x), abs(th_ref))
+    assert abs(th.value - th_ref) <= 1e-12 * scale
+    assert abs(np.linalg.norm(y) - 1.0) <= 1e-14 * np.sqrt(kd)
+    assert abs(np.vdot(y, ref.product(y)).real - th.value) <= 1e-12 * scale
+    assert abs(abs(np.vdot(y, y_ref)) - 1.0) <= 1e-8
+
+
 def test_zero_start_vectors(T):
     env, _, x = setup(T, 16, 16, False)
     ctx = env.ctx
