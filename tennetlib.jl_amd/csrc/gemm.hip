@@ -24,18 +24,22 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const T* __restrict_
 }  // namespace
 
 // Few output tiles with a long K (K-reductions over whole tensors, Gram
-// matrices of tall matrices) leave most of the chip idle: split K into
-// chunks computed as one batched GEMM into FP64/FP32 partials, then reduce.
-// Chunk length along K of the split (0: no split).  The reduction is one more
-// launch (about 4 us); a 32 x 32 tile runs K at about 7 ns a row, so from
-// half a chip of idle CUs and chunks of 256 rows on the split pays.
+// matrices of tall matrices) leave most of the chip idle: split K into chunks,
+// the last one shorter, computed as one batched GEMM into FP64/FP32 partials,
+// then reduce.  Chunk length along K (0: no split).  The reduction is one more
+// launch (about 4 us); a 32 x 32 FP64 tile runs K at about 7 ns a row, so from
+// half a chip of idle CUs and chunks of 256 rows on the split pays; the 64 x 64
+// FP32 tile is slower per row: chunks of 128.  H psi with chi_l = 4, d = 2, in
+// us, chunks of 64 / 128 / 256: FP32 w = 3, chi_r = 128 32.1 / 32.8 / 36.2; FP64
+// 25.9 / 26.0 / 27.0.
 static long split_chunk(Prec p, const GemmDesc& g) {
   if (!(p == Prec::F64 || p == Prec::F32) || g.batch != 1) return 0;
   const long t128 = ((g.M + 127) / 128) * ((g.N + 127) / 128);
   const long b = p == Prec::F64 ? 32 : 64, tiles = ((g.M + b - 1) / b) * ((g.N + b - 1) / b);
+  const long chunk = p == Prec::F64 ? 256 : 128;
   long P0;
   if (t128 < 64 && g.K >= 4096) P0 = std::min<long>(g.K / 512, 256 / t128);
-  else if (tiles <= 128 && g.K >= 512) P0 = std::min<long>(g.K / 256, 256 / tiles);
+  else if (tiles <= 128 && g.K >= 2 * chunk) P0 = std::min<long>(g.K / chunk, 256 / tiles);
   else return 0;
   if (P0 < 2) return 0;
   return ((g.K + P0 - 1) / P0 + 15) / 16 * 16;
@@ -45,7 +49,6 @@ static bool gemm_split_k(tn_ctx* c, Prec p, const GemmDesc& g) {
   const long Kc = split_chunk(p, g);
   if (Kc == 0) return false;
   const long P = (g.K + Kc - 1) / Kc;
-  const long full = g.K / Kc;  // chunks of exactly Kc
   const size_t es = (p == Prec::F64) ? 8 : 4;
   const size_t need = (size_t)P * g.M * g.N * es;
   char* part;
@@ -58,21 +61,30 @@ static bool gemm_split_k(tn_ctx* c, Prec p, const GemmDesc& g) {
   GemmDesc q = g;
   q.alpha = 1.0;
   q.beta = 0.0;
-  q.K = Kc;
+  q.kstep = Kc;
   q.C = part;
   q.ldc = g.N;
   q.sC = g.M * g.N;
   q.sA = g.tA ? Kc * g.lda : Kc;
   q.sB = g.tB ? Kc : Kc * g.ldb;
-  q.batch = (int)full;
+  // the shorter last chunk goes with the others, unless their workgroups fill
+  // the chip and it would cost all of them another round: 32 x 181 outputs, K =
+  // 543 in two, H psi 29.7 us together, 37.6 apart; 1020 x 253, K = 5060 in nine,
+  // product 70 us together, 61 apart
+  const long last = g.K - (P - 1) * Kc;
+  const double others = gemm_tile_work(p, g.M, g.N, P - 1);
+  const bool together = last == Kc || gemm_tile_work(p, g.M, g.N, P) * Kc <=
+                                          others * Kc + gemm_tile_work(p, g.M, g.N, 1) * last;
+  q.batch = (int)(together ? P : P - 1);
   gemm_tiles(c, p, q);
-  if (full < P) {  // the shorter last chunk
+  if (!together) {
     GemmDesc r = q;
     r.batch = 1;
-    r.K = g.K - full * Kc;
-    r.A = (const char*)g.A + (size_t)(full * q.sA) * es;
-    r.B = (const char*)g.B + (size_t)(full * q.sB) * es;
-    r.C = part + (size_t)(full * q.sC) * es;
+    r.K = last;
+    r.kstep = 0;
+    r.A = (const char*)g.A + (size_t)((P - 1) * q.sA) * es;
+    r.B = (const char*)g.B + (size_t)((P - 1) * q.sB) * es;
+    r.C = part + (size_t)((P - 1) * q.sC) * es;
     gemm_tiles(c, p, r);
   }
   const long tot = g.M * g.N;

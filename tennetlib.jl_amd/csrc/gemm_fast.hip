@@ -41,6 +41,7 @@ struct FArgs {
   void* C; long ldc; long sC;
   double alpha, beta;
   int cA, cB;  // complex: conjugated operands
+  long kstep, Kall;  // batch z sums rows z kstep .. of K alone, at most K of Kall
 };
 
 __device__ __forceinline__ void tile_coords2(int ntm, int ntn, int& tm, int& tn) {
@@ -499,8 +500,11 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(FArgs a) {
   int tm, tn;
   tile_coords2(ntm, ntn, tm, tn);
   const long m0 = (long)tm * BM, n0 = (long)tn * BM, bz = blockIdx.z;
-  OneSeg seg{reinterpret_cast<const T*>(a.A) + bz * a.sA, reinterpret_cast<const T*>(a.B) + bz * a.sB, a.K, a.wA, a.wB,
-             a.K <= 0};
+  // the last part of a split K is shorter
+  const long kb = bz * a.kstep, K = min(a.K, a.Kall - kb);
+  const long wA = TA || a.kstep == 0 ? a.wA : min(a.K, a.wA - kb), wB = !TB || a.kstep == 0 ? a.wB : min(a.K, a.wB - kb);
+  OneSeg seg{reinterpret_cast<const T*>(a.A) + bz * a.sA, reinterpret_cast<const T*>(a.B) + bz * a.sB, K, wA, wB,
+             K <= 0};
   typename Acc<T>::type acc[CF::F][CF::F];
   tile_zero<CF, T>(acc);
   tile_product<CF, T, TA, TB, AL, false, false>(seg, a.M, a.N, m0, n0, a.lda, a.ldb, a.cA, a.cB,
@@ -847,7 +851,7 @@ static bool extent_ok(long ld, long rows, long tile_rows, size_t es) {
 // tile size keeps the MFMAs fed (measured on full grids: FP64 128 63 TF/s,
 // 64 55, 32 30; complex 64 about the same as 32 with a quarter of the loads).
 // Complex products and FP32 have no 128 / 32 tile respectively.
-static int pick_tile(Prec p, long M, long N, long batch) {
+static int pick_tile(Prec p, long M, long N, long batch, double* work = nullptr) {
   int best = 0;
   double cost = 0.0;
   for (int b : {128, 64, 32}) {
@@ -860,7 +864,13 @@ static int pick_tile(Prec p, long M, long N, long batch) {
       cost = t;
     }
   }
+  if (work) *work = cost;
   return best;
+}
+double gemm_tile_work(Prec p, long M, long N, long batch) {
+  double work;
+  pick_tile(p, M, N, batch, &work);
+  return work;
 }
 
 namespace {
@@ -905,6 +915,8 @@ void gemm_tiles(tn_ctx* c, Prec p, const GemmDesc& g) {
   a.wB = aligned ? width_b(p, g) : (g.tB ? g.K : g.N);
   a.C = g.C; a.ldc = g.ldc; a.sC = g.sC;
   a.alpha = g.alpha; a.beta = g.beta;
+  a.kstep = g.kstep; a.Kall = g.K;
+  if (g.kstep) a.K = g.kstep;
   const int bm = pick_tile(p, g.M, g.N, g.batch);
   if (p == Prec::Z64) {
     if (far) launch_ops<double2, LOAD_FAR>(c, a, g, bm);

@@ -237,6 +237,8 @@ struct GemmDesc {
   void* C = nullptr; long ldc = 0; long sC = 0;
   int batch = 1;
   double alpha = 1.0, beta = 0.0;
+  // K in parts: batch z sums its rows z kstep .. (z + 1) kstep alone (0: all of K)
+  long kstep = 0;
   // split-K partial products: a caller-owned device buffer of split_cap bytes
   // used instead of the context workspace when set (no split if it is too small)
   void* split_ws = nullptr;
@@ -292,6 +294,8 @@ struct BsDesc {
 void gemm_blocksparse(tn_ctx* c, Prec p, const BsDesc& d);
 // gemm() without the checks and split-K (gemm_fast.hip)
 void gemm_tiles(tn_ctx* c, Prec p, const GemmDesc& g);
+// work on the busiest CU per row of K, in outputs of the fastest tile
+double gemm_tile_work(Prec p, long M, long N, long batch);
 // C (M x N, float) = A * B^T with A (M x K) and B (N x K) as bf16 hi/lo
 // pairs, rows padded to multiples of 8 elements
 void gemm_bf16x3_nt(tn_ctx* c, long M, long N, long K, const unsigned short* Ah, const unsigned short* Al,

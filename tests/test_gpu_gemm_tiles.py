@@ -56,6 +56,14 @@ def test_products_over_k_lengths(T, chil, chir, cplx):
         assert err <= n * eps * scale, (prec, err / scale)
 
 
+# K of the last product (3 chi right) split into parts of 256 (FP64) or 128 rows:
+# the first split sizes, equal parts, and last parts of one row and more
+@pytest.mark.parametrize("chil,chir", [(2, 85), (2, 86), (1, 128), (2, 170), (3, 171), (5, 181), (2, 256), (1, 343)])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_products_over_split_k(T, chil, chir, cplx):
+    test_products_over_k_lengths(T, chil, chir, cplx)
+
+
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("p,n", [(2, 2 ** 21 + 74), (126, 2 ** 21 + 74), (2, 2 ** 22 + 74), (2, 2 ** 25 + 2)])
 def test_rows_beyond_32_bit_offsets(T, p, n, cplx):
