@@ -1,7 +1,9 @@
 """H psi at the K lengths where the pipelined products change: no, one and
 several K tiles (16, 32 rows) ahead in registers, whole and ragged, for output
 sizes at the edges of 32, 64 and 128 tiles; real, complex and FP32, aligned
-and unaligned rows, against the oracle's contraction."""
+and unaligned rows, against the oracle's contraction; in FP64 also in place, since
+small separate vectors take a one-launch product without these kernels.  Products
+with K in parts, and with rows past 32-bit tile offsets."""
 
 import ctypes as C
 
@@ -9,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import tn_oracle as O
+from tests.test_gpu_wstep import in_place_product
 
 pytestmark = pytest.mark.gpu
 
@@ -54,6 +57,9 @@ def test_products_over_k_lengths(T, chil, chir, cplx):
         got = T.product(env, psi, precision=prec).reshape(want.shape)
         err = np.linalg.norm(got - want)
         assert err <= n * eps * scale, (prec, err / scale)
+        if prec == "fp64":  # in place: three launches also where separate vectors take one
+            err = np.linalg.norm(in_place_product(T, env, psi) - want)
+            assert err <= n * eps * scale, ("in place", err / scale)
 
 
 # K of the last product (3 chi right) split into parts of 256 (FP64) or 128 rows:

@@ -1,7 +1,8 @@
 """H psi where the operator step changes kernels: operators of one to 128 rows
 and columns (blocks of 16 rows in FP64, 32 in FP32, K groups of 20 and 10),
 dense and sparse, with column counts at the edges of a strip (32 and 64), odd
-ones and one column, against the oracle's contraction."""
+ones and one column, against the oracle's contraction; in FP64 also in place,
+since small separate vectors take a one-launch product without this step."""
 
 import numpy as np
 import pytest
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # (MPO bond, d, sites, chi left, chi right): rows and columns = bond * d^sites
 SIZES = [(1, 2, 1, 5, 1), (5, 2, 1, 16, 33), (8, 2, 1, 16, 64), (17, 1, 1, 9, 31), (5, 2, 2, 40, 64),
          (8, 2, 2, 3, 66), (11, 3, 1, 7, 65), (4, 4, 2, 16, 30), (20, 2, 2, 33, 97), (24, 2, 2, 20, 32),
-         (7, 4, 2, 6, 34), (32, 2, 2, 37, 63), (8, 4, 2, 64, 128)]
+         (7, 4, 2, 6, 34), (32, 2, 2, 37, 63), (8, 4, 2, 64, 128), (24, 2, 1, 64, 65), (16, 2, 2, 33, 98),
+         (20, 2, 2, 17, 66), (24, 2, 2, 64, 65), (6, 4, 2, 64, 66), (7, 4, 2, 33, 67), (3, 2, 1, 40, 1)]
 
 
 @pytest.fixture(scope="module")
@@ -33,6 +35,16 @@ def chain(w, d, chil, chir, fill, seed):
         Ws.append(W * (rng.random(W.shape) < fill))
     A = [rng.standard_normal((cd[k], d, cd[k + 1])) for k in range(4)]
     return Ws, A, rng
+
+
+def in_place_product(T, env, psi):
+    """H psi in FP64 with the output over the input, which takes the GEMM, the
+    operator step and the GEMM at any size."""
+    buf = T.DeviceArray.from_numpy(env.ctx, psi)
+    env.ctx.check(env.ctx.lib.tn_env_matvec(env.h, buf.ptr, buf.ptr, 0))
+    out = buf.numpy()
+    buf.free()
+    return out
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "w%d_d%d_n%d_%dx%d" % s)
@@ -65,6 +77,9 @@ def test_operator_step(T, size, fill):
         got = T.product(env, psi, precision=prec).reshape(want.shape)
         err = np.linalg.norm(got - want)
         assert err <= tol * scale, (prec, err / max(scale, 1e-300))
+        if prec == "fp64":  # in place: three launches also where separate vectors take one
+            err = np.linalg.norm(in_place_product(T, env, psi) - want)
+            assert err <= tol * scale, ("in place", err / max(scale, 1e-300))
 
 
 @pytest.mark.parametrize("chi", [8, 15, 64, 65])
