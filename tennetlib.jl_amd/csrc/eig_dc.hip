@@ -2,13 +2,17 @@
 // Up to DC_SMALL_MAX rows one workgroup does each stage (eig_small.hip).
 // Above that:
 //
-//  1. Householder tridiagonalisation G = H T H^T on the device, one column
-//     per step: trd_reflect_kernel forms the reflector from row j (every
-//     workgroup redundantly, so no extra launch) and y = tau G22 v;
-//     trd_update_kernel applies G22 -= v w^T + w v^T.  The reflectors are
-//     kept below the diagonal of G.  The last TRD_SMALL_MAX columns are
-//     reduced by one workgroup in registers (416 us for 192 columns; 136
-//     columns in LDS took 556 us, one launch per column 7.1 us each).
+//  1. Householder tridiagonalisation G = H T H^T on the device, the reflectors
+//     kept below the diagonal of G.  Real matrices below TRD_BLOCKED_MIN rows:
+//     trd_reflect_kernel forms reflector 0 and y = tau G22 v, one launch per
+//     column (trd_step_reg_kernel where a row fits a wavefront's registers,
+//     trd_step_kernel above) applies G22 -= v w^T + w v^T and forms the next
+//     reflector and y, trd_update_kernel applies the last one.  Larger ones:
+//     panels of columns (trd_panel_*, trd_symv_*).  Complex ones:
+//     trdz_reflect_kernel and trdz_update_kernel for every column.  The last
+//     TRD_SMALL_MAX columns (complex TRD_SMALL_MAX_Z) are reduced by one
+//     workgroup in registers (416 us for 192 columns; 136 columns in LDS took
+//     556 us, one launch per column 7.1 us each).
 //  2. Divide and conquer on T (Cuppen's tearing, bottom-up): leaves of at
 //     most DC_SMALL_MAX rows are solved one workgroup each (dc_small); each
 //     merge of two neighbouring blocks solves
@@ -123,7 +127,7 @@ __global__ __launch_bounds__(256) void trd_reflect_kernel(double* __restrict__ A
     // v below the diagonal of column j (never read again as matrix data)
     for (int c = tid; c < m; c += 256) {
       A[(long)(j + 1 + c) * ld + j] = vs[c];
-      if (vcont) vcont[c] = vs[c];
+      vcont[c] = vs[c];
     }
     if (tid == 0) {
       dv[j] = A[(long)j * ld + j];
@@ -211,7 +215,8 @@ __global__ __launch_bounds__(256) void trd_update_kernel(double* __restrict__ A,
 //   y_{j+1}[r] = tau (old_r . v' - v_j[r] (w_j . v') - w_j[r] (v_j . v'))
 // so each row is read once and written once per column, by one workgroup.
 // Vectors are indexed from row j + 1 (v_j, w_j) and from row j + 2 (v').
-// Dynamic LDS: 3 (p - j - 1) doubles.
+// Dynamic LDS: 3 (p - j - 1) doubles.  mn = p - j - 2 <= STEP_ROW.
+constexpr int STEP_ROW = 12 * 256;
 __global__ __launch_bounds__(256) void trd_step_kernel(double* __restrict__ A, long ld, int p, int j,
                                                        const double* __restrict__ vj_in,
                                                        const double* __restrict__ yj,
@@ -228,8 +233,8 @@ __global__ __launch_bounds__(256) void trd_step_kernel(double* __restrict__ A, l
   double* vn = wj + mj;
   const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // issue the loads of row j+1 up front, so their latency overlaps the vector
-  // set-up (rows up to 6144 long)
-  constexpr int OV = 24;
+  // set-up
+  constexpr int OV = STEP_ROW / 256;
   const double* orow = A + (long)(j + 1) * ld + (j + 2);
   double ov[OV];
 #pragma unroll
@@ -1826,10 +1831,13 @@ void wy_tsolve(tn_ctx* c, const double* S, const double* tauv, int j0, int nb, d
   TN_HIP(hipGetLastError());
 }
 
-// smallest p reduced in panels: below it one fused launch per column is
-// faster (measured: p = 2048 takes 45 ms fused against 57 ms in panels,
-// p = 4096 245 ms against 171 ms)
+// smallest p reduced in panels; below it one fused launch per column.  The line
+// is that of earlier panel kernels (p = 2048 45 ms fused, 57 in panels; 4096 245
+// and 171).  With the present ones the two cross near 1700: whole factorisation,
+// ms, fused and panels, p = 1280 13.6 and 17.5, 1536 21.3 and 22.5, 2048 39.7 and
+// 33.4, 2560 71.9 and 45.5, 3070 110.7 and 59.2.
 constexpr int TRD_BLOCKED_MIN = 3072;
+static_assert(TRD_BLOCKED_MIN <= STEP_ROW, "rows of the fused step");
 // smallest trailing block whose product reads only the lower triangle (two
 // launches per column instead of one)
 constexpr int TRD_TILE_MIN = 1024;

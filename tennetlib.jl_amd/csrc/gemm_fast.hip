@@ -201,7 +201,7 @@ struct TileCfg {
 // K tile of a tile size: 128 holds two 35 KB stages per operand pair, the
 // small tiles trade LDS for fewer barriers
 template <typename T> constexpr int tile_bk(int bm) {
-  return sizeof(T) == 8 ? (bm == 128 ? 16 : 32) : sizeof(T) == 4 ? (bm == 128 ? 32 : 32) : 16;
+  return sizeof(T) == 8 ? (bm == 128 ? 16 : 32) : sizeof(T) == 4 ? 32 : 16;
 }
 
 // acc += sum over the K segments of seg of A_s (rows m0..) * B_s (columns
@@ -849,8 +849,10 @@ static bool extent_ok(long ld, long rows, long tile_rows, size_t es) {
 // Tile of an M x N product over a batch: the one with the least work on the
 // busiest CU, tiles / 256 rounds of b^2 outputs each, weighted by how well a
 // tile size keeps the MFMAs fed (measured on full grids: FP64 128 63 TF/s,
-// 64 55, 32 30; complex 64 about the same as 32 with a quarter of the loads).
-// Complex products and FP32 have no 128 / 32 tile respectively.
+// 64 55, 32 30).  Complex products and FP32 have no 128 / 32 tile respectively.
+// Complex products take the FP64 weights; 64 and 32 tiles run at about the same
+// rate there.  H psi (w = 5), us, by the rule and on 32 tiles throughout: chi =
+// 200 112 and 114, 256 168 and 152, 400 552 and 484, 512 800 and 855.
 static int pick_tile(Prec p, long M, long N, long batch, double* work = nullptr) {
   int best = 0;
   double cost = 0.0;

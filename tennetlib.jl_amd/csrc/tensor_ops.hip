@@ -439,12 +439,13 @@ __global__ __launch_bounds__(256) void multidot_stage2(const double* __restrict_
 // registers.  Others: a launch per pass over V -- dots; update and the second
 // pass's dots, from one read of V; update and norm; scaling -- where every
 // workgroup sums the previous launch's partial sums for itself, or a launch in
-// between sums them (KP_SELF_SUM), in a fixed order.  Bound by launches and load latency up to about 10^6 elements (n = 1.4
-// 10^5, 10 vectors: V is 11 MB, 3 us), so all loads of a tile are issued before
-// the first is used.  A solve of 7 steps at n = 137k took 750 us with nine
-// launches a step (dots and their sums, update, twice; norm and its sum;
-// scaling) and the start's norm read by the host, with four 590 us, with six 550;
-// two-site sweeps of 20 spins, mostly short vectors, 58 -> 49 ms.
+// between sums them (KP_SELF_SUM), in a fixed order.  Bound by launches and load
+// latency up to about 10^6 elements (n = 1.4 10^5, 10 vectors: V is 11 MB, 3
+// us), so all loads of a tile are issued before the first is used.  A solve of 7
+// steps at n = 137k took 750 us with nine launches a step (dots and their sums,
+// update, twice; norm and its sum; scaling) and the start's norm read by the
+// host, with four 590 us, with six 550; two-site sweeps of 20 spins, mostly
+// short vectors, 58 -> 49 ms.
 // ---------------------------------------------------------------------------
 constexpr int KS_THREADS = 1024;  // one-workgroup step
 constexpr int KP_TILE = 512;      // elements per tile of the others, two a thread

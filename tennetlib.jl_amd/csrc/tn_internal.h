@@ -485,7 +485,8 @@ void dc_small(tn_ctx* c, int nmax, int nb, const SmallEig& one, const SmallEig* 
               double* Q, double* lam);
 void back_small(tn_ctx* c, bool cplx, int nmax, int nb, const SmallEig& one, const SmallEig* list, const void* A,
                 const void* tau, const double* Q, void* V);
-// Symmetric blocks of at most BACK_SMALL_MAX rows together: block i (n x n at
+// Symmetric blocks of at most BACK_SMALL_MAX rows together (columns beyond a
+// block's last TRD_SMALL_MAX one block after another): block i (n x n at
 // a, row stride lda in G, overwritten) leaves its eigenvectors as rows at v
 // (row stride ldv) in V; w receives the eigenvalues, block after block.  de, q,
 // ldq and flags are the function's own.

@@ -1884,7 +1884,8 @@ void replacebond(tn_env* e, int b, const double* phi, bool ortho_left, long maxd
 // combined (link, site) index.  Rows of M (ortho left; columns, through the
 // transpose, for ortho right) are gathered sector by sector; blocks of at most
 // BACK_SMALL_MAX rows are formed by one block-sparse product and diagonalised
-// together, larger ones one by one.  All weights go through
+// together (columns beyond a block's last TRD_SMALL_MAX block after block),
+// larger ones one by one.  All weights go through
 // truncate!!; each block keeps its weights above docut (whole multiplets split
 // across blocks are dropped together, exact zeros go).  The new link lists
 // the kept sectors in ascending QN order, weights descending within each.
@@ -1949,7 +1950,8 @@ void replacebond_qn(tn_env* e, int b, const double* phi, bool ortho_left, long m
   double* Vd = (double*)c->workspace(WS_QN_V, (size_t)std::max<long>(vtot, 1) * sizeof(double));
   // rho_q = G_q G_q^T of every block that the batched eigensolver takes, by one
   // block-sparse product into a stack.  A step of the eigensolver lasts as long
-  // as its largest block takes: H psi and this factorisation with sectors of
+  // as its largest block takes, except the columns beyond a block's last
+  // TRD_SMALL_MAX, whose launches add up over the blocks: H psi and this factorisation with sectors of
   // 292, 4 x 188, 4 x 121, 4 x 46 and 15 more of at most 29 rows took 9.2 ms
   // with the blocks above 96 rows one by one and batched Jacobi rotations below
   // (17.1 ms when each block also took more launches), together 2.7 ms.

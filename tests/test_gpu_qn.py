@@ -211,7 +211,7 @@ def test_qn_dmrg_hubbard_n32_matches_golden(T):
     2e-16 perturbations of its density matrices (the maxdim cut splits
     multiplets; tests/test_oracle_qn.py::test_hubbard_n32_sensitivity), and
     by 7e-7 under 2e-14 perturbations (the backward error of an eigensolver
-    of another kind, such as the Jacobi of small blocks here), so: first
+    of another kind than the oracle's), so: first
     sweep to 1e-10 per site, ramp sweeps to 1e-5, the last sweep to 5e-9;
     maxchi exact; every link's sectors allowed and its dimension within 4 of
     the oracle's."""
