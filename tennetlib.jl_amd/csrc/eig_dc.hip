@@ -11,7 +11,7 @@
 //     panels of columns (trd_panel_*, trd_symv_*).  Complex ones:
 //     trdz_reflect_kernel and trdz_update_kernel for every column.  The last
 //     TRD_SMALL_MAX columns (complex TRD_SMALL_MAX_Z) are reduced by one
-//     workgroup in registers (416 us for 192 columns; 136 columns in LDS took
+//     workgroup in registers (420 us for 192 columns; 136 columns in LDS took
 //     556 us, one launch per column 7.1 us each).
 //  2. Divide and conquer on T (Cuppen's tearing, bottom-up): leaves of at
 //     most DC_SMALL_MAX rows are solved one workgroup each (dc_small); each

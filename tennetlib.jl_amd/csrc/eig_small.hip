@@ -109,7 +109,7 @@ __device__ __forceinline__ double sum4(double x) {
 // dead after step j and keeps the reflector, as does row j.
 // SE_ROWS: row j of A receives the reflector right of the diagonal and
 // zeros elsewhere.
-// Measured: 32 rows 13 us, 64 rows 64 us, 192 rows 416 us (136 rows in LDS
+// Measured: 32 rows 13 us, 64 rows 63 us, 192 rows 420 us (136 rows in LDS
 // with 256 threads: 504 us; the same registers over 1024 threads: 910 us, the
 // sums and divisions repeated by every wavefront then bound it).
 // ---------------------------------------------------------------------------
