@@ -41,7 +41,7 @@ struct FArgs {
   void* C; long ldc; long sC;
   double alpha, beta;
   int cA, cB;  // complex: conjugated operands
-  long kstep, Kall;  // batch z sums rows z kstep .. of K alone, at most K of Kall
+  long Kall;   // K in parts: batch z sums rows z K .. (z + 1) K of Kall
 };
 
 __device__ __forceinline__ void tile_coords2(int ntm, int ntn, int& tm, int& tn) {
@@ -492,7 +492,9 @@ struct OneSeg {  // a plain product: one segment
   __device__ __forceinline__ void next() { end = true; }
 };
 
-template <typename T, int TA, int TB, int AL, int BM>
+// PARTS: K in parts (a kernel of its own: the last part's length costs the
+// others 0.1 to 0.2 us)
+template <typename T, int TA, int TB, int AL, int BM, bool PARTS>
 __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(FArgs a) {
   using CF = TileCfg<T, TA, TB, BM, tile_bk<T>(BM)>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -500,11 +502,14 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(FArgs a) {
   int tm, tn;
   tile_coords2(ntm, ntn, tm, tn);
   const long m0 = (long)tm * BM, n0 = (long)tn * BM, bz = blockIdx.z;
-  // the last part of a split K is shorter
-  const long kb = bz * a.kstep, K = min(a.K, a.Kall - kb);
-  const long wA = TA || a.kstep == 0 ? a.wA : min(a.K, a.wA - kb), wB = !TB || a.kstep == 0 ? a.wB : min(a.K, a.wB - kb);
-  OneSeg seg{reinterpret_cast<const T*>(a.A) + bz * a.sA, reinterpret_cast<const T*>(a.B) + bz * a.sB, K, wA, wB,
-             K <= 0};
+  OneSeg seg{reinterpret_cast<const T*>(a.A) + bz * a.sA, reinterpret_cast<const T*>(a.B) + bz * a.sB, a.K, a.wA, a.wB,
+             a.K <= 0};
+  if constexpr (PARTS) {  // the last part may be shorter
+    const long kb = bz * a.K;
+    seg.K = min(a.K, a.Kall - kb);
+    if (!TA) seg.wA = min(a.K, a.wA - kb);
+    if (TB) seg.wB = min(a.K, a.wB - kb);
+  }
   typename Acc<T>::type acc[CF::F][CF::F];
   tile_zero<CF, T>(acc);
   tile_product<CF, T, TA, TB, AL, false, false>(seg, a.M, a.N, m0, n0, a.lda, a.ldb, a.cA, a.cB,
@@ -881,9 +886,13 @@ void launch_tile(tn_ctx* c, const FArgs& a, int batch) {
   constexpr size_t shm = TileCfg<T, TA, TB, BM, tile_bk<T>(BM)>::LDS;
   const long tiles = ((a.M + BM - 1) / BM) * ((a.N + BM - 1) / BM);
   TN_REQUIRE(tiles < (1L << 31), TN_E_INVALID, "gemm: too many tiles");
-  allow_lds((const void*)gemm_fast_kernel<T, TA, TB, AL, BM>, shm);
-  hipLaunchKernelGGL((gemm_fast_kernel<T, TA, TB, AL, BM>), dim3((unsigned)tiles, 1, (unsigned)batch), dim3(256), shm,
-                     c->stream, a);
+  auto launch = [&](auto kern) {
+    allow_lds((const void*)kern, shm);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, 1, (unsigned)batch), dim3(256), shm, c->stream, a);
+  };
+  if constexpr (sizeof(T) != 16)
+    if (a.Kall > a.K) return launch(gemm_fast_kernel<T, TA, TB, AL, BM, true>);
+  launch(gemm_fast_kernel<T, TA, TB, AL, BM, false>);
 }
 template <typename T, int TA, int TB, int AL>
 void launch_bm(tn_ctx* c, const FArgs& a, int batch, int bm) {
@@ -917,7 +926,7 @@ void gemm_tiles(tn_ctx* c, Prec p, const GemmDesc& g) {
   a.wB = aligned ? width_b(p, g) : (g.tB ? g.K : g.N);
   a.C = g.C; a.ldc = g.ldc; a.sC = g.sC;
   a.alpha = g.alpha; a.beta = g.beta;
-  a.kstep = g.kstep; a.Kall = g.K;
+  a.Kall = g.K;
   if (g.kstep) a.K = g.kstep;
   const int bm = pick_tile(p, g.M, g.N, g.batch);
   if (p == Prec::Z64) {
