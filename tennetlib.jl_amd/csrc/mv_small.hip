@@ -245,20 +245,27 @@ __global__ __launch_bounds__(MV_THREADS) void mv_small_kernel(MvArgs g) {
   __syncthreads();
   // T2: rows (c, S'), columns (ga, b)
   mv_stage<1, 1>(wave, un2, unit2, la2, lb2, [&](const Unit& t, const d4 (&acc)[1]) {
+    auto put2 = [&](const d4& x) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = t.m0 + kg + 4 * r;
-      if (row < M2 && t.c0 + ln < N2) {
-        double x = acc[0][r];
-        if (x - x != 0.0) {  // Inf or NaN: only the operator's entries may meet it, not its zeros
-          x = 0.0;
-          for (int k = 0; k < K2; ++k) {
-            const double o = mv_ld<double>(op, (unsigned)(row * K2 + k) * 8u);
-            if (o != 0.0) x = fma(o, T1[t.ob + koff[k]], x);
-          }
-        }
-        T2[t.x + roff[row]] = x;
+      for (int r = 0; r < 4; ++r) {
+        const int row = t.m0 + kg + 4 * r;
+        if (row < M2 && t.c0 + ln < N2) T2[t.x + roff[row]] = x[r];
       }
+    };
+    put2(acc[0]);
+    // NaN if a result is not finite
+    const double nf = fma(acc[0][0], 0.0, acc[0][1] * 0.0) + fma(acc[0][2], 0.0, acc[0][3] * 0.0);
+    if (__any(nf != 0.0)) {  // only the operator's entries may meet an Inf or NaN, not its zeros: again, entry by entry
+      d4 x{0, 0, 0, 0};
+      for (int k = 0; k < K2; ++k) {
+        const double v = T1[t.ob + koff[k]];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double o = mv_ld<double>(op, (unsigned)(min(t.m0 + kg + 4 * r, M2 - 1) * K2 + k) * 8u);
+          if (o != 0.0) x[r] = fma(o, v, x[r]);
+        }
+      }
+      put2(x);
     }
   }, ga2, gb2);
   __syncthreads();

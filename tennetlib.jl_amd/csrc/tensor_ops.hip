@@ -240,12 +240,15 @@ __global__ __launch_bounds__(256, 2) void wstep_mfma_kernel(WmArgs<T> w) {
         if (c1 < w.nB) w.out[off + c1] = x1;
       }
     };
-    T fin = T(0);  // NaN if any result is not finite
+    T nf0 = T(0), nf1 = T(0);  // NaN if any result is not finite
 #pragma unroll
     for (int i = 0; i < NMB; ++i)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) fin += (acc[i][0][r] - acc[i][0][r]) + (acc[i][1][r] - acc[i][1][r]);
-    if (__any(fin != T(0))) {
+      for (int r = 0; r < NR; ++r) {
+        nf0 = fma(acc[i][0][r], T(0), nf0);
+        nf1 = fma(acc[i][1][r], T(0), nf1);
+      }
+    if (__any(nf0 + nf1 != T(0))) {
       // only the operator's entries may meet an Inf or NaN, not its zeros: the strip again, entry by entry
       for (int m = kg; m < w.M; m += 64 / MB) {
         T x0 = T(0), x1 = T(0);
